@@ -27,6 +27,7 @@
 #include "sp_gemv1.h"
 #include "sp_pack.h"
 #include "sp_sample.h"
+#include "sp_wide.h"
 
 namespace {
 
@@ -412,6 +413,91 @@ void launch_rope(int n, const RopeArgs &ra, int np, hipStream_t st) {
     by_slices(np, [&](auto c) { hipLaunchKernelGGL((k_rope_kv<decltype(c)::value>), dim3(n, 2), dim3(ROPE_THREADS), 0, st, ra); });
 }
 
+// ------------------------------------------------------------------------------------------- wide column steps
+// Columns of one wide pass (a prefill of more columns runs in passes of this many).
+constexpr int WIDE_COLS = 2048;
+// Column tiles that a split product's slices may hold together (the partial buffer's size).
+constexpr int WIDE_PART_COLS = 2 * WIDE_COLS;
+
+template <int FMT, int MTW, int RW, int WM, int WN, bool PAIR, bool LO>
+void launch_wide_t(wide::GemmArgs &a, int slices, hipStream_t st) {
+    using T = wide::Tile<FMT, MTW, RW, WM, WN, LO>;
+    a.mblocks = (a.mtp + T::BMT - 1) / T::BMT;
+    a.nblocks = (a.nrg + T::BNG - 1) / T::BNG;
+    a.nst = a.nkt / T::TPS;
+    a.kslice = (a.nst + slices - 1) / slices;
+    hipLaunchKernelGGL((wide::k_gemm_wide<FMT, MTW, RW, WM, WN, PAIR, LO>), dim3(a.mblocks * a.nblocks, slices),
+                       dim3(64 * T::NW), T::SMEM, st, a);
+}
+// Block tiles, columns x weight rows: 0: 128 x 128 (8 waves), 1: 64 x 128 (8 waves), 2: 64 x 64 (4 waves).
+constexpr int WIDE_BM[3] = {128, 64, 64}, WIDE_BN[3] = {128, 128, 64};
+template <int FMT, bool PAIR, bool LO>
+void launch_wide_tile(int tile, wide::GemmArgs &a, int slices, hipStream_t st) {
+    if (tile == 0) launch_wide_t<FMT, 4, 2, 2, 4, PAIR, LO>(a, slices, st);
+    else if (tile == 1) launch_wide_t<FMT, 2, 2, 2, 4, PAIR, LO>(a, slices, st);
+    else launch_wide_t<FMT, 2, 2, 2, 2, PAIR, LO>(a, slices, st);
+}
+template <int FMT>
+void launch_wide_fmt(int tile, bool pair, wide::GemmArgs &a, int slices, hipStream_t st) {
+    if (pair) launch_wide_tile<FMT, true, false>(tile, a, slices, st);
+    else if (a.xlo) launch_wide_tile<FMT, false, true>(tile, a, slices, st);
+    else launch_wide_tile<FMT, false, false>(tile, a, slices, st);
+}
+struct WidePlan { int tile, slices; };
+// The largest tile whose grid fills the 256 CUs; where even the smallest leaves CUs idle, a product whose consumer
+// adds slices is split along K.
+WidePlan plan_wide(const DevMat &m, int n, bool split_ok) {
+    const int nrg = m.rows_pad / 16;
+    auto blocks = [&](int t) { return ((n + WIDE_BM[t] - 1) / WIDE_BM[t]) * ((nrg * 16 + WIDE_BN[t] - 1) / WIDE_BN[t]); };
+    int tile = 0;
+    while (tile < 2 && blocks(tile) < 256) ++tile;
+    int s = 1;
+    if (split_ok && blocks(tile) < 256) {
+        const int nst = m.cols / 128, ncol = (n + 15) / 16 * 16;
+        s = std::min({256 / blocks(tile), GEMV_MAX_SLICES, WIDE_PART_COLS / ncol, std::max(1, nst / 4)});
+        s = std::max(1, s);
+        const int ks = (nst + s - 1) / s;
+        s = (nst + ks - 1) / ks;
+    }
+    return {tile, s};
+}
+
+// y = W x for n columns (fragment-major x with mtp column tiles).  Returns the slice count the consumer must add (raw
+// sums in part; plus the bias for EPI_STORE) or 0 when the epilogue was applied.
+int launch_gemm_wide(const DevMat &m, int epi, const f16 *x, const f16 *xlo, int n, int mtp, float *out_f32, f16 *out_f16,
+                     int ldo, const float *bias, float *part, size_t pstride, hipStream_t st) {
+    require((epi == EPI_SILU) == m.paired, SP_EINVAL, "gemm epilogue does not match the matrix packing");
+    require(n >= 1 && mtp == (n + 15) / 16 && m.cols % 128 == 0, SP_EINVAL, "gemm shape out of range");
+    const WidePlan p = plan_wide(m, n, part != nullptr && !m.paired);
+    wide::GemmArgs a{};
+    a.w = m.w; a.sz = m.sz; a.nkt = m.nkt; a.nrg = m.rows_pad / 16;
+    a.n_real = m.paired ? m.rows / 2 : m.rows;
+    a.x = x; a.xlo = xlo; a.mtp = mtp; a.m = n;
+    a.out_f32 = out_f32; a.out_f16 = out_f16; a.ldo = ldo; a.bias = bias; a.epi = epi; a.pstride = pstride;
+    if (p.slices > 1) { a.epi = EPI_PART; a.out_f32 = part; a.bias = nullptr; }
+    switch (m.fmt) {
+        case 1: launch_wide_fmt<1>(p.tile, m.paired, a, p.slices, st); break;
+        case 2: launch_wide_fmt<2>(p.tile, m.paired, a, p.slices, st); break;
+        default: launch_wide_fmt<3>(p.tile, m.paired, a, p.slices, st); break;
+    }
+    return p.slices > 1 ? p.slices : 0;
+}
+
+template <int HD>
+void launch_attn_wide(int G, dim3 grid, hipStream_t st, const wide::AttnWideArgs &a) {
+    switch (G) {
+        case 1: hipLaunchKernelGGL((wide::k_attn_wide<HD, 1, 1>), grid, dim3(256), 0, st, a); break;
+        case 2: hipLaunchKernelGGL((wide::k_attn_wide<HD, 2, 1>), grid, dim3(256), 0, st, a); break;
+        case 3: hipLaunchKernelGGL((wide::k_attn_wide<HD, 3, 1>), grid, dim3(256), 0, st, a); break;
+        case 4: hipLaunchKernelGGL((wide::k_attn_wide<HD, 4, 1>), grid, dim3(256), 0, st, a); break;
+        case 5: hipLaunchKernelGGL((wide::k_attn_wide<HD, 5, 1>), grid, dim3(256), 0, st, a); break;
+        case 6: hipLaunchKernelGGL((wide::k_attn_wide<HD, 6, 1>), grid, dim3(256), 0, st, a); break;
+        case 7: hipLaunchKernelGGL((wide::k_attn_wide<HD, 7, 1>), grid, dim3(256), 0, st, a); break;
+        default: hipLaunchKernelGGL((wide::k_attn_wide<HD, 8, 1>), grid, dim3(256), 0, st, a); break;
+    }
+}
+constexpr int WIDE_ATT_ROWS = 64;       // query rows per attention block
+
 // decode attention split: waves per block x 32-key sub-chunks per wave
 struct DecShape { int nwv, sub; };
 // Keys per decode-attention block: 1024 (2 waves streaming 16 sub-chunks of 32 keys, two sub-chunks of loads in
@@ -558,6 +644,22 @@ struct sp_engine {
     bool run_d1(const sp_token &t, int flags);        // + the error word copy, the head GEMV and the argmax
     void check_d1_error();
 
+    // wide passes (sp_engine_prefill): activations for up to WIDE_COLS columns, allocated by the first such call
+    struct Wide {
+        float *x = nullptr, *qkv = nullptr, *q = nullptr, *part = nullptr;
+        float2 *rtab = nullptr;
+        f16 *xn = nullptr, *xn_lo = nullptr, *attn = nullptr, *act = nullptr, *kn = nullptr, *vn = nullptr;
+        char *mem = nullptr, *d_up = nullptr, *h_up = nullptr;      // mem: the allocation that holds all of them
+        hipEvent_t up_done = nullptr;
+        // parts of the upload: column records, runs, attention items, ring flags, output columns
+        size_t o_runs = 0, o_items = 0, o_keep = 0, o_out = 0, up_bytes = 0;
+        int max_items = 0;
+    } wd;
+    void alloc_wide();
+    void free_wide();
+    void prefill_pass(int n, const sp_token *toks, int n_out, const int *out_cols, float *logits_dev, bool argmax);
+    void head_rows(int n, float *xrows, int pend, float *logits_dev, bool argmax);
+
     // attention plan of one forward call: same-sequence column groups (multi-query kernel) or one block row per column
     struct AttnPlan {
         bool mq = false;
@@ -582,6 +684,7 @@ struct sp_engine {
 
 void sp_engine::free_all() {
     drop_graphs();
+    free_wide();
     dev_free(d1_ll); dev_free(d1_err); dev_free(d1_layers); dev_free(d1_static);
     if (h_d1err) (void)hipHostFree(h_d1err);
     d1_ll = nullptr; d1_err = nullptr; d1_layers = nullptr; d1_static = nullptr; h_d1err = nullptr; d1_state = 0;
@@ -918,6 +1021,181 @@ void sp_engine::step(int n, int flags, const AttnPlan &ap, int l0, int l1) {
         if (flags & SP_F_ARGMAX) {
             hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, st, logits, d.vocab, d.vocab, am_v, am_i);
             hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(64), 0, st, am_v, am_i, am_out);
+        }
+    }
+    HIPCHK(hipGetLastError());
+}
+
+// ------------------------------------------------------------------------------------------- wide passes
+void sp_engine::free_wide() {
+    dev_free(wd.mem);
+    if (wd.h_up) (void)hipHostFree(wd.h_up);
+    if (wd.up_done) (void)hipEventDestroy(wd.up_done);
+    wd = Wide();
+}
+
+// Buffers of a wide pass, once per engine, in one allocation (Qwen2-1.5B 0.16 GB, Qwen2-7B 0.34 GB).
+void sp_engine::alloc_wide() {
+    if (wd.h_up) return;
+    const size_t P = WIDE_COLS, H = d.hidden, I = d.intermediate, NHD = (size_t)d.n_heads * d.head_dim;
+    const size_t KV = P * d.n_kv_heads * d.head_dim;
+    auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    // a run of c columns has ceil(c G / rows) attention items: at most one partial item per run (P runs)
+    wd.max_items = (int)(P * (d.n_heads / d.n_kv_heads) / WIDE_ATT_ROWS + P);
+    wd.o_runs = up256(P * sizeof(sp_token));
+    wd.o_items = wd.o_runs + up256(P * sizeof(wide::Run));
+    wd.o_keep = wd.o_items + up256(wd.max_items * sizeof(wide::Item));
+    wd.o_out = wd.o_keep + up256(P * sizeof(int));
+    wd.up_bytes = wd.o_out + up256(P * sizeof(int));
+    const size_t sizes[] = {P * H * 4, P * Nqkv * 4, P * NHD * 4, (size_t)WIDE_PART_COLS * std::max<size_t>(H, Nqkv) * 4,
+                            P * (d.head_dim / 2) * sizeof(float2), P * H * 2, P * H * 2, P * NHD * 2, P * I * 2, KV * 2, KV * 2,
+                            wd.up_bytes};
+    size_t total = 0;
+    for (size_t b : sizes) total += up256(b);
+    try {
+        wd.mem = dev_alloc<char>(total);
+        HIPCHK(hipEventCreateWithFlags(&wd.up_done, hipEventDisableTiming));
+        HIPCHK(hipHostMalloc((void **)&wd.h_up, wd.up_bytes, hipHostMallocDefault));
+    } catch (...) {
+        free_wide();
+        throw;
+    }
+    char *p = wd.mem;
+    int i = 0;
+    auto take = [&](auto *&dst) { dst = (std::remove_reference_t<decltype(dst)>)p; p += up256(sizes[i++]); };
+    take(wd.x); take(wd.qkv); take(wd.q); take(wd.part); take(wd.rtab); take(wd.xn); take(wd.xn_lo); take(wd.attn); take(wd.act);
+    take(wd.kn); take(wd.vn); take(wd.d_up);
+}
+
+// Final norm (adding pend pending slices in gpart), LM head and (argmax) the greedy ids of n <= 64 residual rows; logits
+// to the engine's rows and, when given, to logits_dev.
+void sp_engine::head_rows(int n, float *xrows, int pend, float *logits_dev, bool argmax) {
+    const int mtp = n > 1 ? (n + 15) / 16 : 0;
+    const DevMat &hm = d.tied_head ? embed : head;
+    launch_rmsnorm(n, xrows, d.hidden, gpart, pend, gpart_stride, final_norm, d.rms_eps, xn, nullptr, stream, mtp);
+    launch_gemv(hm, EPI_STORE, xn, d.hidden, n, logits, nullptr, d.vocab, nullptr, stream, nullptr, 0, PRO_NONE, nullptr, 0, 0, mtp);
+    if (argmax) {
+        hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_v, am_i);
+        hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(64), 0, stream, am_v, am_i, am_out);
+    }
+    if (logits_dev)
+        HIPCHK(hipMemcpyAsync(logits_dev, logits, (size_t)n * d.vocab * sizeof(float), hipMemcpyDeviceToDevice, stream));
+}
+
+// One wide pass: n <= WIDE_COLS plain columns (runs of consecutive positions, each sequence once) through every layer.
+// The logits of columns out_cols go to logits_dev [n_out][vocab] (and, for n_out <= maxT, the engine's rows and ids).
+void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *out_cols, float *logits_dev, bool argmax) {
+    const int H = d.hidden, I = d.intermediate, NH = d.n_heads, NKV = d.n_kv_heads, HD = d.head_dim, G = NH / NKV;
+    const int mtp = (n + 15) / 16;
+    // ---- runs, attention items, which columns the ring keeps, and whether a new key may be stored before the attention
+    std::vector<wide::Run> runs;
+    std::vector<wide::Item> items;
+    std::vector<int> keep(n, 0);
+    bool to_ring = true, last_only = n_out <= std::min(maxT, 64);
+    std::vector<char> is_last(n, 0);
+    for (int c = 0; c < n;) {
+        int e = c + 1;
+        while (e < n && toks[e].seq == toks[c].seq) ++e;
+        const int p0 = toks[c].ctx_hi, p1 = toks[e - 1].ctx_hi;
+        runs.push_back({c, e - c, toks[c].seq, p0});
+        to_ring = to_ring && p1 - toks[c].ctx_lo + 1 <= n_slots;
+        for (int i = c; i < e; ++i) keep[i] = toks[i].ctx_hi > p1 - n_slots;
+        for (int r0 = 0; r0 < (e - c) * G; r0 += WIDE_ATT_ROWS) items.push_back({(int)runs.size() - 1, r0});
+        is_last[e - 1] = 1;
+        c = e;
+    }
+    for (int i = 0; i < n_out; ++i) last_only = last_only && is_last[out_cols[i]];
+    require((int)items.size() <= wd.max_items, SP_EINVAL, "prefill plan out of range");
+    // ---- one upload from pinned memory
+    HIPCHK(hipEventSynchronize(wd.up_done));
+    std::memcpy(wd.h_up, toks, n * sizeof(sp_token));
+    std::memcpy(wd.h_up + wd.o_runs, runs.data(), runs.size() * sizeof(wide::Run));
+    std::memcpy(wd.h_up + wd.o_items, items.data(), items.size() * sizeof(wide::Item));
+    std::memcpy(wd.h_up + wd.o_keep, keep.data(), n * sizeof(int));
+    if (n_out) std::memcpy(wd.h_up + wd.o_out, out_cols, n_out * sizeof(int));
+    HIPCHK(hipMemcpyAsync(wd.d_up, wd.h_up, wd.up_bytes, hipMemcpyHostToDevice, stream));
+    HIPCHK(hipEventRecord(wd.up_done, stream));
+    const sp_token *dt = (const sp_token *)wd.d_up;
+    const int *dout = (const int *)(wd.d_up + wd.o_out);
+    switch (embed.fmt) {
+        case 1: launch_embed<1>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
+        case 2: launch_embed<2>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
+        default: launch_embed<3>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
+    }
+    const size_t ps = (size_t)n * std::max(H, Nqkv);       // slices lie n columns apart
+    const float scale = 1.0f / std::sqrt((float)HD);
+    int pend = 0;
+    for (int l = 0; l < d.n_layers; ++l) {
+        Layer &ly = layers[l];
+        const bool last = l + 1 == d.n_layers;
+        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
+        const int sq = launch_gemm_wide(ly.qkv, EPI_STORE, wd.xn, wd.xn_lo, n, mtp, wd.qkv, nullptr, Nqkv, ly.qkv_b, wd.part, ps,
+                                        stream);
+        wide::RopeWideArgs ra{RopeArgs{wd.qkv, Nqkv, NH, NKV, HD, wd.rtab, dt, wd.q, kc[l], vc[l], n_slots, wd.part, ps, ly.qkv_b},
+                              wd.kn, wd.vn, WIDE_COLS, to_ring ? 1 : 0};
+        by_slices(sq, [&](auto c) {
+            hipLaunchKernelGGL((wide::k_rope_wide<decltype(c)::value>), dim3(n), dim3(256), 0, stream, ra);
+        });
+        auto commit = [&] {
+            if (!to_ring)
+                hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt,
+                                   (const int *)(wd.d_up + wd.o_keep), NKV, HD, n_slots, WIDE_COLS);
+        };
+        if (last && n_out == 0) { commit(); break; }
+        if (last && last_only) {
+            // only the output columns go on: the rest of the last layer and the head run as a batch of n_out decode
+            // columns over the ring, which now holds every key they see
+            commit();
+            std::vector<sp_token> ot(n_out);
+            for (int i = 0; i < n_out; ++i) ot[i] = toks[out_cols[i]];
+            AttnPlan ap = plan_attention(n_out, ot.data(), false);
+            upload(n_out, ot.data(), ap);
+            const int m1 = n_out > 1 ? (n_out + 15) / 16 : 0;
+            hipLaunchKernelGGL(wide::k_gather_rows, dim3(n_out), dim3(256), 0, stream, wd.x, dout, H, x);
+            hipLaunchKernelGGL(wide::k_gather_rows, dim3(n_out), dim3(256), 0, stream, wd.q, dout, NH * HD, q);
+            launch_attention(l, n_out, ap, m1, stream);
+            if (!ap.dec_direct)
+                hipLaunchKernelGGL(k_attn_combine, dim3(NH, n_out), dim3(HD), 0, stream, attn_part, dcolnc, NH, HD, ap.nchunk,
+                                   attn, NH * HD, m1);
+            pend = launch_gemv(ly.o, EPI_RESID, attn, NH * HD, n_out, x, nullptr, H, nullptr, stream, gpart, gpart_stride,
+                               PRO_NONE, nullptr, 0, 0, m1);
+            f16 *xlo = n_out == 1 ? xn_lo : nullptr, *alo = n_out == 1 ? act_lo : nullptr;
+            launch_rmsnorm(n_out, x, H, gpart, pend, gpart_stride, ly.post_norm, d.rms_eps, xn, xlo, stream, m1);
+            launch_gemv(ly.gate_up, EPI_SILU, xn, H, n_out, nullptr, act, I, nullptr, stream, nullptr, 0, PRO_NONE, nullptr, 0, 0,
+                        m1, m1, xlo, alo);
+            pend = launch_gemv(ly.down, EPI_RESID, act, I, n_out, x, nullptr, H, nullptr, stream, gpart, gpart_stride, PRO_NONE,
+                               nullptr, n_out == 1 ? 8 : 0, n_out == 1 ? 8 : 0, m1, 0, alo);
+            head_rows(n_out, x, pend, logits_dev, argmax);
+            HIPCHK(hipGetLastError());
+            return;
+        }
+        wide::AttnWideArgs aa{wd.q, kc[l], vc[l], wd.kn, wd.vn, dt, (const wide::Run *)(wd.d_up + wd.o_runs),
+                              (const wide::Item *)(wd.d_up + wd.o_items), NH, NKV, n_slots, WIDE_COLS, mtp, scale, wd.attn};
+        const dim3 agrid((unsigned)items.size(), NKV);
+        if (HD == 64) launch_attn_wide<64>(G, agrid, stream, aa);
+        else launch_attn_wide<128>(G, agrid, stream, aa);
+        commit();
+        pend = launch_gemm_wide(ly.o, EPI_RESID, wd.attn, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
+        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
+        launch_gemm_wide(ly.gate_up, EPI_SILU, wd.xn, nullptr, n, mtp, nullptr, wd.act, I, nullptr, nullptr, 0, stream);
+        pend = launch_gemm_wide(ly.down, EPI_RESID, wd.act, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
+    }
+    if (n_out > 0) {
+        // every column's final residual is needed: the pending slices go in with the norm (whose output is used when
+        // all columns have logits)
+        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, final_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
+        bool all = n_out == n && logits_dev && !argmax;
+        for (int i = 0; i < n_out; ++i) all = all && out_cols[i] == i;
+        if (all) {
+            launch_gemm_wide(d.tied_head ? embed : head, EPI_STORE, wd.xn, nullptr, n, mtp, logits_dev, nullptr, d.vocab, nullptr,
+                             nullptr, 0, stream);
+        } else {
+            const int step = std::min(maxT, 64);
+            for (int i = 0; i < n_out; i += step) {
+                const int c = std::min(step, n_out - i);
+                hipLaunchKernelGGL(wide::k_gather_rows, dim3(c), dim3(256), 0, stream, wd.x, dout + i, H, x);
+                head_rows(c, x, 0, logits_dev ? logits_dev + (size_t)i * d.vocab : nullptr, argmax);
+            }
         }
     }
     HIPCHK(hipGetLastError());
@@ -1401,6 +1679,50 @@ int sp_engine_forward(sp_engine *e, int32_t n, const sp_token *toks, int32_t fla
             HIPCHK(hipMemcpyAsync(e->h_ids, e->am_out, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
             HIPCHK(hipStreamSynchronize(e->stream));
             std::memcpy(argmax_host, e->h_ids, n * sizeof(int32_t));
+        }
+    });
+}
+
+int sp_engine_prefill(sp_engine *e, int32_t n, const sp_token *toks, int32_t n_out, const int32_t *out_cols, float *logits_dev,
+                      int32_t *argmax_host) {
+    if (!e) { g_err = "engine is NULL"; return SP_EINVAL; }
+    return guarded(e, [&] {
+        const sp_model_desc &d = e->d;
+        require(n >= 1 && n <= WIDE_COLS, SP_ECAPACITY, "column count must be in [1, 2048]");
+        require(toks != nullptr, SP_EINVAL, "toks is NULL");
+        require(n_out >= 0 && n_out <= n && (n_out == 0 || out_cols), SP_EINVAL, "n_out must be in [0, n], with its columns");
+        require(!argmax_host || (n_out >= 1 && n_out <= e->maxT), SP_EINVAL, "greedy ids need 1 to max_tokens output columns");
+        require(n_out == 0 || logits_dev || argmax_host, SP_EINVAL, "output columns need logits_dev or argmax_host");
+        require(e->n_seq > 0, SP_ESTATE, "KV cache not reserved");
+        require(e->embed.w && e->final_norm && (d.tied_head || e->head.w), SP_ESTATE, "embedding / head / final norm not loaded");
+        for (auto &l : e->layers)
+            require(l.qkv.w && l.o.w && l.gate_up.w && l.down.w && l.qkv_b && l.in_norm && l.post_norm, SP_ESTATE,
+                    "a layer's weights are not loaded");
+        e->check_columns(n, toks, false);
+        std::vector<char> seen(e->n_seq, 0);
+        for (int i = 0; i < n; ++i) {
+            const sp_token &t = toks[i];
+            require(t.tree_count == 0 && t.ctx_hi >= t.ctx_lo && t.slot == t.ctx_hi % e->n_slots, SP_EINVAL,
+                    "prefill takes plain columns (no tree block, the slot of the newest visible position)");
+            if (i > 0 && toks[i - 1].seq == t.seq) {
+                require(t.ctx_hi == toks[i - 1].ctx_hi + 1 && t.ctx_lo >= toks[i - 1].ctx_lo, SP_EINVAL,
+                        "a sequence's columns must be at consecutive positions");
+            } else {
+                require(!seen[t.seq], SP_EINVAL, "a sequence's columns must be consecutive");
+                seen[t.seq] = 1;
+            }
+        }
+        for (int i = 0; i < n_out; ++i) require(out_cols[i] >= 0 && out_cols[i] < n, SP_EINVAL, "output column out of range");
+        e->check_d1_error();
+        e->alloc_wide();
+        e->prefill_pass(n, toks, n_out, out_cols, logits_dev, argmax_host != nullptr);
+        e->last_path = 0;
+        e->last_dispatches = -1;
+        if (argmax_host) {
+            e->argmax_cols = n_out;
+            HIPCHK(hipMemcpyAsync(e->h_ids, e->am_out, n_out * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
+            HIPCHK(hipStreamSynchronize(e->stream));
+            std::memcpy(argmax_host, e->h_ids, n_out * sizeof(int32_t));
         }
     });
 }

@@ -29,6 +29,7 @@ from . import _lib
 from . import native_bundle
 
 GROUP = 32
+WIDE_COLS = 2048          # most columns of one wide prefill pass (sp_engine_prefill)
 
 
 class _KVLayers:
@@ -381,6 +382,28 @@ class Qwen2Engine:
         in place (TreeVerifier.forward)."""
         return self._forward(n, cols_addr, flags, logits_out, want_ids)
 
+    def _prompt_columns(self, ids, cache, first, positions=None):
+        """The columns of tokens `ids` at cache positions first, first + 1, ... (RoPE at `positions` when given)."""
+        p = np.arange(first, first + len(ids), dtype=np.int64)
+        a = np.zeros(len(ids), dtype=_lib.TOKEN_DTYPE)
+        a['token'] = np.asarray(ids, dtype=np.int64).astype(np.int32)
+        a['seq'] = cache.seq
+        a['pos'] = p if positions is None else np.asarray(positions, dtype=np.int64).astype(np.int32)
+        a['slot'] = p % self._pool_slots
+        a['ctx_hi'] = p
+        if cache.window is not None:
+            a['ctx_lo'] = np.maximum(0, p - cache.window + 1)
+        return a
+
+    def _wide(self, cols, out, logits_out=None, want_ids=False):
+        """One wide pass (sp_engine_prefill) over a TOKEN_DTYPE array of at most WIDE_COLS columns; logits (and greedy
+        ids) of the columns `out`."""
+        out = np.ascontiguousarray(out, dtype=np.int32)
+        ids = np.zeros(len(out), dtype=np.int32) if want_ids else None
+        dst = ctypes.c_void_p(logits_out.data_ptr()) if logits_out is not None else None
+        _lib.check(self.lib.sp_engine_prefill(self.h, len(cols), _ptr(cols), len(out), _ptr(out), dst, _ptr(ids)), self.h)
+        return ids
+
     def _forward(self, n, arr, flags, logits_out, want_ids):
         ids = np.zeros(n, dtype=np.int32) if want_ids else None
         if want_ids:
@@ -409,6 +432,18 @@ class Qwen2Engine:
             raise ValueError('positions must match input_ids')
         logits = torch.empty((qlen if all_logits else 1, self.vocab), dtype=torch.float32, device=self.device)
         T = self.max_tokens
+        if qlen > T:
+            cols = self._prompt_columns(ids, cache, start, positions)
+            for c0 in range(0, qlen, WIDE_COLS):
+                part = cols[c0:c0 + WIDE_COLS]
+                if all_logits:
+                    self._wide(part, np.arange(len(part)), logits_out=logits[c0:c0 + len(part)])
+                elif c0 + len(part) == qlen:
+                    self._wide(part, [len(part) - 1], logits_out=logits)
+                else:
+                    self._wide(part, [])
+            cache.length += qlen
+            return logits, cache
         for c0 in range(0, qlen, T):
             c1 = min(qlen, c0 + T)
             cols = [self._column(ids[i], cache, slots[i], positions[i]) for i in range(c0, c1)]
@@ -613,6 +648,16 @@ class Qwen2Engine:
         T = self.max_tokens
         start = cache.length
         out = None
+        if len(ids) > T:
+            cols = self._prompt_columns(ids, cache, start)
+            for c0 in range(0, len(ids), WIDE_COLS):
+                part = cols[c0:c0 + WIDE_COLS]
+                if c0 + len(part) == len(ids):
+                    out = int(self._wide(part, [len(part) - 1], want_ids=True)[0])
+                else:
+                    self._wide(part, [])
+            cache.length += len(ids)
+            return out
         for c0 in range(0, len(ids), T):
             c1 = min(len(ids), c0 + T)
             cols = [self._column(ids[i], cache, start + i, start + i) for i in range(c0, c1)]
@@ -629,6 +674,11 @@ class Qwen2Engine:
         Returns the greedy next token of every sequence."""
         nxt = [None] * len(prompts)
         T = self.max_tokens
+        if sum(len(p) for p in prompts) > T and len({c.seq for c in caches}) == len(caches) == len(prompts):
+            self._prefill_wide(prompts, caches, nxt)
+            for s, p in enumerate(prompts):
+                caches[s].length += len(p)
+            return nxt
         queue = [(s, i, t) for s, p in enumerate(prompts) for i, t in enumerate(p)]
         for c0 in range(0, len(queue), T):
             chunk = queue[c0:c0 + T]
@@ -640,6 +690,32 @@ class Qwen2Engine:
         for s, p in enumerate(prompts):
             caches[s].length += len(p)
         return nxt
+
+    def _prefill_wide(self, prompts, caches, nxt):
+        """prefill() of distinct sequences in wide passes: each takes up to WIDE_COLS columns, a prompt cut where a pass
+        is full, and ends at most max_tokens prompts (the greedy ids of one call)."""
+        parts, n, ends = [], 0, []              # columns of the pass, their count, (prompt, last column) pairs
+
+        def flush():
+            nonlocal parts, n, ends
+            if parts:
+                ids = self._wide(np.concatenate(parts), [c for _, c in ends], want_ids=bool(ends))
+                for (s, _), tid in zip(ends, ids if ends else []):
+                    nxt[s] = int(tid)
+            parts, n, ends = [], 0, []
+
+        for s, p in enumerate(prompts):
+            cols = self._prompt_columns([int(t) for t in p], caches[s], caches[s].length)
+            c0 = 0
+            while c0 < len(cols):
+                take = min(WIDE_COLS - n, len(cols) - c0)
+                parts.append(cols[c0:c0 + take])
+                c0, n = c0 + take, n + take
+                if c0 == len(cols):
+                    ends.append((s, n - 1))
+                if n == WIDE_COLS or len(ends) == self.max_tokens:
+                    flush()
+        flush()
 
     @torch.inference_mode()
     def generate_batch(self, prompts, max_new_tokens=32, eos_token_id=None, window=None, graph=True):
