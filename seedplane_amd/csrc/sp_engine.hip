@@ -2139,7 +2139,7 @@ int sp_op_gemv(const sp_weight *w, const void *x_dev, int32_t m_cols, float *y_d
 // sp_library_release (or the process end); each map is guarded by its mutex.
 namespace lib_scratch {
 struct Smp { float *pmax; double *csum; };
-struct Fm { FmHist *hist; FmState *st; };
+struct Fm { FmState *st; FmPair *list; };
 struct Acc { unsigned long long *xbuf; unsigned *err; int32_t *host; };
 struct Stage { unsigned char *buf = nullptr; size_t cap = 0; hipEvent_t done = nullptr; bool used = false; };
 std::map<int, Smp> smp;
@@ -2195,34 +2195,49 @@ int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, co
         require(temperature > 0.0, SP_EINVAL, "temperature must be positive");
         require(top_p > 0.0, SP_EINVAL, "top_p must be positive");
         hipStream_t st = (hipStream_t)stream;
-        // histograms and per-row state for FM_ROWS draws, one set per device (calls on one device must not overlap)
+        // histograms, lists and per-row state for FM_ROWS draws, one set per device (calls on one device must not
+        // overlap); zeroed once, each call's last kernel clears what the call used
         int dev = 0;
         HIPCHK(hipGetDevice(&dev));
         lib_scratch::Fm sc;
         {
             std::lock_guard<std::mutex> lock(lib_scratch::fm_mu);
             auto it = lib_scratch::fm.find(dev);
-            if (it == lib_scratch::fm.end())
-                it = lib_scratch::fm.emplace(dev, lib_scratch::Fm{dev_alloc<FmHist>((size_t)FM_ROWS * FM_NLEV),
-                                                                  dev_alloc<FmState>(FM_ROWS)}).first;
+            if (it == lib_scratch::fm.end()) {
+                lib_scratch::Fm f{dev_alloc<FmState>(FM_ROWS), nullptr};
+                try {
+                    f.list = dev_alloc<FmPair>((size_t)3 * FM_ROWS * FM_CAP);
+                    HIPCHK(hipMemset(f.st, 0, FM_ROWS * sizeof(FmState)));
+                } catch (...) {
+                    dev_free(f.st);
+                    dev_free(f.list);
+                    throw;
+                }
+                it = lib_scratch::fm.emplace(dev, f).first;
+            }
             sc = it->second;
         }
         const int nb = (vocab + FM_SPAN - 1) / FM_SPAN;
-        const bool topk = top_k > 0 && top_k < vocab;
+        const int k = top_k > 0 && top_k < vocab ? top_k : 0;
         for (int r0 = 0; r0 < n; r0 += FM_ROWS) {
             const int nr = std::min(FM_ROWS, n - r0);
-            const FmArgs a{logits_dev, vocab, ld, row_dev, u_dev, (float)temperature, top_k, top_p, out_dev, sc.hist,
-                           sc.st, r0};
+            const FmArgs a{logits_dev, vocab, ld, row_dev, u_dev, (float)temperature, k, top_p, out_dev, sc.st, sc.list, r0};
             const dim3 grid(nb, nr), block(FS_THREADS);
-            hipLaunchKernelGGL(k_fm_init, dim3(nr), dim3(256), 0, st, a);
-            hipLaunchKernelGGL(k_fm_max, grid, block, 0, st, a);
-            if (topk)
-                for (int j = 0; j < 4; ++j) hipLaunchKernelGGL(k_fm_topk, grid, block, 0, st, a, j);
-            hipLaunchKernelGGL(k_fm_h1, grid, block, 0, st, a);
-            if (top_p < 1.0)
-                for (int j = 0; j < 3; ++j) hipLaunchKernelGGL(k_fm_select<false>, grid, block, 0, st, a, j);
-            for (int j = 0; j < 3; ++j) hipLaunchKernelGGL(k_fm_select<true>, grid, block, 0, st, a, j);
-            hipLaunchKernelGGL(k_fm_finish, dim3(nr), block, 0, st, a);
+            hipLaunchKernelGGL(k_fm_top, grid, block, 0, st, a);
+            if (k && k <= FM_SMALL_K) {
+                hipLaunchKernelGGL(k_fm_gather<0>, grid, block, 0, st, a);
+                hipLaunchKernelGGL(k_fm_finish<true>, dim3(nr), block, 0, st, a);
+            } else {
+                if (k) {
+                    hipLaunchKernelGGL(k_fm_gather<1>, grid, block, 0, st, a);
+                    hipLaunchKernelGGL(k_fm_mass<true>, grid, block, 0, st, a);
+                } else {
+                    hipLaunchKernelGGL(k_fm_mass<false>, grid, block, 0, st, a);
+                }
+                if (top_p < 1.0) hipLaunchKernelGGL(k_fm_gather<2>, grid, block, 0, st, a);
+                hipLaunchKernelGGL(k_fm_gather<3>, grid, block, 0, st, a);
+                hipLaunchKernelGGL(k_fm_finish<false>, dim3(nr), block, 0, st, a);
+            }
             HIPCHK(hipGetLastError());
         }
     });
@@ -2416,7 +2431,7 @@ int sp_library_release(void) {
                 HIPCHK(hipDeviceSynchronize());
             }
             for (auto &kv : lib_scratch::smp) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.pmax); dev_free(kv.second.csum); }
-            for (auto &kv : lib_scratch::fm) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.hist); dev_free(kv.second.st); }
+            for (auto &kv : lib_scratch::fm) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.st); dev_free(kv.second.list); }
             for (auto &kv : lib_scratch::acc) {
                 HIPCHK(hipSetDevice(kv.first));
                 dev_free(kv.second.xbuf);

@@ -645,10 +645,22 @@ __global__ void __launch_bounds__(ACC_T) k_accept_tree(AcceptArgs a) {
 //         is <= floor(p * F) (first index whose inclusive mass exceeds that, and everything before it);
 //   draw: target = floor(u * K) (clamped below K) over the kept mass K; the token is the first in sorted order whose
 //         inclusive cumulative mass exceeds the target (inverse CDF, Sampler::draw, sampler.hpp:93-97).
-// Selections in sorted order never sort: a radix descent over the 32-bit order key (8 bits per level, LDS histograms
-// of counts and 64-bit masses restricted to the candidates, added into global histograms) finds the bin holding the
-// k-th token / the target mass; at the last level the bin is one z value, whose tokens (equal masses) are ordered
-// by index.
+// Selections in sorted order never sort.  The 32-bit order key is split 12 + 10 + 10 bits: a histogram of the top 12
+// bits over the row (counts for the k-th largest, 64-bit masses for a cumulative target; 4096 bins in LDS per block,
+// added into the row's global histogram with integer atomics) names the bin that holds the token looked for, the
+// entries of that bin are gathered into a list, and two 10-bit levels over the list end at one key, whose tokens (equal
+// masses) are ordered by index.
+//
+// Launches (each covers a row with one block per FM_SPAN entries, so all passes over a row run on the whole chip):
+//   k_fm_top      row maximum; with top-k the count histogram
+//   top-k up to FM_SMALL_K:  k_fm_gather collects every entry of the boundary bin and above (the k kept tokens are among
+//                 them) and k_fm_finish does the rest on the list, one block per row
+//   otherwise:    [k_fm_gather: the boundary bin of top-k], k_fm_mass: mass histogram of the kept entries,
+//                 [k_fm_gather: the bin of the top-p cut], k_fm_gather: the bin of the draw, k_fm_finish
+// 16 draws over 151936 entries on an MI355X, where each launch costs about 4-7 us and each radix level of 8 bits over
+// the whole row used to be one: see the launch sequence in sp_op_sample_filtered for the measured times.
+// A list that would hold more than FM_CAP entries (a row whose logits are mostly equal) is not used: the block that
+// needs it scans the row instead.
 constexpr int FS_THREADS = 1024;
 
 __device__ __forceinline__ uint32_t fs_key(float z) {      // monotone: larger z, larger key
@@ -662,50 +674,45 @@ __device__ __forceinline__ unsigned long long fs_mass(float z, float zmax) {
     return (unsigned long long)(exp((double)z - (double)zmax) * 1099511627776.0);    // 2^40
 }
 
-struct FsShared {
-    unsigned long long hmass[256];
-    unsigned int hcnt[256];
-    unsigned int hidx[256];             // last level: the smallest index in each bin
-    unsigned long long h1mass[256];     // first-level (top 8 key bits) histogram of the candidates, built once
-    unsigned int h1cnt[256];
-    unsigned long long red64[FS_THREADS / 64];
-    unsigned int redu[FS_THREADS / 64];
-    unsigned int sel_bin;
-    unsigned long long above;
-    unsigned int scan[FS_THREADS];
+constexpr int FM_U = 8;                            // entries per thread and pass
+constexpr int FM_SPAN = FS_THREADS * FM_U;         // entries of a row per block
+constexpr int FM_ROWS = 256;                       // rows per launch sequence (the scratch holds this many)
+constexpr int FM_B0 = 4096, FM_B1 = 1024;          // bins of the first level (key >> 20) and of the two below
+constexpr int FM_CAP = 8192;                       // entries a list holds
+// top-k up to this runs on one list: with at most 1024 kept tokens the boundary bin and those above it (an eighth of an
+// octave of z each) hold a few thousand entries at most for ordinary logits
+constexpr int FM_SMALL_K = 1024;
+struct FmPair { uint32_t key; int idx; };
+// Per-row scratch.  kmax, n and the histograms are zero between calls: the finishing kernel clears what the call used.
+struct FmState {
+    unsigned long long mass[FM_B0];
+    unsigned int cnt[FM_B0];
+    unsigned int kmax;
+    unsigned int n[3];                             // entries of lists 0 (top-k), 1 (top-p), 2 (draw)
+    unsigned int kbin, krem, kmin;                 // top-k: boundary bin, tokens to take from it; smallest kept key
+    unsigned int tbin, dbin;                       // bins of the top-p cut and of the draw
+    unsigned long long tabove, dabove, tp, tgt;    // mass before those bins, and the targets
+    int topp;                                      // 1: the top-p cut applies (tp < kept mass)
+};
+struct FmArgs {
+    const float *logits;
+    int V, ld;
+    const int *rows;
+    const double *u;
+    float T;
+    int top_k;                                     // 0: no top-k
+    double top_p;                                  // < 1: top-p
+    int *out;
+    FmState *st;                                   // [FM_ROWS]
+    FmPair *list;                                  // [3][FM_ROWS][FM_CAP]
+    int row0;                                      // draws row0 .. row0 + gridDim.y - 1 (blockIdx.y = draw - row0)
 };
 
-// Histogram add with the wave's lanes combined per bin first: most keys of a row share their top bits, and 64 lanes
-// adding to one LDS word serialise.  Up to FS_AGG distinct bins of the wave are combined (one atomic per bin, from
-// the lowest active lane); lanes left after that add on their own.  Integer sums: the result is order-independent.
-#ifndef SP_FS_AGG
-#define SP_FS_AGG 1
-#endif
-constexpr int FS_AGG = SP_FS_AGG;
-template <bool MASS>
-__device__ __forceinline__ void fs_hist_add(FsShared &sh, bool act, int bin, unsigned long long mass) {
-    const int lane = threadIdx.x & 63;
-    for (int it = 0; it < FS_AGG; ++it) {
-        const unsigned long long pend = __ballot(act);
-        if (pend == 0) return;
-        const int leader = __ffsll((long long)pend) - 1;
-        const int lb = __shfl(bin, leader);
-        const bool mine = act && bin == lb;
-        const unsigned long long mm = __ballot(mine);
-        if constexpr (MASS) {
-            unsigned long long v = mine ? mass : 0ull;
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            if (lane == leader) atomicAdd(&sh.hmass[lb], v);
-        }
-        if (lane == leader) atomicAdd(&sh.hcnt[lb], (unsigned)__popcll(mm));
-        act = act && !mine;
-    }
-    if (act) {
-        if constexpr (MASS) atomicAdd(&sh.hmass[bin], mass);
-        atomicAdd(&sh.hcnt[bin], 1u);
-    }
-}
-
+struct FmScan {                                    // LDS of the block-wide choices
+    unsigned long long wave[FS_THREADS / 64];
+    unsigned long long above;
+    unsigned int bin;
+};
 // Inclusive prefix sums over the 64 lanes of a wave.
 template <typename I>
 __device__ __forceinline__ I fs_wave_scan(I v) {
@@ -716,69 +723,296 @@ __device__ __forceinline__ I fs_wave_scan(I v) {
     }
     return v;
 }
-
-// Bin choice of one radix level, by wave 0 (bins in descending order, 4 per lane: lane l holds 255 - 4l - j).
-// MASS: the first bin at which above + (mass of the bins before it, inclusive) exceeds `target`; sh.above = the mass
-// before that bin.  !MASS: the first bin at which the running count reaches `rem`; sh.redu[0] = rem minus the count
-// before it.  Same choice as walking the bins one by one from 255 down.
-template <bool MASS>
-__device__ __forceinline__ void fs_choose_bin(FsShared &sh, unsigned long long above, unsigned long long target,
-                                              unsigned int rem) {
-    if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x;
-    unsigned long long v[4], ls = 0;
+// The block's sum of v and, in excl, the sum over the earlier threads.
+__device__ __forceinline__ unsigned long long fm_block_scan(unsigned long long v, unsigned long long &excl, FmScan &sc) {
+    const int w = threadIdx.x >> 6;
+    const unsigned long long incl = fs_wave_scan<unsigned long long>(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 63) sc.wave[w] = incl;
+    __syncthreads();
+    unsigned long long before = 0, total = 0;
+    for (int i = 0; i < FS_THREADS / 64; ++i) {
+        const unsigned long long t = sc.wave[i];
+        before += i < w ? t : 0ull;
+        total += t;
+    }
+    excl = before + incl - v;
+    return total;
+}
+// Choice over NB bins in descending order (thread t holds bins NB - 1 - t PB - j): the first bin at which `above` plus
+// the bins before it and the bin itself exceeds `target` (for counts: reaches target + 1); every thread gets the bin
+// and the sum before it.  No such bin (a degenerate row): bin 0.
+template <int NB, typename H>
+__device__ __forceinline__ unsigned int fm_choose(const H *h, unsigned long long above, unsigned long long target,
+                                                  unsigned long long &above_out, FmScan &sc) {
+    constexpr int PB = NB / FS_THREADS;
+    unsigned long long v[PB], ls = 0, excl;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int b = 255 - 4 * lane - j;
-        v[j] = MASS ? sh.hmass[b] : (unsigned long long)sh.hcnt[b];
+    for (int j = 0; j < PB; ++j) {
+        v[j] = h[NB - 1 - (int)threadIdx.x * PB - j];
         ls += v[j];
     }
-    const unsigned long long incl = fs_wave_scan<unsigned long long>(ls);
-    const bool hit = MASS ? above + incl > target : incl >= (unsigned long long)rem;
-    const unsigned long long m = __ballot(hit);
-    const int L = m ? __ffsll((long long)m) - 1 : 63;
-    if (lane == L) {
-        unsigned long long a = (MASS ? above : 0ull) + (incl - ls);
-        int chosen = 255 - 4 * lane - 3;
-        bool found = false;
+    const unsigned long long total = fm_block_scan(ls, excl, sc);
+    if (threadIdx.x == 0) { sc.bin = 0; sc.above = above + total; }
+    __syncthreads();
+    if (above + excl <= target && above + excl + ls > target) {
+        unsigned long long a = above + excl;
+        int bin = NB - 1 - (int)threadIdx.x * PB;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (found) continue;
-            const bool take = MASS ? a + v[j] > target : a + v[j] >= (unsigned long long)rem;
-            if (take) { chosen = 255 - 4 * lane - j; found = true; }
-            else a += v[j];
-        }
-        if (!found) a -= v[3];     // walked past the lane's last bin: that bin is the choice (the serial walk ends there)
-        sh.sel_bin = (unsigned)chosen;
-        if (MASS) sh.above = a;
-        else sh.redu[0] = rem - (unsigned)a;
+        for (int j = 0; j < PB - 1; ++j)
+            if (a + v[j] <= target && bin == NB - 1 - (int)threadIdx.x * PB - j) { a += v[j]; --bin; }
+        sc.bin = (unsigned)bin;
+        sc.above = a;
     }
+    __syncthreads();
+    above_out = sc.above;
+    const unsigned int bin = sc.bin;
+    __syncthreads();
+    return bin;
+}
+template <typename H>
+__device__ __forceinline__ unsigned long long fm_total(const H *h, FmScan &sc) {
+    unsigned long long s = 0, e;
+    for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS) s += h[b];
+    return fm_block_scan(s, e, sc);
 }
 
-// Block sum of a 64-bit integer (exact, any order).
-__device__ __forceinline__ unsigned long long fs_block_sum(unsigned long long v, FsShared &sh) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh.red64[w] = v;
-    __syncthreads();
-    unsigned long long t = 0;
-    for (int i = 0; i < FS_THREADS / 64; ++i) t += sh.red64[i];
-    return t;
+// Histogram add with the lanes that share the first active lane's bin combined: most keys of a row share their top
+// bits, and 64 lanes adding to one LDS word serialise.  Integer sums: the result is order-independent.
+template <typename H>
+__device__ __forceinline__ void fm_add(H *h, bool act, int bin, H v) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long pend = __ballot(act);
+    if (pend == 0) return;
+    const int leader = __ffsll((long long)pend) - 1;
+    const bool mine = act && bin == __shfl(bin, leader);
+    H s = mine ? v : (H)0;
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == leader) atomicAdd(&h[bin], s);
+    else if (act && !mine) atomicAdd(&h[bin], v);
 }
 
-// Index of the rank-th token (index order) whose key equals `key` (a block-wide scan over contiguous chunks).
-__device__ int fs_index_of(const float *row, int V, float T, uint32_t key, unsigned long long rank, FsShared &sh) {
-    const int C = (V + FS_THREADS - 1) / FS_THREADS, lo = threadIdx.x * C, hi = min(V, lo + C);
+// The entries a level looks at: a list in LDS, or (list too long) the whole row.
+struct FmSource {
+    bool listed;
+    int n;
+    const FmPair *pairs;
+    const float *row;
+    float T;
+    // fn(active, key, index) for every entry, by all threads together
+    template <typename F>
+    __device__ __forceinline__ void each(F &&fn) const {
+        for (int i0 = 0; i0 < n; i0 += FS_THREADS) {
+            const int i = i0 + threadIdx.x;
+            const bool in = i < n;
+            uint32_t key = 0;
+            int idx = 0;
+            if (in && listed) { key = pairs[i].key; idx = pairs[i].idx; }
+            if (in && !listed) { key = fs_key(__fdiv_rn(row[i], T)); idx = i; }
+            fn(in, key, idx);
+        }
+    }
+};
+// List `which` of row r into LDS, or the row when the list overflowed.
+__device__ __forceinline__ FmSource fm_source(const FmArgs &a, int r, int which, const float *row, FmPair *lds) {
+    const unsigned int n = a.st[r].n[which];
+    FmSource s{n <= (unsigned)FM_CAP, n <= (unsigned)FM_CAP ? (int)n : a.V, lds, row, a.T};
+    if (s.listed) {
+        const FmPair *src = a.list + ((size_t)which * FM_ROWS + r) * FM_CAP;
+        for (int i = threadIdx.x; i < s.n; i += FS_THREADS) lds[i] = src[i];
+    }
+    __syncthreads();
+    return s;
+}
+// The key that holds `target` among the entries of bin `bin` (first level) with key >= kmin, and the mass (COUNT: the
+// number of entries) before it in sorted order.
+template <bool COUNT>
+__device__ __forceinline__ uint32_t fm_descend(const FmSource &src, uint32_t bin, uint32_t kmin, float zmax,
+                                               unsigned long long above, unsigned long long target,
+                                               unsigned long long &above_out, unsigned long long *h, FmScan &sc) {
+    uint32_t prefix = bin;
+#pragma unroll
+    for (int level = 0; level < 2; ++level) {
+        const int hi = level == 0 ? 20 : 10, lo = hi - 10;
+        for (int b = threadIdx.x; b < FM_B1; b += FS_THREADS) h[b] = 0ull;
+        __syncthreads();
+        src.each([&](bool in, uint32_t key, int) {
+            const bool act = in && (key >> hi) == prefix && key >= kmin;
+            unsigned long long m = 1ull;
+            if constexpr (!COUNT) m = act ? fs_mass(fs_unkey(key), zmax) : 0ull;
+            fm_add<unsigned long long>(h, act, (key >> lo) & (FM_B1 - 1), m);
+        });
+        __syncthreads();
+        prefix = (prefix << 10) | fm_choose<FM_B1>(h, above, target, above, sc);
+    }
+    above_out = above;
+    return prefix;
+}
+
+__global__ void __launch_bounds__(FS_THREADS) k_fm_top(FmArgs a) {
+    __shared__ unsigned int red[FS_THREADS / 64];
+    __shared__ unsigned int h[FM_B0];
+    const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
+    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    float lv[FM_U];
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
+    if (a.top_k) {
+        for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS) h[b] = 0u;
+        __syncthreads();
+    }
+    uint32_t k = 0;
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) {
+        const uint32_t key = fs_key(__fdiv_rn(lv[u], a.T));
+        const bool in = i0 + u * FS_THREADS + (int)threadIdx.x < a.V;
+        k = max(k, key);                           // an entry past the row repeats the last one
+        if (a.top_k) fm_add<unsigned int>(h, in, key >> 20, 1u);
+    }
+    for (int o = 32; o > 0; o >>= 1) k = max(k, (uint32_t)__shfl_xor((int)k, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = k;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < FS_THREADS / 64; ++i) k = max(k, red[i]);
+        atomicMax(&a.st[r].kmax, k);
+    }
+    if (a.top_k)
+        for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS)
+            if (h[b]) atomicAdd(&a.st[r].cnt[b], h[b]);
+}
+
+// Smallest key kept by top-k: the krem-th largest of the boundary bin.
+__device__ __forceinline__ uint32_t fm_kmin(const FmArgs &a, int r, const FmSource &src, unsigned long long *h, FmScan &sc) {
+    unsigned long long above;
+    return fm_descend<true>(src, a.st[r].kbin, 0u, 0.f, 0ull, (unsigned long long)a.st[r].krem - 1, above, h, sc);
+}
+
+// Mass histogram of the kept entries (after top-k: those of at least kmin, found from list 0 by every block).
+template <bool TOPK>
+__global__ void __launch_bounds__(FS_THREADS) k_fm_mass(FmArgs a) {
+    __shared__ unsigned long long m0[FM_B0];
+    __shared__ unsigned long long h[TOPK ? FM_B1 : 1];
+    __shared__ FmPair lds[TOPK ? FM_CAP : 1];
+    __shared__ FmScan sc;
+    const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
+    FmState &S = a.st[r];
+    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    float lv[FM_U];
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
+    for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS) m0[b] = 0ull;
+    uint32_t kmin = 0;
+    if constexpr (TOPK) {
+        const FmSource src = fm_source(a, r, 0, row, lds);
+        kmin = fm_kmin(a, r, src, h, sc);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) S.kmin = kmin;
+    __syncthreads();
+    const float zmax = fs_unkey(S.kmax);
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) {
+        const float z = __fdiv_rn(lv[u], a.T);
+        const uint32_t key = fs_key(z);
+        const bool in = i0 + u * FS_THREADS + (int)threadIdx.x < a.V && key >= kmin;
+        const unsigned long long m = in ? fs_mass(z, zmax) : 0ull;
+        fm_add<unsigned long long>(m0, m != 0ull, key >> 20, m);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS)
+        if (m0[b]) atomicAdd(&S.mass[b], m0[b]);
+}
+
+// What the top-p cut keeps: floor(top_p F) of the kept mass F is the target of the cut.
+__device__ __forceinline__ bool fm_cut(const FmArgs &a, unsigned long long F, unsigned long long &tp) {
+    tp = (unsigned long long)(a.top_p * (double)F);
+    return a.top_p < 1.0 && tp < F;
+}
+__device__ __forceinline__ unsigned long long fm_target(const FmArgs &a, int r, unsigned long long K) {
+    unsigned long long t = (unsigned long long)(a.u[a.row0 + r] * (double)K);
+    return t >= K ? K - 1 : t;
+}
+// The kept mass after the cut: the tokens before the cut's key and those of the key up to the cut.
+__device__ __forceinline__ unsigned long long fm_kept(uint32_t key, float zmax, unsigned long long above,
+                                                      unsigned long long tp) {
+    const unsigned long long m = fs_mass(fs_unkey(key), zmax);
+    return above + ((m > 0 ? (tp - above) / m : 0) + 1) * m;
+}
+
+// Collects entries of a row into a list.  MODE 0: the boundary bin of top-k and every bin above it; 1: the boundary bin
+// alone; 2: the bin of the top-p cut; 3: the bin of the draw (with top-p: after the cut, resolved from list 1).
+template <int MODE>
+__global__ void __launch_bounds__(FS_THREADS) k_fm_gather(FmArgs a) {
+    constexpr int WHICH = MODE <= 1 ? 0 : MODE - 1;
+    __shared__ unsigned long long h[MODE == 3 ? FM_B1 : 1];
+    __shared__ FmPair lds[MODE == 3 ? FM_CAP : 1];
+    __shared__ FmScan sc;
+    __shared__ unsigned int base;
+    const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
+    FmState &S = a.st[r];
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    float lv[FM_U];
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
+    unsigned long long above;
+    uint32_t bin, kmin = 0;
+    if constexpr (MODE <= 1) {
+        bin = fm_choose<FM_B0>(S.cnt, 0ull, (unsigned long long)a.top_k - 1, above, sc);
+        if (lead) { S.kbin = bin; S.krem = (unsigned)a.top_k - (unsigned)above; }
+    } else {
+        kmin = S.kmin;
+        const unsigned long long F = fm_total(S.mass, sc);
+        unsigned long long tp;
+        const bool cut = fm_cut(a, F, tp);
+        if constexpr (MODE == 2) {
+            if (lead) { S.topp = cut; S.tp = tp; }
+            if (!cut) return;
+            bin = fm_choose<FM_B0>(S.mass, 0ull, tp, above, sc);
+            if (lead) { S.tbin = bin; S.tabove = above; }
+        } else {
+            unsigned long long K = F;
+            if (cut) {
+                const float zmax = fs_unkey(S.kmax);
+                const FmSource src = fm_source(a, r, 1, row, lds);
+                const uint32_t key = fm_descend<false>(src, S.tbin, kmin, zmax, S.tabove, tp, above, h, sc);
+                K = fm_kept(key, zmax, above, tp);
+            }
+            const unsigned long long tgt = fm_target(a, r, K);
+            bin = fm_choose<FM_B0>(S.mass, 0ull, tgt, above, sc);
+            if (lead) { S.dbin = bin; S.dabove = above; S.tgt = tgt; }
+        }
+    }
+    uint32_t key[FM_U];
+    unsigned int mine = 0;
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u) {
+        key[u] = fs_key(__fdiv_rn(lv[u], a.T));
+        const bool in = i0 + u * FS_THREADS + (int)threadIdx.x < a.V;
+        const bool take = in && (MODE == 0 ? (key[u] >> 20) >= bin : (key[u] >> 20) == bin && key[u] >= kmin);
+        mine |= (unsigned)take << u;
+    }
+    unsigned long long excl;
+    const unsigned int total = (unsigned)fm_block_scan((unsigned long long)__popc(mine), excl, sc);
+    if (threadIdx.x == 0) base = total ? atomicAdd(&S.n[WHICH], total) : 0u;
+    __syncthreads();
+    FmPair *list = a.list + ((size_t)WHICH * FM_ROWS + r) * FM_CAP;
+    unsigned int at = base + (unsigned)excl;
+#pragma unroll
+    for (int u = 0; u < FM_U; ++u)
+        if ((mine >> u) & 1u) {
+            if (at < (unsigned)FM_CAP) list[at] = FmPair{key[u], i0 + u * FS_THREADS + (int)threadIdx.x};
+            ++at;
+        }
+}
+
+// Index of the rank-th token (index order) whose key equals `key` (a block-wide scan over contiguous chunks), -1 when
+// there is none.
+__device__ int fs_index_of(const float *row, int V, float T, uint32_t key, unsigned long long rank, FmScan &sc) {
+    const int C = (V + FS_THREADS - 1) / FS_THREADS, lo = min(V, (int)threadIdx.x * C), hi = min(V, lo + C);
     unsigned int cnt = 0;
     for (int i = lo; i < hi; ++i) cnt += fs_key(__fdiv_rn(row[i], T)) == key;
-    // exclusive prefix of the counts over the threads, in thread order: wave scans, then the earlier waves' totals
-    const unsigned int incl = fs_wave_scan<unsigned int>(cnt);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 63) sh.scan[w] = incl;
-    __syncthreads();
-    unsigned long long before = incl - cnt;
-    for (int j = 0; j < w; ++j) before += sh.scan[j];
+    unsigned long long before;
+    (void)fm_block_scan(cnt, before, sc);
     __shared__ int found;
     if (threadIdx.x == 0) found = -1;
     __syncthreads();
@@ -794,252 +1028,66 @@ __device__ int fs_index_of(const float *row, int V, float T, uint32_t key, unsig
     return found;
 }
 
-// ---------------------------------------------------------------------------------------------------------------
-// The launches: one block covers FM_SPAN consecutive entries of a row (19 blocks for 151936 entries),
-// so every pass over the row runs on the whole chip instead of one CU.  Each launch first repeats the bin choice of
-// the previous level (every block from the same global histogram, so every block takes the same choice; block 0
-// also records it for the later launches), then histograms its entries into LDS and adds the block's bins to the
-// level's global histogram with integer atomics (exact, order-independent).  Launches per draw batch: init, max,
-// 4 top-k levels (when top-k applies), the candidates' first level, 3 top-p levels (when top-p applies), 3 draw
-// levels, finish.  The scratch (histograms and per-row state) is the library's, one set per device: calls on one
-// device must not overlap.
-#ifndef SP_FM_U
-#define SP_FM_U 8
-#endif
-constexpr int FM_U = SP_FM_U;                      // entries per thread and pass
-constexpr int FM_SPAN = FS_THREADS * FM_U;         // entries of a row per block
-constexpr int FM_ROWS = 256;                       // rows per launch sequence (the scratch holds this many)
-enum { FM_TOPK = 0, FM_H1 = 4, FM_TOPP = 5, FM_DRAW = 8, FM_NLEV = 11 };
-struct FmHist {
-    unsigned long long mass[256];
-    unsigned int cnt[256];
-    unsigned int idx[256];                         // last level: the smallest index in each bin
-};
-struct FmState {
-    unsigned int kmax, kmin;
-    unsigned int prefix[FM_NLEV];                  // key bits chosen above the level's shift
-    unsigned int rem[4];                           // top-k: tokens still to count inside the prefix
-    unsigned long long above[FM_NLEV];             // mass before the prefix (sorted order)
-    unsigned long long F, tp, K, tgt;
-    int topp;                                      // 1: the top-p cut applies (tp < F)
-};
-struct FmArgs {
-    const float *logits;
-    int V, ld;
-    const int *rows;
-    const double *u;
-    float T;
-    int top_k;                                     // > 0 and < V: the top-k levels ran
-    double top_p;                                  // < 1: the top-p levels ran
-    int *out;
-    FmHist *hist;                                  // [FM_ROWS][FM_NLEV]
-    FmState *st;                                   // [FM_ROWS]
-    int row0;                                      // draws row0 .. row0 + gridDim.y - 1 (blockIdx.y = draw - row0)
-};
-
-__global__ void __launch_bounds__(256) k_fm_init(FmArgs a) {
-    const int r = blockIdx.x;
-    unsigned int *h = (unsigned int *)(a.hist + (size_t)r * FM_NLEV);
-    constexpr int W = sizeof(FmHist) / 4, IDX0 = (256 * 8 + 256 * 4) / 4;
-    for (int i = threadIdx.x; i < FM_NLEV * W; i += blockDim.x) h[i] = (i % W) >= IDX0 ? 0xffffffffu : 0u;
-    unsigned int *s = (unsigned int *)(a.st + r);
-    for (int i = threadIdx.x; i < (int)(sizeof(FmState) / 4); i += blockDim.x) s[i] = 0u;
-}
-
-__global__ void __launch_bounds__(FS_THREADS) k_fm_max(FmArgs a) {
-    __shared__ unsigned int red[FS_THREADS / 64];
-    const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
-    float lv[FM_U];
-#pragma unroll
-    for (int u = 0; u < FM_U; ++u) {
-        const int i = i0 + u * FS_THREADS + threadIdx.x;
-        lv[u] = i < a.V ? row[i] : -INFINITY;
-    }
-    uint32_t k = 0;
-#pragma unroll
-    for (int u = 0; u < FM_U; ++u) k = max(k, fs_key(__fdiv_rn(lv[u], a.T)));
-    for (int o = 32; o > 0; o >>= 1) k = max(k, (uint32_t)__shfl_xor((int)k, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = k;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < FS_THREADS / 64; ++i) k = max(k, red[i]);
-        atomicMax(&a.st[r].kmax, k);
-    }
-}
-
-// The level's global histogram into the block's LDS (counts, and masses for a mass level).
-__device__ __forceinline__ void fm_load_hist(FsShared &sh, const FmHist &g, bool mass) {
-    for (int b = threadIdx.x; b < 256; b += FS_THREADS) {
-        sh.hcnt[b] = g.cnt[b];
-        sh.hmass[b] = mass ? g.mass[b] : 0ull;
-    }
-    __syncthreads();
-}
-// One choice of fs_choose_bin on the histogram in LDS; every thread gets (bin, above or rem).
-template <bool MASS>
-__device__ __forceinline__ void fm_choose(FsShared &sh, unsigned long long above, unsigned long long target,
-                                          unsigned int rem, unsigned int &bin, unsigned long long &above_out,
-                                          unsigned int &rem_out) {
-    fs_choose_bin<MASS>(sh, above, target, rem);
-    __syncthreads();
-    bin = sh.sel_bin;
-    above_out = MASS ? sh.above : 0ull;
-    rem_out = MASS ? 0u : sh.redu[0];
-    __syncthreads();
-}
-// Adds this block's entries with (key & mask) == prefix (and key >= kmin) to the level's global histogram by key
-// byte (key >> shift) & 255: counts, masses (MASS), smallest index per bin (IDX).
-template <bool MASS, bool IDX>
-__device__ __forceinline__ void fm_pass(const FmArgs &a, FsShared &sh, const float *row, float zmax, uint32_t kmin,
-                                        uint32_t mask, uint32_t prefix, int shift, FmHist &g) {
-    const int i0 = blockIdx.x * FM_SPAN;
-    float lv[FM_U];
-#pragma unroll
-    for (int u = 0; u < FM_U; ++u) {
-        const int i = i0 + u * FS_THREADS + threadIdx.x;
-        lv[u] = i < a.V ? row[i] : 0.f;
-    }
-    for (int b = threadIdx.x; b < 256; b += FS_THREADS) { sh.hmass[b] = 0ull; sh.hcnt[b] = 0u; sh.hidx[b] = 0xffffffffu; }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < FM_U; ++u) {
-        const int i = i0 + u * FS_THREADS + threadIdx.x;
-        const float z = __fdiv_rn(lv[u], a.T);
-        const uint32_t k = fs_key(z);
-        const bool act = i < a.V && k >= kmin && (k & mask) == prefix;
-        fs_hist_add<MASS>(sh, act, (k >> shift) & 255, MASS && act ? fs_mass(z, zmax) : 0ull);
-        if (IDX && act) atomicMin(&sh.hidx[(k >> shift) & 255], (unsigned)i);
-    }
-    __syncthreads();
-    for (int b = threadIdx.x; b < 256; b += FS_THREADS) {
-        if (sh.hcnt[b] == 0) continue;
-        atomicAdd(&g.cnt[b], sh.hcnt[b]);
-        if (MASS) atomicAdd(&g.mass[b], sh.hmass[b]);
-        if (IDX) atomicMin(&g.idx[b], sh.hidx[b]);
-    }
-}
-__device__ __forceinline__ uint32_t fm_mask(int shift) { return shift >= 24 ? 0u : 0xffffffffu << (shift + 8); }
-
-// Top-k count level j (shift 24 - 8j): the k-th largest key by a radix descent on counts.
-__global__ void __launch_bounds__(FS_THREADS) k_fm_topk(FmArgs a, int j) {
-    __shared__ FsShared sh;
-    const int r = blockIdx.y;
-    FmState &S = a.st[r];
-    FmHist *H = a.hist + (size_t)r * FM_NLEV;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
-    uint32_t prefix = 0, rem = (unsigned)a.top_k;
-    if (j > 0) {
-        fm_load_hist(sh, H[FM_TOPK + j - 1], false);
-        unsigned int bin, rn;
-        unsigned long long ab;
-        fm_choose<false>(sh, 0ull, 0ull, S.rem[j - 1], bin, ab, rn);
-        prefix = S.prefix[FM_TOPK + j - 1] | (bin << (32 - 8 * j));
-        rem = rn;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) { S.prefix[FM_TOPK + j] = prefix; S.rem[j] = rem; }
-    const int shift = 24 - 8 * j;
-    fm_pass<false, false>(a, sh, row, 0.f, 0u, fm_mask(shift), prefix, shift, H[FM_TOPK + j]);
-}
-
-// The candidates' first level (count and mass by the top key byte), after the top-k cut.
-__global__ void __launch_bounds__(FS_THREADS) k_fm_h1(FmArgs a) {
-    __shared__ FsShared sh;
-    const int r = blockIdx.y;
-    FmState &S = a.st[r];
-    FmHist *H = a.hist + (size_t)r * FM_NLEV;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
-    uint32_t kmin = 0;
-    if (a.top_k > 0 && a.top_k < a.V) {
-        fm_load_hist(sh, H[FM_TOPK + 3], false);
-        unsigned int bin, rn;
-        unsigned long long ab;
-        fm_choose<false>(sh, 0ull, 0ull, S.rem[3], bin, ab, rn);
-        kmin = S.prefix[FM_TOPK + 3] | bin;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) S.kmin = kmin;
-    fm_pass<true, false>(a, sh, row, fs_unkey(S.kmax), kmin, 0u, 0u, 24, H[FM_H1]);
-}
-
-// Total mass F of the candidates (sum of the first-level bins).
-__device__ __forceinline__ unsigned long long fm_total(FsShared &sh, const FmHist &h1) {
-    unsigned long long f = 0;
-    for (int b = threadIdx.x; b < 256; b += FS_THREADS) f += h1.mass[b];
-    return fs_block_sum(f, sh);
-}
-
-// Mass-selection level j (shift 16 - 8j) of the top-p cut (DRAW false) or of the draw (DRAW true).
-template <bool DRAW>
-__global__ void __launch_bounds__(FS_THREADS) k_fm_select(FmArgs a, int j) {
-    __shared__ FsShared sh;
-    const int r = blockIdx.y;
-    FmState &S = a.st[r];
-    FmHist *H = a.hist + (size_t)r * FM_NLEV;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
-    const float zmax = fs_unkey(S.kmax);
-    const int base = DRAW ? FM_DRAW : FM_TOPP;
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    unsigned long long target, above;
-    uint32_t prefix;
-    unsigned int bin, rn;
-    if (j == 0) {
-        if (!DRAW) {
-            const unsigned long long F = fm_total(sh, H[FM_H1]);
-            const unsigned long long tp = (unsigned long long)(a.top_p * (double)F);
-            const int on = tp < F;
-            if (lead) { S.F = F; S.tp = tp; S.topp = on; }
-            if (!on) return;
-            target = tp;
-        } else {
-            // the kept mass K: the top-p cut's result when it applied, else the candidates' total
-            unsigned long long K;
-            if (a.top_p < 1.0 && S.topp) {
-                fm_load_hist(sh, H[FM_TOPP + 2], true);
-                fm_choose<true>(sh, S.above[FM_TOPP + 2], S.tp, 0u, bin, above, rn);
-                const uint32_t key = S.prefix[FM_TOPP + 2] | bin;
-                const unsigned long long m = fs_mass(fs_unkey(key), zmax);
-                const unsigned long long rank = m > 0 ? (S.tp - above) / m : 0;
-                K = above + (rank + 1) * m;
-            } else {
-                K = a.top_p < 1.0 ? S.F : fm_total(sh, H[FM_H1]);
-            }
-            unsigned long long tgt = (unsigned long long)(a.u[a.row0 + r] * (double)K);
-            if (tgt >= K) tgt = K - 1;
-            if (lead) { S.K = K; S.tgt = tgt; }
-            target = tgt;
-        }
-        fm_load_hist(sh, H[FM_H1], true);
-        fm_choose<true>(sh, 0ull, target, 0u, bin, above, rn);
-        prefix = bin << 24;
-    } else {
-        if (!DRAW && !S.topp) return;
-        target = DRAW ? S.tgt : S.tp;
-        fm_load_hist(sh, H[base + j - 1], true);
-        fm_choose<true>(sh, S.above[base + j - 1], target, 0u, bin, above, rn);
-        prefix = S.prefix[base + j - 1] | (bin << (24 - 8 * j));
-    }
-    if (lead) { S.prefix[base + j] = prefix; S.above[base + j] = above; }
-    const int shift = 16 - 8 * j;
-    if (shift == 0) fm_pass<true, true>(a, sh, row, zmax, S.kmin, fm_mask(0), prefix, 0, H[base + j]);
-    else fm_pass<true, false>(a, sh, row, zmax, S.kmin, fm_mask(shift), prefix, shift, H[base + j]);
-}
-
-// The drawn token: the last draw level's choice, its rank inside the tie group, and its index.
+// The drawn token.  SMALL: everything after the gather of MODE 0, on the list; else: the draw bin's list (2).  Then the
+// row's scratch is cleared for the next call.
+template <bool SMALL>
 __global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
-    __shared__ FsShared sh;
+    __shared__ unsigned long long m0[SMALL ? FM_B0 : 1];
+    __shared__ unsigned long long h[FM_B1];
+    __shared__ FmPair lds[FM_CAP];
+    __shared__ FmScan sc;
+    __shared__ unsigned int first;
     const int r = blockIdx.x;
     FmState &S = a.st[r];
-    FmHist *H = a.hist + (size_t)r * FM_NLEV;
     const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
     const float zmax = fs_unkey(S.kmax);
-    fm_load_hist(sh, H[FM_DRAW + 2], true);
-    unsigned int bin, rn;
-    unsigned long long above;
-    fm_choose<true>(sh, S.above[FM_DRAW + 2], S.tgt, 0u, bin, above, rn);
-    const uint32_t key = S.prefix[FM_DRAW + 2] | bin;
+    const FmSource src = fm_source(a, r, SMALL ? 0 : 2, row, lds);
+    unsigned long long above, tgt;
+    uint32_t key;
+    if constexpr (SMALL) {
+        const uint32_t kmin = fm_kmin(a, r, src, h, sc);
+        for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS) m0[b] = 0ull;
+        __syncthreads();
+        src.each([&](bool in, uint32_t k, int) {
+            const unsigned long long m = in && k >= kmin ? fs_mass(fs_unkey(k), zmax) : 0ull;
+            fm_add<unsigned long long>(m0, m != 0ull, k >> 20, m);
+        });
+        __syncthreads();
+        unsigned long long K = fm_total(m0, sc), tp;
+        if (fm_cut(a, K, tp)) {
+            const uint32_t bin = fm_choose<FM_B0>(m0, 0ull, tp, above, sc);
+            key = fm_descend<false>(src, bin, kmin, zmax, above, tp, above, h, sc);
+            K = fm_kept(key, zmax, above, tp);
+        }
+        tgt = fm_target(a, r, K);
+        const uint32_t bin = fm_choose<FM_B0>(m0, 0ull, tgt, above, sc);
+        key = fm_descend<false>(src, bin, kmin, zmax, above, tgt, above, h, sc);
+    } else {
+        tgt = S.tgt;
+        key = fm_descend<false>(src, S.dbin, S.kmin, zmax, S.dabove, tgt, above, h, sc);
+    }
     const unsigned long long m = fs_mass(fs_unkey(key), zmax);
-    const unsigned long long rank = m > 0 ? (S.tgt - above) / m : 0;
-    // rank 0 (always, unless the drawn z value is shared by several tokens) is the group's smallest index
-    const int tok = rank == 0 ? (int)H[FM_DRAW + 2].idx[key & 255] : fs_index_of(row, a.V, a.T, key, rank, sh);
-    if (threadIdx.x == 0) a.out[a.row0 + r] = tok;
+    const unsigned long long rank = m > 0 ? (tgt - above) / m : 0;
+    int tok;
+    if (rank == 0) {
+        // always, unless the drawn z value is shared by several tokens: the group's smallest index
+        if (threadIdx.x == 0) first = 0xffffffffu;
+        __syncthreads();
+        src.each([&](bool in, uint32_t k, int idx) {
+            if (in && k == key) atomicMin(&first, (unsigned)idx);
+        });
+        __syncthreads();
+        tok = (int)first;
+    } else {
+        tok = fs_index_of(row, a.V, a.T, key, rank, sc);
+    }
+    if (threadIdx.x == 0) {
+        a.out[a.row0 + r] = tok;
+        S.kmax = 0u;
+        S.n[0] = S.n[1] = S.n[2] = 0u;
+    }
+    for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS) {
+        if (a.top_k) S.cnt[b] = 0u;
+        if (!SMALL) S.mass[b] = 0ull;
+    }
 }
