@@ -416,7 +416,7 @@ void launch_rope(int n, const RopeArgs &ra, int np, hipStream_t st) {
 // ------------------------------------------------------------------------------------------- wide column steps
 // Columns of one wide pass (a prefill of more columns runs in passes of this many).
 constexpr int WIDE_COLS = 2048;
-// Column tiles that a split product's slices may hold together (the partial buffer's size).
+// Columns that a split product's slices may hold together (the partial buffer's size).
 constexpr int WIDE_PART_COLS = 2 * WIDE_COLS;
 
 template <int FMT, int MTW, int RW, int WM, int WN, bool PAIR, bool LO>
@@ -444,22 +444,33 @@ void launch_wide_fmt(int tile, bool pair, wide::GemmArgs &a, int slices, hipStre
     else launch_wide_tile<FMT, false, false>(tile, a, slices, st);
 }
 struct WidePlan { int tile, slices; };
-// The largest tile whose grid fills the 256 CUs; where even the smallest leaves CUs idle, a product whose consumer
-// adds slices is split along K.
+// Tile and k-slices of one product: the pair with the smallest modelled time.  A CU works through its share of the
+// B = tiles x slices blocks one block's time each (ceil(B / 256) rounds, 1/slices of K per round); a grid of at most
+// one block per CU has nothing to overlap its copies and barriers with (a quarter more); smaller tiles do less work per
+// byte copied.  Slices cost the consumer a read and the product a write of every further partial sum (4 TB/s).
+// Only products whose consumer adds slices are split.  Measured (us, best and the rules it replaced: the largest tile
+// with 256 blocks, split only below 256 blocks): Qwen2-1.5B down, 2048 columns 104 (140), 700 columns 45 (77);
+// Qwen2-7B int4 down and o, 777 columns 259 (350) and 53 (67); Qwen2-0.5B fp16 down, 1152 columns 20 (31).
 WidePlan plan_wide(const DevMat &m, int n, bool split_ok) {
-    const int nrg = m.rows_pad / 16;
-    auto blocks = [&](int t) { return ((n + WIDE_BM[t] - 1) / WIDE_BM[t]) * ((nrg * 16 + WIDE_BN[t] - 1) / WIDE_BN[t]); };
-    int tile = 0;
-    while (tile < 2 && blocks(tile) < 256) ++tile;
-    int s = 1;
-    if (split_ok && blocks(tile) < 256) {
-        const int nst = m.cols / 128, ncol = (n + 15) / 16 * 16;
-        s = std::min({256 / blocks(tile), GEMV_MAX_SLICES, WIDE_PART_COLS / ncol, std::max(1, nst / 4)});
-        s = std::max(1, s);
-        const int ks = (nst + s - 1) / s;
-        s = (nst + ks - 1) / ks;
+    const int nrg = m.rows_pad / 16, units = m.cols / 128;       // units: the granularity of a split
+    const double eff[3] = {m.fmt == 3 ? 0.92 : 1.0, 0.9, 0.65};
+    const double rate = m.fmt == 3 ? 1.76e6 : 2.7e6;             // flop per us and CU of a full grid
+    WidePlan best{0, 1};
+    double tbest = 0.0;
+    for (int t = 0; t < 3; ++t) {
+        const long tiles = (long)((n + WIDE_BM[t] - 1) / WIDE_BM[t]) * ((nrg * 16 + WIDE_BN[t] - 1) / WIDE_BN[t]);
+        const double block_us = 2.0 * WIDE_BM[t] * WIDE_BN[t] * m.cols / eff[t] / rate;
+        const int smax = split_ok ? std::min({GEMV_MAX_SLICES, WIDE_PART_COLS / ((n + 15) / 16 * 16), std::max(1, units / 4)}) : 1;
+        for (int s = 1; s <= smax; ++s) {
+            const int ks = (units + s - 1) / s;
+            if ((units + ks - 1) / ks != s) continue;            // every slice has work
+            const long blocks = tiles * s;
+            const double us = (double)((blocks + 255) / 256) / s * (blocks <= 256 ? 1.25 : 1.0) * block_us +
+                              (s - 1) * 8.0 * n * m.rows / 4e6;
+            if (tbest == 0.0 || us < tbest) { tbest = us; best = {t, s}; }
+        }
     }
-    return {tile, s};
+    return best;
 }
 
 // y = W x for n columns (fragment-major x with mtp column tiles).  Returns the slice count the consumer must add (raw

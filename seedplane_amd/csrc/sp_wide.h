@@ -48,7 +48,9 @@ struct Tile {
     static constexpr int S_PER = FMT == 1 ? 0 : 1;
     static constexpr int COPIES = A_PER + W_PER + S_PER;
     static constexpr int STAGE = (A_KIB + W_KIB) * 1024 + S_BYTES;
-    static constexpr int NS = 3 * STAGE <= 160 * 1024 ? 3 : 2;             // stages in LDS
+    // stages in LDS: 3, or 2 where that lets a CU hold a second block (fp16 128 x 128 tiles, whose stage is 32 KiB:
+    // Qwen2-0.5B gate_up over 1152 columns 48.1 -> 40.3 us; their 64 x 64 tiles lose with 2: 31 -> 53 us)
+    static constexpr int NS = (FMT == 1 && MTW * WM >= 8 && !LO) || 3 * STAGE > 160 * 1024 ? 2 : 3;
     static constexpr int SMEM = NS * STAGE;
     static_assert(A_KIB % NW == 0 && W_KIB % NW == 0, "every wave copies the same number of KiB");
     static_assert(FMT == 1 || (S_PIECES >= 1 && S_PIECES <= NW), "one side copy per wave");
