@@ -312,6 +312,14 @@ int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, co
                           const double *u_dev, int32_t n, double temperature, int32_t top_k, double top_p,
                           int32_t *out_dev, void *hip_stream);
 
+/* sp_op_sample_filtered for callers whose uniforms are in host memory and who want the ids there (the same reference
+ * interface and draws): u_host [n], out_host [n], and the row indices either on the device (row_dev) or in host memory
+ * (row_host; exactly one of the two).  The kernels read the uniforms from and write the ids to pinned memory the
+ * library keeps per device, so no copy runs on the stream; the call returns when the stream has finished. */
+int sp_op_sample_filtered_host(const float *logits_dev, int32_t vocab, int32_t ld, const int32_t *row_dev,
+                               const int32_t *row_host, const double *u_host, int32_t n, double temperature,
+                               int32_t top_k, double top_p, int32_t *out_host, void *hip_stream);
+
 /* No counterpart in the reference, whose verifier is greedy only (seedplane/speculative.py:55-92; README.md:69):
  * speculative acceptance over a draft tree with residual resampling.  Node 0 is the root (the last committed
  * token).  The trials of node i are trials_dev[trial_start[i] .. trial_start[i] + n_trials[i]): the child each

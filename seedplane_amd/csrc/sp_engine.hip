@@ -662,9 +662,7 @@ struct sp_engine {
         f16 *xn = nullptr, *xn_lo = nullptr, *attn = nullptr, *act = nullptr, *kn = nullptr, *vn = nullptr;
         char *mem = nullptr, *d_up = nullptr, *h_up = nullptr;      // mem: the allocation that holds all of them
         hipEvent_t up_done = nullptr;
-        // parts of the upload: column records, runs, attention items, ring flags, output columns
-        size_t o_runs = 0, o_items = 0, o_keep = 0, o_out = 0, up_bytes = 0;
-        int max_items = 0;
+        size_t up_bytes = 0;
     } wd;
     void alloc_wide();
     void free_wide();
@@ -1052,12 +1050,10 @@ void sp_engine::alloc_wide() {
     const size_t KV = P * d.n_kv_heads * d.head_dim;
     auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
     // a run of c columns has ceil(c G / rows) attention items: at most one partial item per run (P runs)
-    wd.max_items = (int)(P * (d.n_heads / d.n_kv_heads) / WIDE_ATT_ROWS + P);
-    wd.o_runs = up256(P * sizeof(sp_token));
-    wd.o_items = wd.o_runs + up256(P * sizeof(wide::Run));
-    wd.o_keep = wd.o_items + up256(wd.max_items * sizeof(wide::Item));
-    wd.o_out = wd.o_keep + up256(P * sizeof(int));
-    wd.up_bytes = wd.o_out + up256(P * sizeof(int));
+    const size_t max_items = P * (d.n_heads / d.n_kv_heads) / WIDE_ATT_ROWS + P;
+    // column records, runs, attention items, ring flags, output columns
+    wd.up_bytes = up256(P * sizeof(sp_token)) + up256(P * sizeof(wide::Run)) + up256(max_items * sizeof(wide::Item)) +
+                  2 * up256(P * sizeof(int));
     const size_t sizes[] = {P * H * 4, P * Nqkv * 4, P * NHD * 4, (size_t)WIDE_PART_COLS * std::max<size_t>(H, Nqkv) * 4,
                             P * (d.head_dim / 2) * sizeof(float2), P * H * 2, P * H * 2, P * NHD * 2, P * I * 2, KV * 2, KV * 2,
                             wd.up_bytes};
@@ -1116,18 +1112,23 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
         c = e;
     }
     for (int i = 0; i < n_out; ++i) last_only = last_only && is_last[out_cols[i]];
-    require((int)items.size() <= wd.max_items, SP_EINVAL, "prefill plan out of range");
     // ---- one upload from pinned memory
     HIPCHK(hipEventSynchronize(wd.up_done));
-    std::memcpy(wd.h_up, toks, n * sizeof(sp_token));
-    std::memcpy(wd.h_up + wd.o_runs, runs.data(), runs.size() * sizeof(wide::Run));
-    std::memcpy(wd.h_up + wd.o_items, items.data(), items.size() * sizeof(wide::Item));
-    std::memcpy(wd.h_up + wd.o_keep, keep.data(), n * sizeof(int));
-    if (n_out) std::memcpy(wd.h_up + wd.o_out, out_cols, n_out * sizeof(int));
-    HIPCHK(hipMemcpyAsync(wd.d_up, wd.h_up, wd.up_bytes, hipMemcpyHostToDevice, stream));
+    size_t off = 0;
+    auto put = [&](const void *src, size_t bytes) {
+        const size_t at = off;
+        off = (off + bytes + 255) & ~(size_t)255;
+        require(off <= wd.up_bytes, SP_EINVAL, "prefill plan out of range");
+        if (bytes) std::memcpy(wd.h_up + at, src, bytes);
+        return (const void *)(wd.d_up + at);
+    };
+    const sp_token *dt = (const sp_token *)put(toks, n * sizeof(sp_token));
+    const wide::Run *druns = (const wide::Run *)put(runs.data(), runs.size() * sizeof(wide::Run));
+    const wide::Item *ditems = (const wide::Item *)put(items.data(), items.size() * sizeof(wide::Item));
+    const int *dkeep = (const int *)put(keep.data(), n * sizeof(int));
+    const int *dout = (const int *)put(out_cols, n_out * sizeof(int));
+    HIPCHK(hipMemcpyAsync(wd.d_up, wd.h_up, off, hipMemcpyHostToDevice, stream));
     HIPCHK(hipEventRecord(wd.up_done, stream));
-    const sp_token *dt = (const sp_token *)wd.d_up;
-    const int *dout = (const int *)(wd.d_up + wd.o_out);
     switch (embed.fmt) {
         case 1: launch_embed<1>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
         case 2: launch_embed<2>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
@@ -1150,7 +1151,7 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
         auto commit = [&] {
             if (!to_ring)
                 hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt,
-                                   (const int *)(wd.d_up + wd.o_keep), NKV, HD, n_slots, WIDE_COLS);
+                                   dkeep, NKV, HD, n_slots, WIDE_COLS);
         };
         if (last && n_out == 0) { commit(); break; }
         if (last && last_only) {
@@ -1180,8 +1181,7 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
             HIPCHK(hipGetLastError());
             return;
         }
-        wide::AttnWideArgs aa{wd.q, kc[l], vc[l], wd.kn, wd.vn, dt, (const wide::Run *)(wd.d_up + wd.o_runs),
-                              (const wide::Item *)(wd.d_up + wd.o_items), NH, NKV, n_slots, WIDE_COLS, mtp, scale, wd.attn};
+        wide::AttnWideArgs aa{wd.q, kc[l], vc[l], wd.kn, wd.vn, dt, druns, ditems, NH, NKV, n_slots, WIDE_COLS, mtp, scale, wd.attn};
         const dim3 agrid((unsigned)items.size(), NKV);
         if (HD == 64) launch_attn_wide<64>(G, agrid, stream, aa);
         else launch_attn_wide<128>(G, agrid, stream, aa);
@@ -2150,7 +2150,8 @@ int sp_op_gemv(const sp_weight *w, const void *x_dev, int32_t m_cols, float *y_d
 // sp_library_release (or the process end); each map is guarded by its mutex.
 namespace lib_scratch {
 struct Smp { float *pmax; double *csum; };
-struct Fm { FmState *st; FmPair *list; };
+struct FmHost { double u[FM_ROWS]; int32_t row[FM_ROWS], id[FM_ROWS]; };       // pinned
+struct Fm { FmState *st; FmPair *list; FmHost *host; };
 struct Acc { unsigned long long *xbuf; unsigned *err; int32_t *host; };
 struct Stage { unsigned char *buf = nullptr; size_t cap = 0; hipEvent_t done = nullptr; bool used = false; };
 std::map<int, Smp> smp;
@@ -2197,59 +2198,93 @@ int sp_op_sample(const float *logits_dev, int32_t vocab, int32_t ld, const int32
     });
 }
 
+}  // extern "C"
+
+// Histograms, lists and per-row state for FM_ROWS draws and the pinned block, one set per device (calls on one device
+// must not overlap); zeroed once, each call's last kernel clears what the call used.
+static lib_scratch::Fm filtered_scratch() {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(lib_scratch::fm_mu);
+    auto it = lib_scratch::fm.find(dev);
+    if (it == lib_scratch::fm.end()) {
+        lib_scratch::Fm f{dev_alloc<FmState>(FM_ROWS), nullptr, nullptr};
+        try {
+            f.list = dev_alloc<FmPair>((size_t)3 * FM_ROWS * FM_CAP);
+            HIPCHK(hipHostMalloc((void **)&f.host, sizeof(lib_scratch::FmHost), hipHostMallocDefault));
+            HIPCHK(hipMemset(f.st, 0, FM_ROWS * sizeof(FmState)));
+        } catch (...) {
+            dev_free(f.st);
+            dev_free(f.list);
+            if (f.host) (void)hipHostFree(f.host);
+            throw;
+        }
+        it = lib_scratch::fm.emplace(dev, f).first;
+    }
+    return it->second;
+}
+
+// The launches of at most FM_ROWS draws.
+static void filtered_launch(const lib_scratch::Fm &sc, const float *logits, int vocab, int ld, const int32_t *rows,
+                            const double *u, int n, double temperature, int top_k, double top_p, int32_t *out,
+                            hipStream_t st) {
+    const int k = top_k > 0 && top_k < vocab ? top_k : 0;
+    const FmArgs a{logits, vocab, ld, rows, u, (float)temperature, k, top_p, out, sc.st, sc.list, 0};
+    const dim3 grid((vocab + FM_SPAN - 1) / FM_SPAN, n), block(FS_THREADS);
+    hipLaunchKernelGGL(k_fm_top, grid, block, 0, st, a);
+    if (k && k <= FM_SMALL_K) {
+        hipLaunchKernelGGL(k_fm_gather<0>, grid, block, 0, st, a);
+        hipLaunchKernelGGL(k_fm_finish<true>, dim3(n), block, 0, st, a);
+    } else {
+        if (k) {
+            hipLaunchKernelGGL(k_fm_gather<1>, grid, block, 0, st, a);
+            hipLaunchKernelGGL(k_fm_mass<true>, grid, block, 0, st, a);
+        } else {
+            hipLaunchKernelGGL(k_fm_mass<false>, grid, block, 0, st, a);
+        }
+        if (top_p < 1.0) hipLaunchKernelGGL(k_fm_gather<2>, grid, block, 0, st, a);
+        hipLaunchKernelGGL(k_fm_gather<3>, grid, block, 0, st, a);
+        hipLaunchKernelGGL(k_fm_finish<false>, dim3(n), block, 0, st, a);
+    }
+    HIPCHK(hipGetLastError());
+}
+static void filtered_check(int32_t vocab, int32_t ld, int32_t n, double temperature, double top_p) {
+    require(vocab >= 1 && ld >= vocab && n >= 1 && n <= 65535, SP_EINVAL, "bad sizes");
+    require(temperature > 0.0, SP_EINVAL, "temperature must be positive");
+    require(top_p > 0.0, SP_EINVAL, "top_p must be positive");
+}
+
+extern "C" {
+
 int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, const int32_t *row_dev,
                           const double *u_dev, int32_t n, double temperature, int32_t top_k, double top_p,
                           int32_t *out_dev, void *stream) {
     return guarded(nullptr, [&] {
         require(logits_dev && row_dev && u_dev && out_dev, SP_EINVAL, "NULL pointer");
-        require(vocab >= 1 && ld >= vocab && n >= 1 && n <= 65535, SP_EINVAL, "bad sizes");
-        require(temperature > 0.0, SP_EINVAL, "temperature must be positive");
-        require(top_p > 0.0, SP_EINVAL, "top_p must be positive");
-        hipStream_t st = (hipStream_t)stream;
-        // histograms, lists and per-row state for FM_ROWS draws, one set per device (calls on one device must not
-        // overlap); zeroed once, each call's last kernel clears what the call used
-        int dev = 0;
-        HIPCHK(hipGetDevice(&dev));
-        lib_scratch::Fm sc;
-        {
-            std::lock_guard<std::mutex> lock(lib_scratch::fm_mu);
-            auto it = lib_scratch::fm.find(dev);
-            if (it == lib_scratch::fm.end()) {
-                lib_scratch::Fm f{dev_alloc<FmState>(FM_ROWS), nullptr};
-                try {
-                    f.list = dev_alloc<FmPair>((size_t)3 * FM_ROWS * FM_CAP);
-                    HIPCHK(hipMemset(f.st, 0, FM_ROWS * sizeof(FmState)));
-                } catch (...) {
-                    dev_free(f.st);
-                    dev_free(f.list);
-                    throw;
-                }
-                it = lib_scratch::fm.emplace(dev, f).first;
-            }
-            sc = it->second;
-        }
-        const int nb = (vocab + FM_SPAN - 1) / FM_SPAN;
-        const int k = top_k > 0 && top_k < vocab ? top_k : 0;
+        filtered_check(vocab, ld, n, temperature, top_p);
+        const lib_scratch::Fm sc = filtered_scratch();
+        for (int r0 = 0; r0 < n; r0 += FM_ROWS)
+            filtered_launch(sc, logits_dev, vocab, ld, row_dev + r0, u_dev + r0, std::min(FM_ROWS, n - r0), temperature, top_k,
+                            top_p, out_dev + r0, (hipStream_t)stream);
+    });
+}
+
+int sp_op_sample_filtered_host(const float *logits_dev, int32_t vocab, int32_t ld, const int32_t *row_dev,
+                               const int32_t *row_host, const double *u_host, int32_t n, double temperature,
+                               int32_t top_k, double top_p, int32_t *out_host, void *stream) {
+    return guarded(nullptr, [&] {
+        require(logits_dev && u_host && out_host && (row_dev != nullptr) != (row_host != nullptr), SP_EINVAL,
+                "NULL pointer, or not exactly one of row_dev and row_host");
+        filtered_check(vocab, ld, n, temperature, top_p);
+        const lib_scratch::Fm sc = filtered_scratch();
         for (int r0 = 0; r0 < n; r0 += FM_ROWS) {
             const int nr = std::min(FM_ROWS, n - r0);
-            const FmArgs a{logits_dev, vocab, ld, row_dev, u_dev, (float)temperature, k, top_p, out_dev, sc.st, sc.list, r0};
-            const dim3 grid(nb, nr), block(FS_THREADS);
-            hipLaunchKernelGGL(k_fm_top, grid, block, 0, st, a);
-            if (k && k <= FM_SMALL_K) {
-                hipLaunchKernelGGL(k_fm_gather<0>, grid, block, 0, st, a);
-                hipLaunchKernelGGL(k_fm_finish<true>, dim3(nr), block, 0, st, a);
-            } else {
-                if (k) {
-                    hipLaunchKernelGGL(k_fm_gather<1>, grid, block, 0, st, a);
-                    hipLaunchKernelGGL(k_fm_mass<true>, grid, block, 0, st, a);
-                } else {
-                    hipLaunchKernelGGL(k_fm_mass<false>, grid, block, 0, st, a);
-                }
-                if (top_p < 1.0) hipLaunchKernelGGL(k_fm_gather<2>, grid, block, 0, st, a);
-                hipLaunchKernelGGL(k_fm_gather<3>, grid, block, 0, st, a);
-                hipLaunchKernelGGL(k_fm_finish<false>, dim3(nr), block, 0, st, a);
-            }
-            HIPCHK(hipGetLastError());
+            std::memcpy(sc.host->u, u_host + r0, nr * sizeof(double));
+            if (row_host) std::memcpy(sc.host->row, row_host + r0, nr * sizeof(int32_t));
+            filtered_launch(sc, logits_dev, vocab, ld, row_host ? sc.host->row : row_dev + r0, sc.host->u, nr, temperature, top_k,
+                            top_p, sc.host->id, (hipStream_t)stream);
+            HIPCHK(hipStreamSynchronize((hipStream_t)stream));
+            std::memcpy(out_host + r0, sc.host->id, nr * sizeof(int32_t));
         }
     });
 }
@@ -2442,7 +2477,7 @@ int sp_library_release(void) {
                 HIPCHK(hipDeviceSynchronize());
             }
             for (auto &kv : lib_scratch::smp) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.pmax); dev_free(kv.second.csum); }
-            for (auto &kv : lib_scratch::fm) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.st); dev_free(kv.second.list); }
+            for (auto &kv : lib_scratch::fm) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.st); dev_free(kv.second.list); if (kv.second.host) HIPCHK(hipHostFree(kv.second.host)); }
             for (auto &kv : lib_scratch::acc) {
                 HIPCHK(hipSetDevice(kv.first));
                 dev_free(kv.second.xbuf);

@@ -89,6 +89,16 @@ def _ptr(a):
     return ctypes.c_void_p(a.ctypes.data) if a is not None else None
 
 
+def _id_array(ids):
+    """Token ids (or positions) of any shape and integer-like type as a flat int64 array (reference:
+    torch.as_tensor(ids, dtype=torch.long).flatten(), qwen_engine.py:107)."""
+    if isinstance(ids, list):
+        a = np.array(ids)                      # a list of plain integers, without a tensor in between
+        if a.dtype == np.int64:
+            return a.reshape(-1)
+    return torch.as_tensor(ids, dtype=torch.long).flatten().cpu().numpy()
+
+
 class Qwen2Engine:
     """Inference-only Qwen2/Qwen2.5 runtime with a persistent HBM KV cache (reference: qwen_engine.py:32-166)."""
 
@@ -159,6 +169,7 @@ class Qwen2Engine:
         self._free = []
         self._live = weakref.WeakValueDictionary()     # sequence index -> its live cache
         self._logits_buf = None
+        self._step_buf = None
 
     # ------------------------------------------------------------------------------------------ loading
     @staticmethod
@@ -363,6 +374,27 @@ class Qwen2Engine:
         lo = 0 if cache.window is None else max(0, cpos - cache.window + 1)
         return (int(token), cache.seq, int(rope_pos), cpos % self._pool_slots, lo, cpos, 0, 0, 0)
 
+    def _step_columns(self, tokens, caches):
+        """The columns of one decode step, token i appended to caches[i], for run(): tuples for a few columns, the
+        engine's own record buffer (reused by the next step) for more, filled field by field."""
+        n = len(caches)
+        if n < 4 or n > self.max_tokens:
+            return [self._column(t, c, c.length, c.length) for t, c in zip(tokens, caches)]
+        if self._step_buf is None:
+            self._step_buf = np.zeros(self.max_tokens, dtype=_lib.TOKEN_DTYPE)
+        a = self._step_buf[:n]
+        p = np.array([c.length for c in caches], dtype=np.int64)
+        a['token'] = np.array([int(t) for t in tokens], dtype=np.int64)
+        a['seq'] = [c.seq for c in caches]
+        a['pos'] = a['ctx_hi'] = p
+        a['slot'] = p % self._pool_slots
+        w = [c.window for c in caches]
+        if any(x is not None for x in w):
+            a['ctx_lo'] = np.maximum(0, p + 1 - np.array([1 << 40 if x is None else x for x in w]))
+        else:
+            a['ctx_lo'] = 0
+        return a
+
     def run(self, cols, flags, logits_out=None, want_ids=False):
         """Low-level: one engine call over column tuples (token, seq, pos, slot, ctx_lo, ctx_hi, tree_base,
         tree_count, tree_mask), or a numpy array of _lib.TOKEN_DTYPE.  Returns greedy ids (numpy int32) when
@@ -371,7 +403,7 @@ class Qwen2Engine:
             if cols.dtype != _lib.TOKEN_DTYPE or not cols.flags.c_contiguous:
                 raise ValueError('column array must be a contiguous TOKEN_DTYPE array')
             n = len(cols)
-            arr = cols.ctypes.data_as(ctypes.POINTER(_lib.Token))
+            arr = cols.ctypes.data
         else:
             n = len(cols)
             arr = (_lib.Token * n)(*[_lib.Token(*c) for c in cols])
@@ -388,7 +420,7 @@ class Qwen2Engine:
         a = np.zeros(len(ids), dtype=_lib.TOKEN_DTYPE)
         a['token'] = np.asarray(ids, dtype=np.int64).astype(np.int32)
         a['seq'] = cache.seq
-        a['pos'] = p if positions is None else np.asarray(positions, dtype=np.int64).astype(np.int32)
+        a['pos'] = p if positions is None else positions.astype(np.int32)
         a['slot'] = p % self._pool_slots
         a['ctx_hi'] = p
         if cache.window is not None:
@@ -417,7 +449,7 @@ class Qwen2Engine:
     def forward(self, input_ids, cache=None, all_logits=False, positions=None):
         """Run tokens through the graph (reference: qwen_engine.py:105-144).  `positions` (default: cache slots) are
         the RoPE position ids.  Returns (fp32 logits [q or 1, vocab] on the GPU, cache)."""
-        ids = torch.as_tensor(input_ids, dtype=torch.long).flatten().tolist()
+        ids = _id_array(input_ids)
         if len(ids) == 0:
             raise ValueError('input_ids cannot be empty')
         if cache is None:
@@ -426,10 +458,10 @@ class Qwen2Engine:
         start, qlen = cache.length, len(ids)
         if cache.window is None and start + qlen > cache.capacity:
             raise ValueError(f'KV cache capacity {cache.capacity} exceeded')
-        slots = list(range(start, start + qlen))
-        positions = slots if positions is None else torch.as_tensor(positions, dtype=torch.long).flatten().tolist()
-        if len(positions) != qlen:
-            raise ValueError('positions must match input_ids')
+        if positions is not None:
+            positions = _id_array(positions)
+            if len(positions) != qlen:
+                raise ValueError('positions must match input_ids')
         logits = torch.empty((qlen if all_logits else 1, self.vocab), dtype=torch.float32, device=self.device)
         T = self.max_tokens
         if qlen > T:
@@ -444,18 +476,15 @@ class Qwen2Engine:
                     self._wide(part, [])
             cache.length += qlen
             return logits, cache
-        for c0 in range(0, qlen, T):
-            c1 = min(qlen, c0 + T)
-            cols = [self._column(ids[i], cache, slots[i], positions[i]) for i in range(c0, c1)]
-            last = c1 == qlen
-            if all_logits:
-                self.run(cols, _lib.SP_F_LOGITS, logits_out=logits[c0:c1])
-            elif last:
-                buf = self._scratch_logits(c1 - c0)
-                self.run(cols, _lib.SP_F_LOGITS, logits_out=buf)
-                logits[0].copy_(buf[c1 - c0 - 1])
-            else:
-                self.run(cols, 0)
+        slots = range(start, start + qlen)
+        positions = slots if positions is None else positions.tolist()
+        cols = [self._column(t, cache, s, p) for t, s, p in zip(ids.tolist(), slots, positions)]
+        if all_logits:
+            self.run(cols, _lib.SP_F_LOGITS, logits_out=logits)
+        else:
+            buf = self._scratch_logits(qlen)
+            self.run(cols, _lib.SP_F_LOGITS, logits_out=buf)
+            logits[0].copy_(buf[qlen - 1])
         cache.length += qlen
         return logits, cache
 
@@ -499,12 +528,11 @@ class Qwen2Engine:
         runs as the kernel chain, captured as a graph when `graph`."""
         if len(tokens) != len(caches) or not tokens:
             raise ValueError('one token per cache')
-        cols = []
-        for t, c in zip(tokens, caches):
+        for c in caches:
             self._check_cache(c)
             if c.window is None and c.length + 1 > c.capacity:
                 raise ValueError(f'KV cache capacity {c.capacity} exceeded')
-            cols.append(self._column(t, c, c.length, c.length))
+        cols = self._step_columns(tokens, caches)
         flags = _lib.SP_F_GRAPH if graph else 0
         ids = self.run(cols, flags, logits_out=logits_out, want_ids=True)
         for c in caches:
@@ -540,7 +568,7 @@ class Qwen2Engine:
             k = min(burst, steps - step)
             for j in range(k):
                 feed = step + j > 0
-                cols = [self._column(-1 if feed else int(t), c, c.length, c.length) for t, c in zip(tokens, caches)]
+                cols = self._step_columns([-1] * n if feed else tokens, caches)
                 self.run(cols, flags | (_lib.SP_F_FEED if feed else 0))
                 _lib.check(self.lib.sp_engine_copy_ids(self.h, n, ctypes.c_void_p(base + 4 * n * j)), self.h)
                 for c in caches:
@@ -618,7 +646,7 @@ class Qwen2Engine:
             raise ValueError('logits must be a 2-D fp32 GPU tensor')
         if logits.stride(1) != 1:
             raise ValueError('logits rows must be contiguous (stride 1 along the vocabulary)')
-        u = np.asarray(u, dtype=np.float64).ravel()
+        u = np.ascontiguousarray(u, dtype=np.float64).ravel()
         if rows_dev is None:
             # the kernel reads row rows[s] for every draw s: check every index before the launch
             rows = [int(r) for r in rows]
@@ -631,15 +659,13 @@ class Qwen2Engine:
             # a device row list is the caller's to keep in range (it is not read back to the host)
             raise ValueError('rows_dev must be a 1-D int32 tensor on the logits device with one entry per draw')
         dev = logits.device
-        r = rows_dev if rows_dev is not None else torch.tensor(rows, dtype=torch.int32, device=dev)
-        ud = torch.as_tensor(u).to(dev, non_blocking=False)
-        out = torch.empty(len(ud), dtype=torch.int32, device=dev)
+        host_rows = None if rows_dev is not None else np.array(rows, dtype=np.int32)
+        out = np.empty(len(u), dtype=np.int32)
         stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        _lib.check(self.lib.sp_op_sample_filtered(ctypes.c_void_p(logits.data_ptr()), logits.shape[1],
-                                                  logits.stride(0), ctypes.c_void_p(r.data_ptr()),
-                                                  ctypes.c_void_p(ud.data_ptr()), len(ud), float(temperature),
-                                                  int(top_k), float(top_p), ctypes.c_void_p(out.data_ptr()), stream))
-        return out.cpu().tolist()
+        _lib.check(self.lib.sp_op_sample_filtered_host(
+            logits.data_ptr(), logits.shape[1], logits.stride(0), None if rows_dev is None else rows_dev.data_ptr(),
+            _ptr(host_rows), u.ctypes.data, len(u), float(temperature), int(top_k), float(top_p), out.ctypes.data, stream))
+        return out.tolist()
 
     def _prefill_greedy(self, prompt_ids, cache):
         ids = [int(t) for t in prompt_ids]
@@ -694,28 +720,37 @@ class Qwen2Engine:
     def _prefill_wide(self, prompts, caches, nxt):
         """prefill() of distinct sequences in wide passes: each takes up to WIDE_COLS columns, a prompt cut where a pass
         is full, and ends at most max_tokens prompts (the greedy ids of one call)."""
-        parts, n, ends = [], 0, []              # columns of the pass, their count, (prompt, last column) pairs
+        lens = np.array([len(p) for p in prompts])
+        first = np.cumsum(lens) - lens                       # each prompt's first column
+        total = int(lens.sum())
+        pos = np.arange(total) + np.repeat(np.array([c.length for c in caches]) - first, lens)
+        cols = np.zeros(total, dtype=_lib.TOKEN_DTYPE)
+        cols['token'] = np.fromiter((int(t) for p in prompts for t in p), np.int64, total).astype(np.int32)
+        cols['seq'] = np.repeat([c.seq for c in caches], lens)
+        cols['pos'] = cols['ctx_hi'] = pos
+        cols['slot'] = pos % self._pool_slots
+        if any(c.window is not None for c in caches):
+            w = np.array([1 << 40 if c.window is None else c.window for c in caches])
+            cols['ctx_lo'] = np.maximum(0, pos + 1 - np.repeat(w, lens))
+        c0, ends = 0, []                                     # first column of the pass, prompts that end in it
 
-        def flush():
-            nonlocal parts, n, ends
-            if parts:
-                ids = self._wide(np.concatenate(parts), [c for _, c in ends], want_ids=bool(ends))
-                for (s, _), tid in zip(ends, ids if ends else []):
-                    nxt[s] = int(tid)
-            parts, n, ends = [], 0, []
+        def flush(c1):
+            nonlocal c0, ends
+            ids = self._wide(cols[c0:c1], [first[s] + lens[s] - 1 - c0 for s in ends], want_ids=bool(ends))
+            for s, tid in zip(ends, ids if ends else []):
+                nxt[s] = int(tid)
+            c0, ends = c1, []
 
-        for s, p in enumerate(prompts):
-            cols = self._prompt_columns([int(t) for t in p], caches[s], caches[s].length)
-            c0 = 0
-            while c0 < len(cols):
-                take = min(WIDE_COLS - n, len(cols) - c0)
-                parts.append(cols[c0:c0 + take])
-                c0, n = c0 + take, n + take
-                if c0 == len(cols):
-                    ends.append((s, n - 1))
-                if n == WIDE_COLS or len(ends) == self.max_tokens:
-                    flush()
-        flush()
+        for s in range(len(prompts)):
+            end = int(first[s] + lens[s])
+            while end - c0 > WIDE_COLS:
+                flush(c0 + WIDE_COLS)
+            if lens[s]:
+                ends.append(s)
+            if len(ends) == self.max_tokens:
+                flush(end)
+        if c0 < total:
+            flush(total)
 
     @torch.inference_mode()
     def generate_batch(self, prompts, max_new_tokens=32, eos_token_id=None, window=None, graph=True):
