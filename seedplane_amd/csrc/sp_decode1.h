@@ -1,6 +1,6 @@
 // Persistent one-column decode step: every layer of one new token (embedding, RMSNorms, qkv with bias, RoPE and the
 // K/V write, windowed GQA attention with a split-K combine, o_proj, SwiGLU MLP, residual adds, the final RMSNorm) in
-// one cooperative launch of one block per CU.  The LM head and the argmax then run as the kernel chain's GEMV and
+// one launch of one block per CU.  The LM head and the argmax then run as the kernel chain's GEMV and
 // argmax kernels.  Replaces, for one decode column, the same reference computation as the chain in sp_engine::step
 // (seedplane/qwen_engine.py:117-144; native/vulkan_decode/qwen_vk.cpp:372-412 records the whole step once and
 // submits it once per token).

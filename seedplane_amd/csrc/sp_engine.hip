@@ -606,8 +606,13 @@ struct sp_engine {
     // the fp16 remainders (split_f16) of the normalised GEMV inputs (qkv always; gate_up in one-column steps) and of
     // the SwiGLU activation of one-column steps
     f16 *xn_lo = nullptr, *act_lo = nullptr;
-    float *am_v = nullptr;
-    int *am_i = nullptr, *am_out = nullptr;
+    unsigned long long *am_best = nullptr;      // the argmax's row words and counts (zero between calls)
+    unsigned *am_count = nullptr;
+    int *am_out = nullptr;
+    void launch_ids(int n) {
+        hipLaunchKernelGGL(k_argmax_row, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_best, am_count,
+                           am_out, h_ids);
+    }
     int argmax_cols = 0;         // columns whose argmax ids am_out holds (the last SP_F_ARGMAX call)
     // column descriptors of a call: tokens, attention groups, chunk counts, uploaded together from a pinned staging
     // buffer (one copy per call); `upload_done` marks the copy so the staging buffer is not rewritten before it ran
@@ -617,7 +622,7 @@ struct sp_engine {
     char *d_upload = nullptr, *h_upload = nullptr;
     size_t upload_bytes = 0;
     hipEvent_t upload_done = nullptr;
-    int *h_ids = nullptr;        // pinned landing buffer of the greedy ids a call returns to the host
+    int *h_ids = nullptr;        // pinned: the greedy ids of the last SP_F_ARGMAX call, written by the argmax itself
     // SP_F_DEVCOLS: device arrays the columns' tokens and tree masks are read from (sp_engine_set_device_columns)
     const int32_t *dev_tokens = nullptr;
     const uint64_t *dev_masks = nullptr;
@@ -645,11 +650,10 @@ struct sp_engine {
     d1::Geom d1g{};
     const D1Kernel *d1k = nullptr;
     unsigned long long *d1_ll = nullptr;
-    unsigned *d1_err = nullptr, *h_d1err = nullptr;
+    unsigned *h_d1err = nullptr;     // the error word: pinned, written by a block that gives up
     d1::LayerPtr *d1_layers = nullptr;
     d1::Static *d1_static = nullptr;
     unsigned d1_seq = 0;
-    bool d1_plain = false;       // the runtime refused a cooperative launch once: plain launches from then on
     bool prepare_d1();
     bool launch_d1(const sp_token &t, int flags);     // the persistent kernel alone
     bool run_d1(const sp_token &t, int flags);        // + the error word copy, the head GEMV and the argmax
@@ -694,9 +698,9 @@ struct sp_engine {
 void sp_engine::free_all() {
     drop_graphs();
     free_wide();
-    dev_free(d1_ll); dev_free(d1_err); dev_free(d1_layers); dev_free(d1_static);
+    dev_free(d1_ll); dev_free(d1_layers); dev_free(d1_static);
     if (h_d1err) (void)hipHostFree(h_d1err);
-    d1_ll = nullptr; d1_err = nullptr; d1_layers = nullptr; d1_static = nullptr; h_d1err = nullptr; d1_state = 0;
+    d1_ll = nullptr; d1_layers = nullptr; d1_static = nullptr; h_d1err = nullptr; d1_state = 0;
     for (auto &l : layers) {
         l.qkv.release(); l.o.release(); l.gate_up.release(); l.down.release();
         dev_free(l.qkv_b); dev_free(l.in_norm); dev_free(l.post_norm);
@@ -706,7 +710,7 @@ void sp_engine::free_all() {
     dev_free(final_norm); dev_free(inv_freq);
     for (void *p : {(void *)x, (void *)x2, (void *)qkv, (void *)q, (void *)rtab, (void *)logits, (void *)attn_part, (void *)gpart,
                     (void *)gpart2, (void *)xn, (void *)attn, (void *)xn_lo, (void *)act_lo,
-                    (void *)act, (void *)am_v, (void *)am_i, (void *)am_out,
+                    (void *)act, (void *)am_best, (void *)am_count, (void *)am_out,
                     (void *)d_upload, (void *)d_kl, (void *)d_vl, (void *)d_move})
         dev_free(p);
     for (auto p : kc) dev_free(p);
@@ -744,8 +748,10 @@ void sp_engine::alloc_activations() {
     attn = dev_alloc<f16>(tpad * d.n_heads * d.head_dim);
     act = dev_alloc<f16>(tpad * I);
     logits = dev_alloc<float>((size_t)maxT * V);
-    am_v = dev_alloc<float>((size_t)maxT * ARGMAX_BLOCKS);
-    am_i = dev_alloc<int>((size_t)maxT * ARGMAX_BLOCKS);
+    am_best = dev_alloc<unsigned long long>(maxT);
+    am_count = dev_alloc<unsigned>(maxT);
+    HIPCHK(hipMemset(am_best, 0, maxT * sizeof(unsigned long long)));
+    HIPCHK(hipMemset(am_count, 0, maxT * sizeof(unsigned)));
     am_out = dev_alloc<int>(maxT);
     HIPCHK(hipMemset(am_out, 0, maxT * sizeof(int)));
     argmax_cols = 0;
@@ -1027,10 +1033,7 @@ void sp_engine::step(int n, int flags, const AttnPlan &ap, int l0, int l1) {
         // activation reads
         launch_rmsnorm(n, res, H, gpart, pend, ps, final_norm, d.rms_eps, xn, nullptr, st, mtp);
         launch_gemv(hm, EPI_STORE, xn, H, n, logits, nullptr, d.vocab, nullptr, st, nullptr, 0, PRO_NONE, nullptr, 0, 0, mtp);
-        if (flags & SP_F_ARGMAX) {
-            hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, st, logits, d.vocab, d.vocab, am_v, am_i);
-            hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(64), 0, st, am_v, am_i, am_out);
-        }
+        if (flags & SP_F_ARGMAX) launch_ids(n);
     }
     HIPCHK(hipGetLastError());
 }
@@ -1081,10 +1084,7 @@ void sp_engine::head_rows(int n, float *xrows, int pend, float *logits_dev, bool
     const DevMat &hm = d.tied_head ? embed : head;
     launch_rmsnorm(n, xrows, d.hidden, gpart, pend, gpart_stride, final_norm, d.rms_eps, xn, nullptr, stream, mtp);
     launch_gemv(hm, EPI_STORE, xn, d.hidden, n, logits, nullptr, d.vocab, nullptr, stream, nullptr, 0, PRO_NONE, nullptr, 0, 0, mtp);
-    if (argmax) {
-        hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_v, am_i);
-        hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(64), 0, stream, am_v, am_i, am_out);
-    }
+    if (argmax) launch_ids(n);
     if (logits_dev)
         HIPCHK(hipMemcpyAsync(logits_dev, logits, (size_t)n * d.vocab * sizeof(float), hipMemcpyDeviceToDevice, stream));
 }
@@ -1235,9 +1235,7 @@ bool sp_engine::prepare_d1() {
     d1_ll = nullptr; d1_layers = nullptr; d1_static = nullptr;
     d1_ll = dev_alloc<unsigned long long>(d1g.words);
     HIPCHK(hipMemset(d1_ll, 0, d1g.words * sizeof(unsigned long long)));     // tag 0 is never current
-    if (!d1_err) {
-        d1_err = dev_alloc<unsigned>(1);
-        HIPCHK(hipMemset(d1_err, 0, sizeof(unsigned)));
+    if (!h_d1err) {
         HIPCHK(hipHostMalloc((void **)&h_d1err, sizeof(unsigned), hipHostMallocDefault));
         *h_d1err = 0;
     }
@@ -1258,7 +1256,7 @@ bool sp_engine::prepare_d1() {
     sa.final_norm = final_norm; sa.inv_freq = inv_freq;
     sa.eps = d.rms_eps; sa.scale = 1.0f / std::sqrt((float)d.head_dim);
     sa.ll = d1_ll;
-    sa.err = d1_err;
+    sa.err = h_d1err;
     sa.xn = xn;
     d1_static = dev_alloc<d1::Static>(1);
     HIPCHK(hipMemcpy(d1_static, &sa, sizeof(sa), hipMemcpyHostToDevice));
@@ -1267,13 +1265,28 @@ bool sp_engine::prepare_d1() {
     return true;
 }
 
+// The stream of the last persistent launch on each device.  Two such kernels must not run at once (each needs every CU
+// for one of its blocks): a launch on another stream first waits for that one.  The entry is dropped, after a
+// synchronisation, when an engine leaves a stream, so the stream named here belongs to a live engine.
+namespace {
+struct D1Last { hipStream_t stream = nullptr; hipEvent_t ev = nullptr; bool any = false; };
+std::mutex d1_mu;
+std::map<int, D1Last> d1_last;
+void d1_leave_stream(int device, hipStream_t stream) {
+    std::lock_guard<std::mutex> lock(d1_mu);
+    (void)hipStreamSynchronize(stream);
+    auto it = d1_last.find(device);
+    if (it != d1_last.end() && it->second.stream == stream) it->second.any = false;
+}
+}  // namespace
+
 // One column through the persistent kernel, then the LM head GEMV and the argmax as in the chain.
 // The kernel needs its blocks co-resident (one per CU; the LDS size allows no second one, checked in prepare_d1) but
-// no grid barrier.  It is launched cooperatively; where the runtime refuses that (a second process on the device can
-// find the cooperative-launch resources taken), as a plain launch of the same grid, which an otherwise idle device
-// also places one block per CU.  Either way every wait in the kernel is bounded: a grid that is not all resident
-// ends with the error word set, never a hang.  Returns false, with nothing enqueued, if both launches fail (the step
-// is then marked as not applying and the caller runs the chain).
+// no grid barrier: a plain launch of one block per CU, whose blocks are all placed as soon as the kernels before them
+// have left the CUs.  (A cooperative launch goes through a queue of its own: the head GEMV after it started 11 us
+// later.)  Every wait in the kernel is bounded: a grid that is not all resident ends with the error word set, never a
+// hang.  Returns false, with nothing enqueued, if the launch fails (the step is then marked as not applying and the
+// caller runs the chain).
 bool sp_engine::launch_d1(const sp_token &t, int flags) {
     d1::Step a{};
     a.tok = t;
@@ -1283,32 +1296,29 @@ bool sp_engine::launch_d1(const sp_token &t, int flags) {
     a.seq = d1_seq;
     const d1::Static *sp = d1_static;
     void *args[] = {(void *)&sp, &a};
-    hipError_t le = d1_plain ? hipErrorNotSupported
-                             : hipLaunchCooperativeKernel(d1k->fn, dim3(d1g.nb), dim3(d1::NT), args, d1::SMEM_BYTES, stream);
-    if (le != hipSuccess) {
-        (void)hipGetLastError();
-        d1_plain = true;
-        le = hipLaunchKernel(d1k->fn, dim3(d1g.nb), dim3(d1::NT), args, d1::SMEM_BYTES, stream);
+    std::lock_guard<std::mutex> lock(d1_mu);
+    D1Last &last = d1_last[device];
+    if (last.any && last.stream != stream) {
+        if (!last.ev) HIPCHK(hipEventCreateWithFlags(&last.ev, hipEventDisableTiming));
+        HIPCHK(hipEventRecord(last.ev, last.stream));
+        HIPCHK(hipStreamWaitEvent(stream, last.ev, 0));
     }
+    const hipError_t le = hipLaunchKernel(d1k->fn, dim3(d1g.nb), dim3(d1::NT), args, d1::SMEM_BYTES, stream);
     if (le != hipSuccess) {
         (void)hipGetLastError();
         d1_state = -1;
         d1_why = std::string("launch refused: ") + hipGetErrorString(le);
         return false;
     }
+    last.any = true;
+    last.stream = stream;
     return true;
 }
 bool sp_engine::run_d1(const sp_token &t, int flags) {
     if (!launch_d1(t, flags)) return false;
     const DevMat &hm = d.tied_head ? embed : head;
     launch_gemv(hm, EPI_STORE, xn, d.hidden, 1, logits, nullptr, d.vocab, nullptr, stream);
-    if (flags & SP_F_ARGMAX) {
-        hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_BLOCKS, 1), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_v, am_i);
-        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(64), 0, stream, am_v, am_i, am_out);
-    }
-    // the error word's read-back goes last: a copy between the kernel and the head would delay the head (the word
-    // is checked only after a synchronisation)
-    HIPCHK(hipMemcpyAsync(h_d1err, d1_err, sizeof(unsigned), hipMemcpyDeviceToHost, stream));
+    if (flags & SP_F_ARGMAX) launch_ids(1);
     HIPCHK(hipGetLastError());
     return true;
 }
@@ -1317,7 +1327,6 @@ bool sp_engine::run_d1(const sp_token &t, int flags) {
 void sp_engine::check_d1_error() {
     if (!h_d1err || *(volatile unsigned *)h_d1err == 0) return;
     *(volatile unsigned *)h_d1err = 0;
-    (void)hipMemsetAsync(d1_err, 0, sizeof(unsigned), stream);
     throw Fail{SP_EHIP, "persistent decode step: a block hand-off timed out (the step's results are invalid)"};
 }
 
@@ -1383,7 +1392,7 @@ int sp_engine_create(const sp_model_desc *desc, sp_engine **out) {
 
 void sp_engine_destroy(sp_engine *e) {
     if (!e) return;
-    if (e->stream) (void)hipStreamSynchronize(e->stream);
+    d1_leave_stream(e->device, e->stream);
     e->free_all();
     delete e;
 }
@@ -1392,6 +1401,7 @@ int sp_engine_set_stream(sp_engine *e, void *s) {
     if (!e) { g_err = "engine is NULL"; return SP_EINVAL; }
     return guarded(e, [&] {
         HIPCHK(hipStreamSynchronize(e->stream));
+        d1_leave_stream(e->device, e->stream);
         if (e->own_stream) HIPCHK(hipStreamDestroy(e->stream));
         e->drop_graphs();
         e->stream = (hipStream_t)s;
@@ -1595,12 +1605,11 @@ int sp_engine_forward(sp_engine *e, int32_t n, const sp_token *toks, int32_t fla
         if (n == 1 && (flags & SP_F_LOGITS) && !(flags & (SP_F_UNFUSED | SP_F_CHAIN | SP_F_DEVCOLS)) && t0.tree_count == 0 &&
             t0.ctx_hi >= t0.ctx_lo && t0.slot == t0.ctx_hi % e->n_slots && e->prepare_d1() && e->run_d1(t0, sflags)) {
             e->last_path = 1;
-            e->last_dispatches = (sflags & SP_F_ARGMAX) ? 4 : 2;
+            e->last_dispatches = (sflags & SP_F_ARGMAX) ? 3 : 2;
             if (sflags & SP_F_ARGMAX) e->argmax_cols = 1;
             if (logits_dev)
                 HIPCHK(hipMemcpyAsync(logits_dev, e->logits, (size_t)d.vocab * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
             if (argmax_host) {
-                HIPCHK(hipMemcpyAsync(e->h_ids, e->am_out, sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
                 HIPCHK(hipStreamSynchronize(e->stream));
                 e->check_d1_error();
                 std::memcpy(argmax_host, e->h_ids, sizeof(int32_t));
@@ -1686,8 +1695,6 @@ int sp_engine_forward(sp_engine *e, int32_t n, const sp_token *toks, int32_t fla
         if (logits_dev && (flags & SP_F_LOGITS))
             HIPCHK(hipMemcpyAsync(logits_dev, e->logits, (size_t)n * d.vocab * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
         if (argmax_host) {
-            // through pinned memory: a device-to-host copy into pageable memory is staged by the runtime
-            HIPCHK(hipMemcpyAsync(e->h_ids, e->am_out, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
             HIPCHK(hipStreamSynchronize(e->stream));
             std::memcpy(argmax_host, e->h_ids, n * sizeof(int32_t));
         }
@@ -1731,7 +1738,6 @@ int sp_engine_prefill(sp_engine *e, int32_t n, const sp_token *toks, int32_t n_o
         e->last_dispatches = -1;
         if (argmax_host) {
             e->argmax_cols = n_out;
-            HIPCHK(hipMemcpyAsync(e->h_ids, e->am_out, n_out * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
             HIPCHK(hipStreamSynchronize(e->stream));
             std::memcpy(argmax_host, e->h_ids, n_out * sizeof(int32_t));
         }
@@ -1911,7 +1917,6 @@ int sp_engine_time_persistent(sp_engine *e, const sp_token *tok, int32_t iters, 
         HIPCHK(hipEventElapsedTime(&ms, a, b));
         (void)hipEventDestroy(a);
         (void)hipEventDestroy(b);
-        HIPCHK(hipMemcpy(e->h_d1err, e->d1_err, sizeof(unsigned), hipMemcpyDeviceToHost));
         e->check_d1_error();
         *avg_us = ms * 1000.f / iters;
         // algorithmic bytes: every layer's packed weights (codes + scales), norms and qkv bias, the visible K / V
