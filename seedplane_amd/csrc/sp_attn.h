@@ -677,12 +677,16 @@ __device__ __forceinline__ void argmax_range(const float *x, int lo, int hi, flo
 // 64-bit atomic maximum, the larger value first and the smaller index on equal values (-0 counts as +0); the block that
 // completes the row's count writes the id, also to pinned host memory (host, so that a caller's read-back is no copy of
 // its own), and clears both words for the next call.  Relaxed agent-scope atomics only: the count is raised after the
-// maximum has returned.  One 151936-entry row: 10.8 us as two launches and serial loads, then a 4 us copy of the id.
+// maximum has returned.  gridDim.x: argmax_blocks(cols), one load batch per thread for short rows (their blocks would
+// do little but queue on the row's words).  One 151936-entry row: 10.8 us as two launches and serial loads, then a 4 us copy of the id.
+__host__ __device__ constexpr int argmax_blocks(int cols) {
+    return cols <= 2048 ? 1 : cols >= 2048 * ARGMAX_BLOCKS ? ARGMAX_BLOCKS : (cols + 2047) / 2048;
+}
 __global__ void __launch_bounds__(256) k_argmax_row(const float *x, int cols, int ld, unsigned long long *best,
                                                     unsigned *count, int *out, int *host) {
     __shared__ float sv[4];
     __shared__ int si[4];
-    const int row = blockIdx.y, per = (cols + ARGMAX_BLOCKS - 1) / ARGMAX_BLOCKS;
+    const int row = blockIdx.y, per = (cols + gridDim.x - 1) / gridDim.x;
     const int lo = blockIdx.x * per, hi = min(cols, lo + per);
     float bv = -INFINITY; int bi = 0x7fffffff;
     argmax_range(x + (size_t)row * ld, lo, hi, bv, bi);
@@ -696,7 +700,7 @@ __global__ void __launch_bounds__(256) k_argmax_row(const float *x, int cols, in
     const unsigned long long mine = ((unsigned long long)key << 32) | (uint32_t)~bi;
     unsigned long long prev = __hip_atomic_fetch_max(best + row, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("" : "+v"(prev)::"memory");
-    if (__hip_atomic_fetch_add(count + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != ARGMAX_BLOCKS - 1) return;
+    if (__hip_atomic_fetch_add(count + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
     const unsigned long long all = __hip_atomic_exchange(best + row, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(count + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int id = (int)~(uint32_t)all;

@@ -610,7 +610,7 @@ struct sp_engine {
     unsigned *am_count = nullptr;
     int *am_out = nullptr;
     void launch_ids(int n) {
-        hipLaunchKernelGGL(k_argmax_row, dim3(ARGMAX_BLOCKS, n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_best, am_count,
+        hipLaunchKernelGGL(k_argmax_row, dim3(argmax_blocks(d.vocab), n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_best, am_count,
                            am_out, h_ids);
     }
     int argmax_cols = 0;         // columns whose argmax ids am_out holds (the last SP_F_ARGMAX call)
