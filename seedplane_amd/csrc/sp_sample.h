@@ -725,8 +725,8 @@ __global__ void __launch_bounds__(ACC_T) k_accept_tree(AcceptArgs a) {
 //                 them) and k_fm_finish does the rest on the list, one block per row
 //   otherwise:    [k_fm_gather: the boundary bin of top-k], k_fm_mass: mass histogram of the kept entries,
 //                 [k_fm_gather: the bin of the top-p cut], k_fm_gather: the bin of the draw, k_fm_finish
-// 16 draws over 151936 entries on an MI355X, where each launch costs about 4-7 us and each radix level of 8 bits over
-// the whole row used to be one: see the launch sequence in sp_op_sample_filtered for the measured times.
+// A radix level of 8 bits used to be one launch over whole rows (9 to 14 launches).  16 rows of 151936 logits, device time
+// per call, before and now: top-k 50 + top-p 0.9 87 -> 26 us, top-p 0.9 95 -> 69, temperature only 65 -> 44.
 // A list that would hold more than FM_CAP entries (a row whose logits are mostly equal) is not used: the block that
 // needs it scans the row instead.
 constexpr int FS_THREADS = 1024;
@@ -845,19 +845,50 @@ __device__ __forceinline__ unsigned long long fm_total(const H *h, FmScan &sc) {
     return fm_block_scan(s, e, sc);
 }
 
-// Histogram add with the lanes that share the first active lane's bin combined: most keys of a row share their top
-// bits, and 64 lanes adding to one LDS word serialise.  Integer sums: the result is order-independent.
-template <typename H>
-__device__ __forceinline__ void fm_add(H *h, bool act, int bin, H v) {
+// Wave sum of 64-bit integers on register moves (the exchanges of acc_wave_sum; integer sums need no order).
+__device__ __forceinline__ unsigned long long fm_wave_sum(unsigned long long v) {
+    auto swap = [&](bool half) {
+        const unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
+        const u32x2 l = half ? __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(lo, lo, false, false))
+                             : __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(lo, lo, false, false));
+        const u32x2 h = half ? __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(hi, hi, false, false))
+                             : __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(hi, hi, false, false));
+        v = (((unsigned long long)h[0] << 32) | l[0]) + (((unsigned long long)h[1] << 32) | l[1]);
+    };
+    swap(true);
+    swap(false);
+    auto turn = [&](auto ctrl) {
+        v += (unsigned long long)__double_as_longlong(acc_dpp<decltype(ctrl)::value>(__longlong_as_double((long long)v)));
+    };
+    turn(std::integral_constant<int, 0x128>());
+    turn(std::integral_constant<int, 0x124>());
+    turn(std::integral_constant<int, 0x4E>());
+    turn(std::integral_constant<int, 0xB1>());
+    return v;
+}
+// Histogram add of a mass with the lanes that share the first active lane's bin combined: most keys of a row share
+// their top bits, and 64 lanes adding to one LDS word serialise.  Integer sums: the result is order-independent.
+__device__ __forceinline__ void fm_add(unsigned long long *h, bool act, int bin, unsigned long long v) {
     const int lane = threadIdx.x & 63;
     const unsigned long long pend = __ballot(act);
     if (pend == 0) return;
     const int leader = __ffsll((long long)pend) - 1;
-    const bool mine = act && bin == __shfl(bin, leader);
-    H s = mine ? v : (H)0;
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    const bool mine = act && bin == __builtin_amdgcn_readlane(bin, leader);
+    const unsigned long long s = fm_wave_sum(mine ? v : 0ull);
     if (lane == leader) atomicAdd(&h[bin], s);
     else if (act && !mine) atomicAdd(&h[bin], v);
+}
+
+// fm_add of one count per active lane: the leader's bin gets the number of lanes that share it from the ballot.
+template <typename H>
+__device__ __forceinline__ void fm_count(H *h, bool act, int bin) {
+    const unsigned long long pend = __ballot(act);
+    if (pend == 0) return;
+    const int leader = __ffsll((long long)pend) - 1;
+    const bool mine = act && bin == __builtin_amdgcn_readlane(bin, leader);
+    const unsigned long long same = __ballot(mine);
+    if ((int)(threadIdx.x & 63) == leader) atomicAdd(&h[bin], (H)__popcll(same));
+    else if (act && !mine) atomicAdd(&h[bin], (H)1);
 }
 
 // The entries a level looks at: a list in LDS, or (list too long) the whole row.
@@ -906,9 +937,9 @@ __device__ __forceinline__ uint32_t fm_descend(const FmSource &src, uint32_t bin
         __syncthreads();
         src.each([&](bool in, uint32_t key, int) {
             const bool act = in && (key >> hi) == prefix && key >= kmin;
-            unsigned long long m = 1ull;
-            if constexpr (!COUNT) m = act ? fs_mass(fs_unkey(key), zmax) : 0ull;
-            fm_add<unsigned long long>(h, act, (key >> lo) & (FM_B1 - 1), m);
+            const int b = (key >> lo) & (FM_B1 - 1);
+            if constexpr (COUNT) fm_count(h, act, b);
+            else fm_add(h, act, b, act ? fs_mass(fs_unkey(key), zmax) : 0ull);
         });
         __syncthreads();
         prefix = (prefix << 10) | fm_choose<FM_B1>(h, above, target, above, sc);
@@ -935,7 +966,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_top(FmArgs a) {
         const uint32_t key = fs_key(__fdiv_rn(lv[u], a.T));
         const bool in = i0 + u * FS_THREADS + (int)threadIdx.x < a.V;
         k = max(k, key);                           // an entry past the row repeats the last one
-        if (a.top_k) fm_add<unsigned int>(h, in, key >> 20, 1u);
+        if (a.top_k) fm_count(h, in, key >> 20);
     }
     for (int o = 32; o > 0; o >>= 1) k = max(k, (uint32_t)__shfl_xor((int)k, o));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = k;
@@ -983,7 +1014,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_mass(FmArgs a) {
         const uint32_t key = fs_key(z);
         const bool in = i0 + u * FS_THREADS + (int)threadIdx.x < a.V && key >= kmin;
         const unsigned long long m = in ? fs_mass(z, zmax) : 0ull;
-        fm_add<unsigned long long>(m0, m != 0ull, key >> 20, m);
+        fm_add(m0, m != 0ull, key >> 20, m);
     }
     __syncthreads();
     for (int b = threadIdx.x; b < FM_B0; b += FS_THREADS)
@@ -1096,20 +1127,59 @@ __device__ int fs_index_of(const float *row, int V, float T, uint32_t key, unsig
     return found;
 }
 
-// The drawn token.  SMALL: everything after the gather of MODE 0, on the list; else: the draw bin's list (2).  Then the
-// row's scratch is cleared for the next call.
+// A list of at most one entry per thread, sorted (z descending, ties by ascending index), and everything after the
+// gather on the sorted masses' prefix sums: the top-k cut is entry top_k - 1's key, the top-p cut and the draw are the
+// first entries whose inclusive mass exceeds their targets.  Bitonic over (key, ~index); exchanges inside a wave are
+// shuffles, the others go through LDS.  16 rows of top-k 50 (lists of a few hundred entries): k_fm_finish 23 -> 9.4 us
+// against the histogram descents below.
+__device__ int fm_small_list(const FmArgs &a, int r, const FmSource &src, float zmax, unsigned long long *h, FmScan &sc) {
+    const int t = threadIdx.x;
+    unsigned long long v = 0ull;
+    if (t < src.n) v = ((unsigned long long)src.pairs[t].key << 32) | (uint32_t)~src.pairs[t].idx;
+    for (int k = 2; k < 2 * src.n && k <= FS_THREADS; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            unsigned long long o;
+            if (j < SP_WAVE) {
+                o = __shfl_xor(v, j);
+            } else {
+                __syncthreads();
+                h[t] = v;
+                __syncthreads();
+                o = h[t ^ j];
+            }
+            const bool larger = ((t & k) == 0) == ((t & j) == 0);       // this thread keeps the larger of the pair
+            v = (o > v) == larger ? o : v;
+        }
+    __shared__ unsigned long long pick;        // K, then the drawn entry
+    __syncthreads();
+    h[t] = v;
+    if (t == 0) pick = 0ull;
+    __syncthreads();
+    const uint32_t kmin = (uint32_t)(h[min(a.top_k, src.n) - 1] >> 32), key = (uint32_t)(v >> 32);
+    const unsigned long long m = t < src.n && key >= kmin ? fs_mass(fs_unkey(key), zmax) : 0ull;
+    unsigned long long excl, tp;
+    unsigned long long K = fm_block_scan(m, excl, sc);
+    if (fm_cut(a, K, tp)) {
+        if (excl <= tp && excl + m > tp) pick = excl + m;
+        __syncthreads();
+        K = pick;
+        __syncthreads();
+    }
+    const unsigned long long tgt = fm_target(a, r, K);
+    if (t == 0) pick = 0xffffffff00000000ull;  // no entry (a degenerate row): -1
+    __syncthreads();
+    if (excl <= tgt && excl + m > tgt) pick = v;
+    __syncthreads();
+    return (int)~(uint32_t)pick;
+}
+
+// The drawn token by histogram descents.  SMALL: everything after the gather of MODE 0, on list 0 (m0: a first-level
+// mass histogram); else: the draw, on list 2.
 template <bool SMALL>
-__global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
-    __shared__ unsigned long long m0[SMALL ? FM_B0 : 1];
-    __shared__ unsigned long long h[FM_B1];
-    __shared__ FmPair lds[FM_CAP];
-    __shared__ FmScan sc;
+__device__ int fm_descents(const FmArgs &a, int r, const FmSource &src, const float *row, float zmax, unsigned long long *m0,
+                           unsigned long long *h, FmScan &sc) {
+    const FmState &S = a.st[r];
     __shared__ unsigned int first;
-    const int r = blockIdx.x;
-    FmState &S = a.st[r];
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
-    const float zmax = fs_unkey(S.kmax);
-    const FmSource src = fm_source(a, r, SMALL ? 0 : 2, row, lds);
     unsigned long long above, tgt;
     uint32_t key;
     if constexpr (SMALL) {
@@ -1118,7 +1188,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
         __syncthreads();
         src.each([&](bool in, uint32_t k, int) {
             const unsigned long long m = in && k >= kmin ? fs_mass(fs_unkey(k), zmax) : 0ull;
-            fm_add<unsigned long long>(m0, m != 0ull, k >> 20, m);
+            fm_add(m0, m != 0ull, k >> 20, m);
         });
         __syncthreads();
         unsigned long long K = fm_total(m0, sc), tp;
@@ -1136,19 +1206,32 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
     }
     const unsigned long long m = fs_mass(fs_unkey(key), zmax);
     const unsigned long long rank = m > 0 ? (tgt - above) / m : 0;
+    if (rank > 0) return fs_index_of(row, a.V, a.T, key, rank, sc);
+    // always, unless the drawn z value is shared by several tokens: the group's smallest index
+    if (threadIdx.x == 0) first = 0xffffffffu;
+    __syncthreads();
+    src.each([&](bool in, uint32_t k, int idx) {
+        if (in && k == key) atomicMin(&first, (unsigned)idx);
+    });
+    __syncthreads();
+    return (int)first;
+}
+
+// The drawn token, then the row's scratch is cleared for the next call.
+template <bool SMALL>
+__global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
+    __shared__ unsigned long long m0[SMALL ? FM_B0 : 1];
+    __shared__ unsigned long long h[FM_B1];
+    __shared__ FmPair lds[FM_CAP];
+    __shared__ FmScan sc;
+    const int r = blockIdx.x;
+    FmState &S = a.st[r];
+    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    const float zmax = fs_unkey(S.kmax);
+    const FmSource src = fm_source(a, r, SMALL ? 0 : 2, row, lds);
     int tok;
-    if (rank == 0) {
-        // always, unless the drawn z value is shared by several tokens: the group's smallest index
-        if (threadIdx.x == 0) first = 0xffffffffu;
-        __syncthreads();
-        src.each([&](bool in, uint32_t k, int idx) {
-            if (in && k == key) atomicMin(&first, (unsigned)idx);
-        });
-        __syncthreads();
-        tok = (int)first;
-    } else {
-        tok = fs_index_of(row, a.V, a.T, key, rank, sc);
-    }
+    if (SMALL && src.listed && src.n >= 1 && src.n <= FS_THREADS) tok = fm_small_list(a, r, src, zmax, h, sc);
+    else tok = fm_descents<SMALL>(a, r, src, row, zmax, m0, h, sc);
     if (threadIdx.x == 0) {
         a.out[a.row0 + r] = tok;
         S.kmax = 0u;
