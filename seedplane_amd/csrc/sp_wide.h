@@ -344,11 +344,14 @@ struct AttnWideArgs {
 // sees, 64 at a time: K row-major and V as transposed key pairs in LDS (the conflict-free layout of k_attn_mq), the
 // next 64 keys' loads in flight meanwhile.  Scores take the queries as fp16 value + remainder (two MFMAs per step);
 // the running maximum, sum and output are fp32.  Keys at or past the run's first position come from the staging
-// area, earlier ones from the ring.
+// area, earlier ones from the ring.  Bound by the vector instructions of a chunk's serial chain (load, stage, scores,
+// softmax, P V), not by its matrix work (2048 columns, window 1024, 12 + 2 heads of 128: 14.5 GFLOP with the remainders
+// in 55 us; 65 us with an address per key and a guarded natural exponential per score).
 template <int HD, int G, int RT>
 __global__ void __launch_bounds__(256) k_attn_wide(AttnWideArgs a) {
     constexpr int CH = 64, KP = HD + 8, VP = CH + 8, NST = CH / 16, NS2 = CH / 32, ST = HD / 32, CPR = HD / 8;
     constexpr int KPER = CH * CPR / 256, VPER = CH / 2 * CPR / 256;
+    constexpr float LOG2E = 1.44269504088896340736f;     // scores in units of log 2: the weights are exp2 of differences
     __shared__ __align__(16) f16 k_s[CH][KP];
     __shared__ __align__(16) f16 vt_s[HD][VP];
     __shared__ __align__(16) f16 p_s[4][16][VP];
@@ -362,31 +365,50 @@ __global__ void __launch_bounds__(256) k_attn_wide(AttnWideArgs a) {
     const int lo_all = a.toks[run.first_col + c_last].ctx_lo, hi_all = run.p0 + c_first;
     const size_t ring = ((size_t)run.seq * a.NKV + kvh) * a.n_slots, stage = (size_t)kvh * a.cap + run.first_col;
 
+    // The thread's pieces of a chunk: K piece i is key (tid + 256 i) / CPR, V item i the key pair (tid + 256 i) % (CH / 2).
+    // A chunk that lies in one piece of memory (all of it staged, or in the ring without a wrap: nearly every chunk) is
+    // loaded from one base address; the others (across the first new position, the ring's end or the last key) find
+    // each key's row by itself.
     f16x8 kf[KPER], vf[VPER][2];
     auto load = [&](int k0) {
-        const int base = k0 % a.n_slots;             // slot of key k0
-        auto row = [&](int j) -> size_t {            // key k0 + j (clamped to the block's last key)
+        const int slot0 = k0 % a.n_slots;            // slot of key k0
+        const bool staged = k0 >= run.p0;
+        if (k0 + CH - 1 <= hi && (staged || (k0 + CH <= run.p0 && slot0 + CH <= a.n_slots))) {
+            const size_t base = (staged ? stage + (k0 - run.p0) : ring + slot0) * HD;
+            const f16 *kb = (staged ? a.kn : a.kc) + base, *vb = (staged ? a.vn : a.vc) + base;
+#pragma unroll
+            for (int i = 0; i < KPER; ++i) kf[i] = *(const f16x8 *)(kb + (tid + 256 * i) * 8);
+#pragma unroll
+            for (int i = 0; i < VPER; ++i) {
+                const int idx = tid + 256 * i, kp2 = idx % (CH / 2), ch = idx / (CH / 2);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) vf[i][h] = *(const f16x8 *)(vb + (2 * kp2 + h) * HD + ch * 8);
+            }
+            return;
+        }
+        auto row = [&](int j, bool &st) -> size_t {  // key k0 + j (clamped to the block's last key)
             const int p = min(k0 + j, hi);
-            int s = base + (p - k0);
+            int s = slot0 + (p - k0);
             s = s >= a.n_slots ? s - a.n_slots : s;
             s = a.n_slots >= CH ? s : p % a.n_slots;
-            return p >= run.p0 ? ((stage + (p - run.p0)) * HD) | ((size_t)1 << 63) : (ring + s) * HD;
+            st = p >= run.p0;
+            return (st ? stage + (p - run.p0) : ring + s) * HD;
         };
 #pragma unroll
         for (int i = 0; i < KPER; ++i) {
             const int idx = tid + 256 * i, j = idx / CPR, ch = idx - j * CPR;
-            const size_t o = row(j);
-            const f16 *src = (o >> 63) ? a.kn : a.kc;
-            kf[i] = *(const f16x8 *)(src + (o & ~((size_t)1 << 63)) + ch * 8);
+            bool st;
+            const size_t o = row(j, st);
+            kf[i] = *(const f16x8 *)((st ? a.kn : a.kc) + o + ch * 8);
         }
 #pragma unroll
         for (int i = 0; i < VPER; ++i) {
             const int idx = tid + 256 * i, kp2 = idx % (CH / 2), ch = idx / (CH / 2);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const size_t o = row(2 * kp2 + h);
-                const f16 *src = (o >> 63) ? a.vn : a.vc;
-                vf[i][h] = *(const f16x8 *)(src + (o & ~((size_t)1 << 63)) + ch * 8);
+                bool st;
+                const size_t o = row(2 * kp2 + h, st);
+                vf[i][h] = *(const f16x8 *)((st ? a.vn : a.vc) + o + ch * 8);
             }
         }
     };
@@ -400,7 +422,7 @@ __global__ void __launch_bounds__(256) k_attn_wide(AttnWideArgs a) {
         const int t0 = it.row0 + (wv * RT + rt) * 16;
         const int row = t0 + r16, rowc = min(row, R - 1), col = rowc / G, h = rowc - col * G;
         const float *qp = a.q + (size_t)(run.first_col + col) * a.NH * HD + (kvh * G + h) * HD + 8 * g4;
-        const float qs = row < R ? a.scale : 0.f;
+        const float qs = row < R ? a.scale * LOG2E : 0.f;
 #pragma unroll
         for (int s = 0; s < ST; ++s) {
             const f32x4 x0 = *(const f32x4 *)(qp + 32 * s), x1 = *(const f32x4 *)(qp + 32 * s + 4);
@@ -479,12 +501,13 @@ __global__ void __launch_bounds__(256) k_attn_wide(AttnWideArgs a) {
 #pragma unroll
                 for (int st = 0; st < NST; ++st) mx = fmaxf(mx, sc[rt][st][j]);
                 mx = row16_max(mx);
-                corr[j] = mrow[rt][j] == -INFINITY ? 0.f : __expf(mrow[rt][j] - mx);
+                // a row without a visible key so far has mx = -inf and takes 0 as its reference: its weights are 0
+                const float ref = mx == -INFINITY ? 0.f : mx;
+                corr[j] = __builtin_amdgcn_exp2f(mrow[rt][j] - ref);
                 float ls = 0.f;
 #pragma unroll
                 for (int st = 0; st < NST; ++st) {
-                    // a row without a visible key so far keeps mx = -inf: its weights are 0
-                    const float e = sc[rt][st][j] == -INFINITY ? 0.f : __expf(sc[rt][st][j] - mx);
+                    const float e = __builtin_amdgcn_exp2f(sc[rt][st][j] - ref);
                     p_s[wv][4 * g4 + j][16 * st + r16] = (f16)e;
                     ls += e;
                 }
