@@ -713,7 +713,7 @@ __global__ void __launch_bounds__(ACC_T) k_accept_tree(AcceptArgs a) {
 //         is <= floor(p * F) (first index whose inclusive mass exceeds that, and everything before it);
 //   draw: target = floor(u * K) (clamped below K) over the kept mass K; the token is the first in sorted order whose
 //         inclusive cumulative mass exceeds the target (inverse CDF, Sampler::draw, sampler.hpp:93-97).
-// Selections in sorted order never sort.  The 32-bit order key is split 12 + 10 + 10 bits: a histogram of the top 12
+// Selections in sorted order sort lists of at most FS_THREADS entries only.  The 32-bit order key is split 12 + 10 + 10 bits: a histogram of the top 12
 // bits over the row (counts for the k-th largest, 64-bit masses for a cumulative target; 4096 bins in LDS per block,
 // added into the row's global histogram with integer atomics) names the bin that holds the token looked for, the
 // entries of that bin are gathered into a list, and two 10-bit levels over the list end at one key, whose tokens (equal
