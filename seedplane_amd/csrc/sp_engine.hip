@@ -419,6 +419,17 @@ constexpr int WIDE_COLS = 2048;
 // Columns that a split product's slices may hold together (the partial buffer's size).
 constexpr int WIDE_PART_COLS = 2 * WIDE_COLS;
 
+// RMSNorm of a wide pass's columns (rows and slices 16-byte aligned: H is a multiple of 8, as every width that the
+// fragment order takes)
+void launch_norm_wide(int n, float *x, int H, const float *part, int np, size_t ps, const float *w, float eps, f16 *out,
+                      f16 *out_lo, hipStream_t st, int mtp) {
+    require(H % 8 == 0 && H <= wide::NORM_MAX_H && ps % 4 == 0, SP_EINVAL, "hidden size does not fit the wide norm");
+    by_slices(np, [&](auto c) {
+        hipLaunchKernelGGL((wide::k_norm_wide<decltype(c)::value>), dim3((n + wide::NORM_COLS - 1) / wide::NORM_COLS),
+                           dim3(wide::NORM_COLS * wide::NORM_LANES), 0, st, x, n, part, ps, w, H, eps, out, out_lo, mtp);
+    });
+}
+
 template <int FMT, int MTW, int RW, int WM, int WN, bool PAIR, bool LO>
 void launch_wide_t(wide::GemmArgs &a, int slices, hipStream_t st) {
     using T = wide::Tile<FMT, MTW, RW, WM, WN, LO>;
@@ -1140,7 +1151,7 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
     for (int l = 0; l < d.n_layers; ++l) {
         Layer &ly = layers[l];
         const bool last = l + 1 == d.n_layers;
-        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
+        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
         const int sq = launch_gemm_wide(ly.qkv, EPI_STORE, wd.xn, wd.xn_lo, n, mtp, wd.qkv, nullptr, Nqkv, ly.qkv_b, wd.part, ps,
                                         stream);
         wide::RopeWideArgs ra{RopeArgs{wd.qkv, Nqkv, NH, NKV, HD, wd.rtab, dt, wd.q, kc[l], vc[l], n_slots, wd.part, ps, ly.qkv_b},
@@ -1187,14 +1198,14 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
         else launch_attn_wide<128>(G, agrid, stream, aa);
         commit();
         pend = launch_gemm_wide(ly.o, EPI_RESID, wd.attn, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
-        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
+        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
         launch_gemm_wide(ly.gate_up, EPI_SILU, wd.xn, nullptr, n, mtp, nullptr, wd.act, I, nullptr, nullptr, 0, stream);
         pend = launch_gemm_wide(ly.down, EPI_RESID, wd.act, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
     }
     if (n_out > 0) {
         // every column's final residual is needed: the pending slices go in with the norm (whose output is used when
         // all columns have logits)
-        launch_rmsnorm(n, wd.x, H, wd.part, pend, ps, final_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
+        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, final_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
         bool all = n_out == n && logits_dev && !argmax;
         for (int i = 0; i < n_out; ++i) all = all && out_cols[i] == i;
         if (all) {

@@ -123,3 +123,18 @@ def test_refused_calls(gpu_device):
     assert call(np.zeros(2049, dtype=_lib.TOKEN_DTYPE)) == _lib.SP_ECAPACITY
     with pytest.raises(ValueError):
         eng.forward([1] * 201, eng.new_cache(200) if eng._free else c0)
+
+
+@pytest.mark.parametrize('hidden,heads,kv,n', [(128, 2, 1, 65), (1024, 8, 2, 66), (1152, 9, 3, 67), (2048, 16, 4, 65),
+                                               (2176, 17, 17, 66), (4096, 32, 8, 67)])
+def test_norm_widths(gpu_device, hidden, heads, kv, n):
+    """Hidden sizes at both edges of the wide norm's one, two and four octets per lane, columns that leave its last
+    block of four part empty."""
+    print(f'hidden={hidden} n={n}', flush=True)
+    cfg, w = make_weights(small_cfg(hidden_size=hidden, num_attention_heads=heads, num_key_value_heads=kv), 'q8', seed=7,
+                          scale_std=0.0005)
+    eng, ref = Qwen2Engine(config=cfg, tensors=w, max_tokens=64), RefQwen2(cfg, w)
+    ids = random_prompt(n, cfg['vocab_size'], seed=n)
+    want = ref.forward(ids, ref.new_cache(n), all_logits=True)
+    rows, _ = eng.forward(ids, eng.new_cache(n), all_logits=True)
+    check_rows(rows.cpu(), want, what=f'hidden {hidden}')
