@@ -566,9 +566,10 @@ __device__ __forceinline__ float stream_dot(const Smem &s, Tiles<FMT, T> &tl, in
 // access of the block that it cannot prove disjoint from the copy, inside the layer loop all of them, wait for every
 // outstanding vector memory operation (the cache and hand-off stores included).  The copy completes in order with
 // the wave's other vector memory loads; the reader of the tiles waits for it explicitly (copy_wait).  M0 (the LDS
-// address) is set here; no other code of this kernel uses M0.
+// address) is set here; no other code of this kernel uses M0.  The s_nop is the wait state that the hardware needs between
+// a scalar write of M0 and a copy that reads it (the compiler adds none inside inline asm).
 __device__ __forceinline__ void lds_copy16(const void *g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(lds) : "memory");
 }
 __device__ __forceinline__ void copy_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

@@ -21,12 +21,13 @@ namespace wide {
 // One global-to-LDS copy per lane: lane i's 16 (4) bytes at base + off land at LDS byte address lds + 16 i (4 i).  Inline
 // asm so that the compiler does not track the copies: it would make every LDS read wait for all of them, and the
 // main loop keeps the next stage's copies in flight while it reads the current one.  They complete in order with the
-// wave's other vector memory operations; copies_wait counts them.  M0 (the LDS address) is used by nothing else here.
+// wave's other vector memory operations; copies_wait counts them.  M0 (the LDS address) is used by nothing else here; a
+// scalar write of M0 needs one wait state before a copy reads it, which the compiler does not add inside inline asm.
 __device__ __forceinline__ void copy16(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
 }
 __device__ __forceinline__ void copy4(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void copies_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
