@@ -149,13 +149,14 @@ int sp_engine_forward(sp_engine *e, int32_t n, const sp_token *toks, int32_t fla
 
 /* Replaces the K/V-batch command buffer of the reference's prefill (qwen_vk.cpp:415-437) and the multi-token case of
  * Qwen2Engine.forward (qwen_engine.py:105-144) for prompts: n <= 2048 plain columns (tree_count 0, slot = ctx_hi mod
- * n_slots) through every layer in one pass whose products are tiled over all columns.  The columns are runs of one
- * sequence each at consecutive positions (ctx_hi rises by one, ctx_lo does not fall), every sequence in one run; a run
- * may be longer than the ring (earlier positions of the run are read from a staging area, and the ring ends up with
- * the last n_slots positions).  out_cols[0..n_out) names the columns whose logits are wanted: logits_dev (may be NULL)
- * receives fp32 [n_out][vocab], argmax_host (may be NULL; n_out <= max_tokens) their greedy ids, and the call then
- * waits for the stream.  n_out == 0 writes K/V only.  The engine's buffers for such passes are allocated by its first
- * call. */
+ * n_slots).  The results (logits, ids, K/V) are bit for bit those of sp_engine_forward calls over max_tokens columns each,
+ * in order; chunks of more than 16 columns go through every layer together, in products tiled over all of them.  The
+ * columns are runs of one sequence each at consecutive positions (ctx_hi rises by one, ctx_lo does not fall), every
+ * sequence in one run; a run may be longer than the ring (earlier positions of the run are read from a staging area, and
+ * the ring ends up with the last n_slots positions).  out_cols[0..n_out) names the columns whose logits are wanted:
+ * logits_dev (may be NULL) receives fp32 [n_out][vocab], argmax_host (may be NULL; n_out <= max_tokens) their greedy ids,
+ * and the call then waits for the stream.  n_out == 0 writes K/V only.  The engine's buffers for such passes are allocated
+ * by the first call that needs them; without the memory for them the columns run in chunks. */
 int sp_engine_prefill(sp_engine *e, int32_t n, const sp_token *toks, int32_t n_out, const int32_t *out_cols,
                       float *logits_dev, int32_t *argmax_host);
 

@@ -612,15 +612,16 @@ __global__ void __launch_bounds__(64 * NWV) k_attn_dec(AttnArgs a, f16 *out, int
 // The chunk outputs are read in batches of CMB_BATCH with every load of a batch in flight together (the first batch
 // before the weights are known); the accumulation runs over the chunks in ascending order.
 constexpr int CMB_BATCH = 16;
+// (col0: the launch's first column, whose records stand first in part.)
 __global__ void __launch_bounds__(128) k_attn_combine(const float *part, const int *col_nchunk, int NH, int HD,
-                                                      int nchunk, f16 *out, int ldo, int mtp) {
+                                                      int nchunk, f16 *out, int ldo, int mtp, int col0) {
     __shared__ float w_s[ATT_MAX_CHUNKS];
     __shared__ float l_s[ATT_MAX_CHUNKS];
     __shared__ float red[16];
-    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
+    const int h = blockIdx.x, b = col0 + blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
     const int nc = col_nchunk[b];
     const int rec = part_floats(HD);
-    const float *p = part + ((size_t)b * NH + h) * nchunk * rec;
+    const float *p = part + ((size_t)blockIdx.y * NH + h) * nchunk * rec;
     const int d = min(tid, HD - 1), last = max(nc - 1, 0);     // clamped: every load is in bounds
     float v[CMB_BATCH];
 #pragma unroll
@@ -794,7 +795,8 @@ __global__ void __launch_bounds__(256) k_kv_fill(f16 *const *kl, f16 *const *vl,
 // ring range and tree-mask bits), chunk-local softmax statistics, O = P V.  Partials use the same layout as
 // k_attn_part, so k_attn_combine merges them (with the group's chunk count per column).
 struct AttnGroup {
-    int first_col, ncols, seq, lo, nlin, tree_base, tree_count, pad;
+    int first_col, ncols, seq, lo, nlin, tree_base, tree_count;
+    int run_col, run_pos;  // STAGED: the first column of the sequence's run in the call, and its position
 };
 
 struct AttnMqArgs {
@@ -806,9 +808,17 @@ struct AttnMqArgs {
     float scale;
     float *part;
     int splits;            // blocks per (chunk, kv head, group); block s takes row tiles 4s .. 4s+3
+    // STAGED only
+    const f16 *kn, *vn;    // K and V of the call's columns [kv_head][cap][HD], beside the ring
+    int cap, col0;         // columns the staging area holds; the launch's first column (its records stand first in part)
 };
 
-template <int HD, int G, int CH>
+// STAGED (wide passes): the group's sequence has a run of columns at consecutive positions in the call, whose keys and values
+// are read from the staging area (k_rope_wide); earlier positions are read from the ring.  One block per key chunk: its
+// partial records are what the combine of a step adds up, so a wide pass gives a step's bits.  2048 columns of
+// Qwen2-1.5B, window 1024: 70 us and 31 for the combine (two chunks per block, one after the other on the same queries: 84;
+// one pass with an online softmax, whose bits differ from a step's: 55).
+template <int HD, int G, int CH, bool STAGED = false>
 __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
     constexpr int KP = HD + 8, VP = CH + 8;          // padded rows (halves), 16-byte aligned
     constexpr int NST = CH / 16, NS2 = CH / 32, NP2 = CH / 2;   // key tiles, P.V k-steps, key pairs
@@ -856,6 +866,14 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
         kp = lin ? gr.lo + vis : ~tj;
         return wrap(lin ? lin_base + j : gr.tree_base + tj);
     };
+    const size_t stage_base = STAGED ? (size_t)kvh * a.cap + gr.run_col : 0;
+    // row (of HD values) of visible key j, in the ring or (staged) in the staging area
+    auto row_at = [&](int j, bool &staged) -> size_t {
+        int kp;
+        const int slot = key_at(j, kp);
+        staged = STAGED && kp >= gr.run_pos;
+        return staged ? stage_base + (kp - gr.run_pos) : head_base + slot;
+    };
 
     // ---- every global load before the first LDS store.  Keys past cnt load key 0 of the chunk (clamped address,
     // unconditional load) and are replaced by zeros.  K: item i = key i / CPR, piece i % CPR.  V: item i = key pair
@@ -864,9 +882,9 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
 #pragma unroll
     for (int i = 0; i < KPER; ++i) {
         const int idx = tid + 256 * i, j = idx / CPR, ch = idx - j * CPR;
-        int kp;
-        const int slot = key_at(j < cnt ? j : 0, kp);
-        kf[i] = *(const f16x8 *)(a.kc + (head_base + slot) * HD + ch * 8);
+        bool sg;
+        const size_t row = row_at(j < cnt ? j : 0, sg);
+        kf[i] = *(const f16x8 *)((sg ? a.kn : a.kc) + row * HD + ch * 8);
     }
 #pragma unroll
     for (int i = 0; i < VPER; ++i) {
@@ -874,9 +892,9 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int j = 2 * kp2 + h;
-            int kp;
-            const int slot = key_at(j < cnt ? j : 0, kp);
-            vf[i][h] = *(const f16x8 *)(a.vc + (head_base + slot) * HD + ch * 8);
+            bool sg;
+            const size_t row = row_at(j < cnt ? j : 0, sg);
+            vf[i][h] = *(const f16x8 *)((sg ? a.vn : a.vc) + row * HD + ch * 8);
         }
     }
     // Q fragments (A operand) of row rt*16 + r16, dims 32s + 8*g4 .. +8, from a clamped row; rows past R are zero.
@@ -1032,7 +1050,8 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
         const int row = rt * 16 + 4 * g4 + j;
         if (row < R) {
             const int col = row / G, h = row - col * G;
-            float *out = a.part + (((size_t)(gr.first_col + col) * a.NH + kvh * G + h) * a.nchunk + c) * part_floats(HD);
+            const size_t pcol = gr.first_col + col - (STAGED ? a.col0 : 0);
+            float *out = a.part + ((pcol * a.NH + kvh * G + h) * a.nchunk + c) * part_floats(HD);
             f16 *oh = (f16 *)(out + 2);
             const float il = lrow[j] > 0.f ? 1.f / lrow[j] : 0.f;
 #pragma unroll

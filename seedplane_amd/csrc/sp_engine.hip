@@ -160,6 +160,13 @@ GemvPlan plan_gemv(const DevMat &m, int mt, bool split_ok, int slices = 0, int w
     return p;
 }
 
+// The k-slices of a batch's qkv and o_proj products where they are not plan_gemv's own (0).  Batches of one column tile:
+// 2 (whole steps, 16 columns: Qwen2-1.5B int8 1.422 -> 1.404 ms for qkv, then 1.406 -> 1.398 for o_proj, Qwen2-0.5B fp16
+// -0.8 %; the RoPE kernel and the norm then add 2 slices instead of 8); int4 o_proj at several column tiles: 4 (Qwen2-7B
+// at 32 columns: -0.3 %).
+int qkv_slices(int n) { return n > 1 && n <= 16 ? 2 : 0; }
+int o_slices(int n, int fmt) { return n > 1 && n <= 16 ? 2 : (n > 16 && fmt == 3 ? 4 : 0); }
+
 // LO: several columns whose inputs come with fp16 remainders (a.xlo): a second MFMA per fragment.  One column takes
 // its remainders in MFMA row 1 of the ONE variant instead.
 template <int FMT, int RG, int R, bool LO>
@@ -366,23 +373,23 @@ void launch_attn_rope_hd(int G, dim3 grid, hipStream_t st, const AttnArgs &a, co
 // Keys per multi-query block (one partial record per block and row): 128 for tree groups (verify pass: 33 x 12
 // query rows, fewer and larger blocks, half the records to merge; -1 % per pass), 64 otherwise (the plain batches
 // and prefill chunks got slower with 128: bs16 +16 %, prefill +3 %).
-template <int HD, int CH>
+template <int HD, int CH, bool STAGED>
 void launch_attn_mq_ch(int G, dim3 grid, hipStream_t st, const AttnMqArgs &a) {
     switch (G) {
-        case 1: hipLaunchKernelGGL((k_attn_mq<HD, 1, CH>), grid, dim3(256), 0, st, a); break;
-        case 2: hipLaunchKernelGGL((k_attn_mq<HD, 2, CH>), grid, dim3(256), 0, st, a); break;
-        case 3: hipLaunchKernelGGL((k_attn_mq<HD, 3, CH>), grid, dim3(256), 0, st, a); break;
-        case 4: hipLaunchKernelGGL((k_attn_mq<HD, 4, CH>), grid, dim3(256), 0, st, a); break;
-        case 5: hipLaunchKernelGGL((k_attn_mq<HD, 5, CH>), grid, dim3(256), 0, st, a); break;
-        case 6: hipLaunchKernelGGL((k_attn_mq<HD, 6, CH>), grid, dim3(256), 0, st, a); break;
-        case 7: hipLaunchKernelGGL((k_attn_mq<HD, 7, CH>), grid, dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL((k_attn_mq<HD, 8, CH>), grid, dim3(256), 0, st, a); break;
+        case 1: hipLaunchKernelGGL((k_attn_mq<HD, 1, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 2: hipLaunchKernelGGL((k_attn_mq<HD, 2, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 3: hipLaunchKernelGGL((k_attn_mq<HD, 3, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 4: hipLaunchKernelGGL((k_attn_mq<HD, 4, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 5: hipLaunchKernelGGL((k_attn_mq<HD, 5, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 6: hipLaunchKernelGGL((k_attn_mq<HD, 6, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        case 7: hipLaunchKernelGGL((k_attn_mq<HD, 7, CH, STAGED>), grid, dim3(256), 0, st, a); break;
+        default: hipLaunchKernelGGL((k_attn_mq<HD, 8, CH, STAGED>), grid, dim3(256), 0, st, a); break;
     }
 }
 template <int HD>
 void launch_attn_mq_hd(int G, int ch, dim3 grid, hipStream_t st, const AttnMqArgs &a) {
-    if (ch == 128) launch_attn_mq_ch<HD, 128>(G, grid, st, a);
-    else launch_attn_mq_ch<HD, 64>(G, grid, st, a);
+    if (ch == 128) launch_attn_mq_ch<HD, 128, false>(G, grid, st, a);
+    else launch_attn_mq_ch<HD, 64, false>(G, grid, st, a);
 }
 
 template <class F>
@@ -416,8 +423,8 @@ void launch_rope(int n, const RopeArgs &ra, int np, hipStream_t st) {
 // ------------------------------------------------------------------------------------------- wide column steps
 // Columns of one wide pass (a prefill of more columns runs in passes of this many).
 constexpr int WIDE_COLS = 2048;
-// Columns that a split product's slices may hold together (the partial buffer's size).
-constexpr int WIDE_PART_COLS = 2 * WIDE_COLS;
+// Columns that a split product's slices may hold together (the partial buffer's size): four slices of a full pass.
+constexpr int WIDE_PART_COLS = 4 * WIDE_COLS;
 
 // RMSNorm of a wide pass's columns (rows and slices 16-byte aligned: H is a multiple of 8, as every width that the
 // fragment order takes)
@@ -430,95 +437,97 @@ void launch_norm_wide(int n, float *x, int H, const float *part, int np, size_t 
     });
 }
 
-template <int FMT, int MTW, int RW, int WM, int WN, bool PAIR, bool LO>
+template <int FMT, int MTW, int RW, int WM, int WN, bool PAIR, bool LO, bool SUM>
 void launch_wide_t(wide::GemmArgs &a, int slices, hipStream_t st) {
     using T = wide::Tile<FMT, MTW, RW, WM, WN, LO>;
     a.mblocks = (a.mtp + T::BMT - 1) / T::BMT;
     a.nblocks = (a.nrg + T::BNG - 1) / T::BNG;
-    a.nst = a.nkt / T::TPS;
-    a.kslice = (a.nst + slices - 1) / slices;
-    hipLaunchKernelGGL((wide::k_gemm_wide<FMT, MTW, RW, WM, WN, PAIR, LO>), dim3(a.mblocks * a.nblocks, slices),
+    hipLaunchKernelGGL((wide::k_gemm_wide<FMT, MTW, RW, WM, WN, PAIR, LO, SUM>), dim3(a.mblocks * a.nblocks, slices),
                        dim3(64 * T::NW), T::SMEM, st, a);
 }
 // Block tiles, columns x weight rows: 0: 128 x 128 (8 waves), 1: 64 x 128 (8 waves), 2: 64 x 64 (4 waves).
 constexpr int WIDE_BM[3] = {128, 64, 64}, WIDE_BN[3] = {128, 128, 64};
-template <int FMT, bool PAIR, bool LO>
+template <int FMT, bool PAIR, bool LO, bool SUM>
 void launch_wide_tile(int tile, wide::GemmArgs &a, int slices, hipStream_t st) {
-    if (tile == 0) launch_wide_t<FMT, 4, 2, 2, 4, PAIR, LO>(a, slices, st);
-    else if (tile == 1) launch_wide_t<FMT, 2, 2, 2, 4, PAIR, LO>(a, slices, st);
-    else launch_wide_t<FMT, 2, 2, 2, 2, PAIR, LO>(a, slices, st);
+    if (tile == 0) launch_wide_t<FMT, 4, 2, 2, 4, PAIR, LO, SUM>(a, slices, st);
+    else if (tile == 1) launch_wide_t<FMT, 2, 2, 2, 4, PAIR, LO, SUM>(a, slices, st);
+    else launch_wide_t<FMT, 2, 2, 2, 2, PAIR, LO, SUM>(a, slices, st);
 }
 template <int FMT>
-void launch_wide_fmt(int tile, bool pair, wide::GemmArgs &a, int slices, hipStream_t st) {
-    if (pair) launch_wide_tile<FMT, true, false>(tile, a, slices, st);
-    else if (a.xlo) launch_wide_tile<FMT, false, true>(tile, a, slices, st);
-    else launch_wide_tile<FMT, false, false>(tile, a, slices, st);
+void launch_wide_fmt(int tile, bool pair, bool sum, wide::GemmArgs &a, int slices, hipStream_t st) {
+    if (pair) launch_wide_tile<FMT, true, false, false>(tile, a, slices, st);
+    else if (sum && a.xlo) launch_wide_tile<FMT, false, true, true>(tile, a, slices, st);
+    else if (sum) launch_wide_tile<FMT, false, false, true>(tile, a, slices, st);
+    else if (a.xlo) launch_wide_tile<FMT, false, true, false>(tile, a, slices, st);
+    else launch_wide_tile<FMT, false, false, false>(tile, a, slices, st);
 }
-struct WidePlan { int tile, slices; };
-// Tile and k-slices of one product: the pair with the smallest modelled time.  A CU works through its share of the
-// B = tiles x slices blocks one block's time each (ceil(B / 256) rounds, 1/slices of K per round); a grid of at most
-// one block per CU has nothing to overlap its copies and barriers with (a quarter more); smaller tiles do less work per
-// byte copied.  Slices cost the consumer a read and the product a write of every further partial sum (4 TB/s).
-// Only products whose consumer adds slices are split.  Measured (us, best and the rules it replaced: the largest tile
-// with 256 blocks, split only below 256 blocks): Qwen2-1.5B down, 2048 columns 104 (140), 700 columns 45 (77);
-// Qwen2-7B int4 down and o, 777 columns 259 (350) and 53 (67); Qwen2-0.5B fp16 down, 1152 columns 20 (31).
-WidePlan plan_wide(const DevMat &m, int n, bool split_ok) {
-    const int nrg = m.rows_pad / 16, units = m.cols / 128;       // units: the granularity of a split
+// The order of a product's sums in the step over mt column tiles that a wide pass stands for: k-tiles per slice, waves
+// of a slice, slices that hold any.
+struct WideOrder {
+    int per, nw, slices;
+    bool operator==(const WideOrder &o) const { return per == o.per && nw == o.nw; }
+};
+WideOrder wide_order(const DevMat &m, int mt, bool split_ok, int slices = 0) {
+    const GemvPlan p = plan_gemv(m, mt, split_ok, slices);
+    return {p.kslice, p.nw, (m.nkt + p.kslice - 1) / p.kslice};
+}
+struct WidePlan { int tile; bool split; };
+// Tile of one product, and whether its slices are blocks of their own (whose sums go through memory to the consumer) or
+// formed in turn by one block: the pair with the smallest modelled time.  A CU works through its share of the B blocks one
+// block's time each (ceil(B / 256) rounds); a grid of at most one block per CU has nothing to overlap its copies and
+// barriers with (a quarter more); smaller tiles do less work per byte copied.  Split slices cost the product a write and
+// the consumer a read of every sum (4 TB/s); slices in one block cost it a third set of sums, felt most by fp16 weights,
+// whose products have no other vector work.  qkv is never split (its consumer reads each sum in pieces of 4 bytes).
+// Measured (us with what the consumer adds, split / in one block, the best tile of each): Qwen2-1.5B int8, 2048 columns, down
+// 108 / 136, o 43 / 35, qkv 64 / 46; Qwen2-7B int4, 777 columns, down 280 / 327, o 70 / 72, qkv 136 / 105; Qwen2-0.5B
+// fp16, 980 columns, down 23 / 42, o 13 / 15, qkv 23 / 18.
+WidePlan plan_wide(const DevMat &m, int n, int slices, size_t part_floats) {
+    const int nrg = m.rows_pad / 16;
     const double eff[3] = {m.fmt == 3 ? 0.92 : 1.0, 0.9, 0.65};
     const double rate = m.fmt == 3 ? 1.76e6 : 2.7e6;             // flop per us and CU of a full grid
-    WidePlan best{0, 1};
+    const double sum = slices < 2 || m.fmt == 3 ? 1.0 : m.fmt == 2 ? 1.2 : 2.0;
+    WidePlan best{0, false};
     double tbest = 0.0;
     for (int t = 0; t < 3; ++t) {
         const long tiles = (long)((n + WIDE_BM[t] - 1) / WIDE_BM[t]) * ((nrg * 16 + WIDE_BN[t] - 1) / WIDE_BN[t]);
         const double block_us = 2.0 * WIDE_BM[t] * WIDE_BN[t] * m.cols / eff[t] / rate;
-        const int smax = split_ok ? std::min({GEMV_MAX_SLICES, WIDE_PART_COLS / ((n + 15) / 16 * 16), std::max(1, units / 4)}) : 1;
-        for (int s = 1; s <= smax; ++s) {
-            const int ks = (units + s - 1) / s;
-            if ((units + ks - 1) / ks != s) continue;            // every slice has work
+        for (int split = 0; split < 2; ++split) {
+            if (split && (slices < 2 || (size_t)slices * n * m.rows > part_floats)) continue;
+            const int s = split ? slices : 1;
             const long blocks = tiles * s;
-            const double us = (double)((blocks + 255) / 256) / s * (blocks <= 256 ? 1.25 : 1.0) * block_us +
-                              (s - 1) * 8.0 * n * m.rows / 4e6;
-            if (tbest == 0.0 || us < tbest) { tbest = us; best = {t, s}; }
+            const double us = (double)((blocks + 255) / 256) / s * (blocks <= 256 ? 1.25 : 1.0) * block_us * (split ? 1.0 : sum) +
+                              (split ? s : 0) * 8.0 * n * m.rows / 4e6;
+            if (tbest == 0.0 || us < tbest) { tbest = us; best = {t, split != 0}; }
         }
     }
     return best;
 }
 
-// y = W x for n columns (fragment-major x with mtp column tiles).  Returns the slice count the consumer must add (raw
-// sums in part; plus the bias for EPI_STORE) or 0 when the epilogue was applied.
-int launch_gemm_wide(const DevMat &m, int epi, const f16 *x, const f16 *xlo, int n, int mtp, float *out_f32, f16 *out_f16,
-                     int ldo, const float *bias, float *part, size_t pstride, hipStream_t st) {
+// y = W x for n columns (fragment-major x with mtp column tiles), summed in the given order.  Returns the slice count the
+// consumer must add (raw sums in part, slices n * ldo floats apart) or 0 when the epilogue was applied.
+int launch_gemm_wide(const DevMat &m, const WideOrder &order, int epi, const f16 *x, const f16 *xlo, int n, int mtp,
+                     float *out_f32, f16 *out_f16, int ldo, const float *bias, float *part, size_t part_floats, hipStream_t st) {
     require((epi == EPI_SILU) == m.paired, SP_EINVAL, "gemm epilogue does not match the matrix packing");
-    require(n >= 1 && mtp == (n + 15) / 16 && m.cols % 128 == 0, SP_EINVAL, "gemm shape out of range");
-    const WidePlan p = plan_wide(m, n, part != nullptr && !m.paired);
+    require(n >= 1 && mtp == (n + 15) / 16, SP_EINVAL, "gemm shape out of range");
+    require(order.per >= 1 && order.nw >= 1 && order.slices >= 1 && order.slices <= GEMV_MAX_SLICES &&
+                (long)order.per * order.slices >= m.nkt && (!m.paired || order.slices == 1), SP_EINVAL, "gemm order out of range");
+    const WidePlan p = plan_wide(m, n, order.slices, part ? part_floats : 0);
     wide::GemmArgs a{};
     a.w = m.w; a.sz = m.sz; a.nkt = m.nkt; a.nrg = m.rows_pad / 16;
     a.n_real = m.paired ? m.rows / 2 : m.rows;
     a.x = x; a.xlo = xlo; a.mtp = mtp; a.m = n;
-    a.out_f32 = out_f32; a.out_f16 = out_f16; a.ldo = ldo; a.bias = bias; a.epi = epi; a.pstride = pstride;
-    if (p.slices > 1) { a.epi = EPI_PART; a.out_f32 = part; a.bias = nullptr; }
+    a.out_f32 = out_f32; a.out_f16 = out_f16; a.ldo = ldo; a.bias = bias; a.epi = epi; a.pstride = (size_t)n * ldo;
+    a.per = order.per; a.nw = order.nw;
+    if (p.split) { a.epi = EPI_PART; a.out_f32 = part; a.bias = nullptr; }
+    const bool sum = order.slices > 1 && !p.split;
+    const int grid_slices = p.split ? order.slices : 1;
     switch (m.fmt) {
-        case 1: launch_wide_fmt<1>(p.tile, m.paired, a, p.slices, st); break;
-        case 2: launch_wide_fmt<2>(p.tile, m.paired, a, p.slices, st); break;
-        default: launch_wide_fmt<3>(p.tile, m.paired, a, p.slices, st); break;
+        case 1: launch_wide_fmt<1>(p.tile, m.paired, sum, a, grid_slices, st); break;
+        case 2: launch_wide_fmt<2>(p.tile, m.paired, sum, a, grid_slices, st); break;
+        default: launch_wide_fmt<3>(p.tile, m.paired, sum, a, grid_slices, st); break;
     }
-    return p.slices > 1 ? p.slices : 0;
+    return p.split ? order.slices : 0;
 }
-
-template <int HD>
-void launch_attn_wide(int G, dim3 grid, hipStream_t st, const wide::AttnWideArgs &a) {
-    switch (G) {
-        case 1: hipLaunchKernelGGL((wide::k_attn_wide<HD, 1, 1>), grid, dim3(256), 0, st, a); break;
-        case 2: hipLaunchKernelGGL((wide::k_attn_wide<HD, 2, 1>), grid, dim3(256), 0, st, a); break;
-        case 3: hipLaunchKernelGGL((wide::k_attn_wide<HD, 3, 1>), grid, dim3(256), 0, st, a); break;
-        case 4: hipLaunchKernelGGL((wide::k_attn_wide<HD, 4, 1>), grid, dim3(256), 0, st, a); break;
-        case 5: hipLaunchKernelGGL((wide::k_attn_wide<HD, 5, 1>), grid, dim3(256), 0, st, a); break;
-        case 6: hipLaunchKernelGGL((wide::k_attn_wide<HD, 6, 1>), grid, dim3(256), 0, st, a); break;
-        case 7: hipLaunchKernelGGL((wide::k_attn_wide<HD, 7, 1>), grid, dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL((wide::k_attn_wide<HD, 8, 1>), grid, dim3(256), 0, st, a); break;
-    }
-}
-constexpr int WIDE_ATT_ROWS = 64;       // query rows per attention block
 
 // decode attention split: waves per block x 32-key sub-chunks per wave
 struct DecShape { int nwv, sub; };
@@ -620,10 +629,6 @@ struct sp_engine {
     unsigned long long *am_best = nullptr;      // the argmax's row words and counts (zero between calls)
     unsigned *am_count = nullptr;
     int *am_out = nullptr;
-    void launch_ids(int n) {
-        hipLaunchKernelGGL(k_argmax_row, dim3(argmax_blocks(d.vocab), n), dim3(256), 0, stream, logits, d.vocab, d.vocab, am_best, am_count,
-                           am_out, h_ids);
-    }
     int argmax_cols = 0;         // columns whose argmax ids am_out holds (the last SP_F_ARGMAX call)
     // column descriptors of a call: tokens, attention groups, chunk counts, uploaded together from a pinned staging
     // buffer (one copy per call); `upload_done` marks the copy so the staging buffer is not rewritten before it ran
@@ -677,12 +682,18 @@ struct sp_engine {
         f16 *xn = nullptr, *xn_lo = nullptr, *attn = nullptr, *act = nullptr, *kn = nullptr, *vn = nullptr;
         char *mem = nullptr, *d_up = nullptr, *h_up = nullptr;      // mem: the allocation that holds all of them
         hipEvent_t up_done = nullptr;
-        size_t up_bytes = 0;
+        size_t up_bytes = 0, part_bytes = 0, act_bytes = 0;
     } wd;
-    void alloc_wide();
+    bool alloc_wide();
     void free_wide();
-    void prefill_pass(int n, const sp_token *toks, int n_out, const int *out_cols, float *logits_dev, bool argmax);
-    void head_rows(int n, float *xrows, int pend, float *logits_dev, bool argmax);
+    struct AttnPlan;
+    // one output of sp_engine_prefill: its place among the outputs, and its column in the call
+    struct Out { int i, col; };
+    bool wide_chunk(int n, const AttnPlan &ap) const;
+    void prefill_pass(int n, const sp_token *toks, const std::vector<AttnPlan> &plans, const std::vector<Out> &outs,
+                      float *logits_dev, bool argmax);
+    void forward_columns(int n, const sp_token *toks, int flags);
+    void launch_ids(const float *rows, int n, int first);
 
     // attention plan of one forward call: same-sequence column groups (multi-query kernel) or one block row per column
     struct AttnPlan {
@@ -696,7 +707,7 @@ struct sp_engine {
         std::vector<AttnGroup> groups;
         std::vector<int> colnc;
     };
-    AttnPlan plan_attention(int n, const sp_token *t, bool graph) const;
+    AttnPlan plan_attention(int n, const sp_token *t, bool graph, bool mq = false) const;
 
     void free_all();
     void alloc_activations();
@@ -785,8 +796,10 @@ void sp_engine::alloc_activations() {
     HIPCHK(hipMemset(act, 0, tpad * I * sizeof(f16)));
 }
 
-sp_engine::AttnPlan sp_engine::plan_attention(int n, const sp_token *t, bool graph) const {
+// mq: on the multi-query kernel whatever the columns.
+sp_engine::AttnPlan sp_engine::plan_attention(int n, const sp_token *t, bool graph, bool mq) const {
     AttnPlan p;
+    p.mq = mq;
     auto nlin_of = [](const sp_token &x) { return x.ctx_hi >= x.ctx_lo ? x.ctx_hi - x.ctx_lo + 1 : 0; };
     // maximal runs of columns with the same sequence and tree block whose union ring range fits the slots
     int i = 0;
@@ -926,7 +939,8 @@ void sp_engine::launch_attention(int l, int n, const AttnPlan &ap, int mtp, hipS
     const int NH = d.n_heads, NKV = d.n_kv_heads, HD = d.head_dim, G = NH / NKV, nchunk = ap.nchunk;
     const float scale = 1.0f / std::sqrt((float)HD);
     if (ap.mq) {
-        AttnMqArgs am{q, kc[l], vc[l], dtoks, dgroups, NH, NKV, HD, n_slots, nchunk, scale, attn_part, ap.splits};
+        AttnMqArgs am{q, kc[l], vc[l], dtoks, dgroups, NH, NKV, HD, n_slots, nchunk, scale, attn_part, ap.splits, nullptr,
+                      nullptr, 0, 0};
         dim3 agrid(nchunk, NKV, ap.ngroups * ap.splits);
         if (HD == 64) launch_attn_mq_hd<64>(G, ap.mq_ch, agrid, st, am);
         else launch_attn_mq_hd<128>(G, ap.mq_ch, agrid, st, am);
@@ -971,10 +985,7 @@ void sp_engine::step(int n, int flags, const AttnPlan &ap, int l0, int l1) {
     const bool one = n == 1 && !layers.empty() && gemv_pro_ok(layers[0].qkv, PRO_NORM, H, HD, one_qs, one_qw) &&
                      gemv_pro_ok(layers[0].o, PRO_COMB, H, HD);
     const bool fuse = one && !(flags & SP_F_UNFUSED);
-    // batches of one column tile: qkv and o_proj in 2 k-slices (whole steps, 16 columns: Qwen2-1.5B int8 1.422 ->
-    // 1.404 ms for qkv, then 1.406 -> 1.398 for o_proj, Qwen2-0.5B fp16 -0.8 %; the RoPE kernel and the norm then add
-    // 2 slices instead of 8); int4 o_proj at several column tiles in 4 (Qwen2-7B at 32 columns: -0.3 %)
-    const int qkv_s = one ? one_qs : (n > 1 && n <= 16 ? 2 : 0), qkv_w = one ? one_qw : 0;
+    const int qkv_s = one ? one_qs : qkv_slices(n), qkv_w = one ? one_qw : 0;
     const int down_s = one ? one_ds : 0, down_w = one ? one_dw : 0;
     float *const qpart = fuse ? gpart2 : gpart;
     float *res = x;                             // residual at the start of the layer
@@ -1020,10 +1031,9 @@ void sp_engine::step(int n, int flags, const AttnPlan &ap, int l0, int l1) {
         } else {
             if (!ap.dec_direct)
                 hipLaunchKernelGGL(k_attn_combine, dim3(NH, n), dim3(HD), 0, st, attn_part, dcolnc, NH, HD, nchunk, attn,
-                                   NH * HD, mtp);
-            const int o_s = n > 1 && n <= 16 ? 2 : (n > 16 && ly.o.fmt == 3 ? 4 : 0);
+                                   NH * HD, mtp, 0);
             pend = launch_gemv(ly.o, EPI_RESID, attn, NH * HD, n, rmid, nullptr, H, nullptr, st, gpart, ps, PRO_NONE,
-                               nullptr, o_s, 0, mtp);
+                               nullptr, o_slices(n, ly.o.fmt), 0, mtp);
         }
         // Remainders where they cost nothing (one column: MFMA row 1) or where the logits need them (the qkv input,
         // above: its rounding reaches the attention scores).  Several columns would pay a second MFMA and twice the
@@ -1044,7 +1054,7 @@ void sp_engine::step(int n, int flags, const AttnPlan &ap, int l0, int l1) {
         // activation reads
         launch_rmsnorm(n, res, H, gpart, pend, ps, final_norm, d.rms_eps, xn, nullptr, st, mtp);
         launch_gemv(hm, EPI_STORE, xn, H, n, logits, nullptr, d.vocab, nullptr, st, nullptr, 0, PRO_NONE, nullptr, 0, 0, mtp);
-        if (flags & SP_F_ARGMAX) launch_ids(n);
+        if (flags & SP_F_ARGMAX) launch_ids(logits, n, 0);
     }
     HIPCHK(hipGetLastError());
 }
@@ -1057,72 +1067,109 @@ void sp_engine::free_wide() {
     wd = Wide();
 }
 
-// Buffers of a wide pass, once per engine, in one allocation (Qwen2-1.5B 0.16 GB, Qwen2-7B 0.34 GB).
-void sp_engine::alloc_wide() {
-    if (wd.h_up) return;
+// Buffers of a wide pass, once per engine, in one allocation (Qwen2-1.5B 0.15 GB, Qwen2-7B 0.34 GB).  False when the
+// memory is not there: the columns then run in chunks of max_tokens.
+bool sp_engine::alloc_wide() {
+    if (wd.h_up) return true;
     const size_t P = WIDE_COLS, H = d.hidden, I = d.intermediate, NHD = (size_t)d.n_heads * d.head_dim;
     const size_t KV = P * d.n_kv_heads * d.head_dim;
     auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    // a run of c columns has ceil(c G / rows) attention items: at most one partial item per run (P runs)
-    const size_t max_items = P * (d.n_heads / d.n_kv_heads) / WIDE_ATT_ROWS + P;
-    // column records, runs, attention items, ring flags, output columns
-    wd.up_bytes = up256(P * sizeof(sp_token)) + up256(P * sizeof(wide::Run)) + up256(max_items * sizeof(wide::Item)) +
-                  2 * up256(P * sizeof(int));
-    const size_t sizes[] = {P * H * 4, P * Nqkv * 4, P * NHD * 4, (size_t)WIDE_PART_COLS * std::max<size_t>(H, Nqkv) * 4,
-                            P * (d.head_dim / 2) * sizeof(float2), P * H * 2, P * H * 2, P * NHD * 2, P * I * 2, KV * 2, KV * 2,
-                            wd.up_bytes};
+    // column records, attention groups, chunk counts, ring flags, output columns
+    wd.up_bytes = up256(P * sizeof(sp_token)) + up256(P * sizeof(AttnGroup)) + 3 * up256(P * sizeof(int));
+    wd.part_bytes = up256((size_t)WIDE_PART_COLS * H * 4);
+    wd.act_bytes = up256(P * I * 2);
+    const size_t sizes[] = {P * H * 4, P * std::max<size_t>(H, Nqkv) * 4, P * NHD * 4, P * (d.head_dim / 2) * sizeof(float2),
+                            P * H * 2, P * H * 2, P * NHD * 2, KV * 2, KV * 2, wd.up_bytes, wd.part_bytes, wd.act_bytes};
     size_t total = 0;
     for (size_t b : sizes) total += up256(b);
     try {
         wd.mem = dev_alloc<char>(total);
         HIPCHK(hipEventCreateWithFlags(&wd.up_done, hipEventDisableTiming));
         HIPCHK(hipHostMalloc((void **)&wd.h_up, wd.up_bytes, hipHostMallocDefault));
-    } catch (...) {
+    } catch (const Fail &) {
+        (void)hipGetLastError();
         free_wide();
-        throw;
+        return false;
     }
     char *p = wd.mem;
     int i = 0;
     auto take = [&](auto *&dst) { dst = (std::remove_reference_t<decltype(dst)>)p; p += up256(sizes[i++]); };
-    take(wd.x); take(wd.qkv); take(wd.q); take(wd.part); take(wd.rtab); take(wd.xn); take(wd.xn_lo); take(wd.attn); take(wd.act);
-    take(wd.kn); take(wd.vn); take(wd.d_up);
+    // part and act are neighbours: the attention partials of a layer use both (neither is live during its attention)
+    take(wd.x); take(wd.qkv); take(wd.q); take(wd.rtab); take(wd.xn); take(wd.xn_lo); take(wd.attn);
+    take(wd.kn); take(wd.vn); take(wd.d_up); take(wd.part); take(wd.act);
+    return true;
 }
 
-// Final norm (adding pend pending slices in gpart), LM head and (argmax) the greedy ids of n <= 64 residual rows; logits
-// to the engine's rows and, when given, to logits_dev.
-void sp_engine::head_rows(int n, float *xrows, int pend, float *logits_dev, bool argmax) {
-    const int mtp = n > 1 ? (n + 15) / 16 : 0;
-    const DevMat &hm = d.tied_head ? embed : head;
-    launch_rmsnorm(n, xrows, d.hidden, gpart, pend, gpart_stride, final_norm, d.rms_eps, xn, nullptr, stream, mtp);
-    launch_gemv(hm, EPI_STORE, xn, d.hidden, n, logits, nullptr, d.vocab, nullptr, stream, nullptr, 0, PRO_NONE, nullptr, 0, 0, mtp);
-    if (argmax) launch_ids(n);
-    if (logits_dev)
-        HIPCHK(hipMemcpyAsync(logits_dev, logits, (size_t)n * d.vocab * sizeof(float), hipMemcpyDeviceToDevice, stream));
+// Greedy ids of n rows of logits (vocab apart) into am_out[first ..) and the pinned copy.
+void sp_engine::launch_ids(const float *rows, int n, int first) {
+    hipLaunchKernelGGL(k_argmax_row, dim3(argmax_blocks(d.vocab), n), dim3(256), 0, stream, rows, d.vocab, d.vocab, am_best,
+                       am_count, am_out + first, h_ids + first);
 }
 
-// One wide pass: n <= WIDE_COLS plain columns (runs of consecutive positions, each sequence once) through every layer.
-// The logits of columns out_cols go to logits_dev [n_out][vocab] (and, for n_out <= maxT, the engine's rows and ids).
-void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *out_cols, float *logits_dev, bool argmax) {
+// Whether a chunk of n columns can be part of a wide pass: its step sums every product in the order of several column tiles
+// (a step of up to 16 columns uses other kernels), the same for all of them, and its attention runs on the multi-query kernel.
+bool sp_engine::wide_chunk(int n, const AttnPlan &ap) const {
+    if (n <= 16 || !ap.mq || ap.mq_ch != ATT_CH) return false;
+    const int mt = (n + 15) / 16;
+    const Layer &ly = layers[0];
+    return wide_order(ly.qkv, mt, true) == wide_order(ly.qkv, GEMV_MAX_MT, true) &&
+           wide_order(ly.o, mt, true, o_slices(n, ly.o.fmt)) == wide_order(ly.o, GEMV_MAX_MT, true, o_slices(n, ly.o.fmt)) &&
+           wide_order(ly.gate_up, mt, false) == wide_order(ly.gate_up, GEMV_MAX_MT, false) &&
+           wide_order(ly.down, mt, true) == wide_order(ly.down, GEMV_MAX_MT, true);
+}
+
+// One wide pass: n <= WIDE_COLS plain columns (runs of consecutive positions, each sequence once), the chunks of max_tokens
+// columns whose attention plans are given (wide_chunk holds for each), through every layer.  Every value is the one that
+// steps over these chunks, one after the other, give (sp_wide.h).  The logits of outs[j].col go to logits_dev's row
+// outs[j].i (when given), its greedy id to am_out[outs[j].i] (argmax).
+void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<AttnPlan> &plans, const std::vector<Out> &outs,
+                             float *logits_dev, bool argmax) {
     const int H = d.hidden, I = d.intermediate, NH = d.n_heads, NKV = d.n_kv_heads, HD = d.head_dim, G = NH / NKV;
-    const int mtp = (n + 15) / 16;
-    // ---- runs, attention items, which columns the ring keeps, and whether a new key may be stored before the attention
-    std::vector<wide::Run> runs;
-    std::vector<wide::Item> items;
-    std::vector<int> keep(n, 0);
-    bool to_ring = true, last_only = n_out <= std::min(maxT, 64);
-    std::vector<char> is_last(n, 0);
+    const int mtp = (n + 15) / 16, n_out = (int)outs.size();
+    // ---- attention groups of all chunks, which columns the ring keeps, and whether a new key may be stored before the
+    // attention (no slot still visible to a column of the call is overwritten)
+    std::vector<AttnGroup> groups;
+    std::vector<int> keep(n, 0), colnc, out_cols;
+    std::vector<int> run_of(n), mt_of(n);    // the first column of a column's run; the column tiles of its chunk
+    bool to_ring = true;
     for (int c = 0; c < n;) {
         int e = c + 1;
         while (e < n && toks[e].seq == toks[c].seq) ++e;
-        const int p0 = toks[c].ctx_hi, p1 = toks[e - 1].ctx_hi;
-        runs.push_back({c, e - c, toks[c].seq, p0});
+        const int p1 = toks[e - 1].ctx_hi;
         to_ring = to_ring && p1 - toks[c].ctx_lo + 1 <= n_slots;
-        for (int i = c; i < e; ++i) keep[i] = toks[i].ctx_hi > p1 - n_slots;
-        for (int r0 = 0; r0 < (e - c) * G; r0 += WIDE_ATT_ROWS) items.push_back({(int)runs.size() - 1, r0});
-        is_last[e - 1] = 1;
+        for (int i = c; i < e; ++i) { keep[i] = toks[i].ctx_hi > p1 - n_slots; run_of[i] = c; }
         c = e;
     }
-    for (int i = 0; i < n_out; ++i) last_only = last_only && is_last[out_cols[i]];
+    // attention launches: consecutive chunks whose partial records fit the buffer (one chunk alone always fits the
+    // step's own)
+    struct Launch { int col0, cols, g0, groups, nchunk, splits; float *part; };
+    std::vector<Launch> launches;
+    const size_t rec = part_floats(HD), room = (wd.part_bytes + wd.act_bytes) / 4;
+    {
+        int col = 0;
+        for (const AttnPlan &ap : plans) {
+            const int g0 = (int)groups.size(), cols = (int)ap.colnc.size();
+            for (AttnGroup g : ap.groups) {
+                g.first_col += col;
+                g.run_col = run_of[g.first_col];
+                g.run_pos = toks[g.run_col].ctx_hi;
+                groups.push_back(g);
+            }
+            colnc.insert(colnc.end(), ap.colnc.begin(), ap.colnc.end());
+            std::fill(mt_of.begin() + col, mt_of.begin() + col + cols, (cols + 15) / 16);
+            const bool small = (size_t)cols * NH * ap.nchunk * rec <= room;
+            Launch *w = launches.empty() ? nullptr : &launches.back();
+            if (w && small && w->part == wd.part && (size_t)(w->cols + cols) * NH * std::max(w->nchunk, ap.nchunk) * rec <= room) {
+                w->cols += cols; w->groups += ap.ngroups;
+                w->nchunk = std::max(w->nchunk, ap.nchunk); w->splits = std::max(w->splits, ap.splits);
+            } else {
+                launches.push_back({col, cols, g0, ap.ngroups, ap.nchunk, ap.splits, small ? wd.part : attn_part});
+            }
+            col += cols;
+        }
+        require(col == n, SP_EINVAL, "prefill plan does not cover the columns");
+    }
+    for (const Out &o : outs) out_cols.push_back(o.col);
     // ---- one upload from pinned memory
     HIPCHK(hipEventSynchronize(wd.up_done));
     size_t off = 0;
@@ -1134,10 +1181,10 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
         return (const void *)(wd.d_up + at);
     };
     const sp_token *dt = (const sp_token *)put(toks, n * sizeof(sp_token));
-    const wide::Run *druns = (const wide::Run *)put(runs.data(), runs.size() * sizeof(wide::Run));
-    const wide::Item *ditems = (const wide::Item *)put(items.data(), items.size() * sizeof(wide::Item));
+    const AttnGroup *dgr = (const AttnGroup *)put(groups.data(), groups.size() * sizeof(AttnGroup));
+    const int *dnc = (const int *)put(colnc.data(), n * sizeof(int));
     const int *dkeep = (const int *)put(keep.data(), n * sizeof(int));
-    const int *dout = (const int *)put(out_cols, n_out * sizeof(int));
+    const int *dout = (const int *)put(out_cols.data(), n_out * sizeof(int));
     HIPCHK(hipMemcpyAsync(wd.d_up, wd.h_up, off, hipMemcpyHostToDevice, stream));
     HIPCHK(hipEventRecord(wd.up_done, stream));
     switch (embed.fmt) {
@@ -1145,80 +1192,66 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, int n_out, const int *
         case 2: launch_embed<2>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
         default: launch_embed<3>(embed, dt, n, H, wd.x, stream, nullptr, d.vocab, inv_freq, HD / 2, wd.rtab); break;
     }
-    const size_t ps = (size_t)n * std::max(H, Nqkv);       // slices lie n columns apart
     const float scale = 1.0f / std::sqrt((float)HD);
-    int pend = 0;
+    int nc = n, mtc = mtp, pend = 0;                   // columns that go on (the output columns after the last attention)
+    float *x = wd.x;
+    f16 *at = wd.attn;
     for (int l = 0; l < d.n_layers; ++l) {
         Layer &ly = layers[l];
         const bool last = l + 1 == d.n_layers;
-        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
-        const int sq = launch_gemm_wide(ly.qkv, EPI_STORE, wd.xn, wd.xn_lo, n, mtp, wd.qkv, nullptr, Nqkv, ly.qkv_b, wd.part, ps,
-                                        stream);
-        wide::RopeWideArgs ra{RopeArgs{wd.qkv, Nqkv, NH, NKV, HD, wd.rtab, dt, wd.q, kc[l], vc[l], n_slots, wd.part, ps, ly.qkv_b},
-                              wd.kn, wd.vn, WIDE_COLS, to_ring ? 1 : 0};
-        by_slices(sq, [&](auto c) {
-            hipLaunchKernelGGL((wide::k_rope_wide<decltype(c)::value>), dim3(n), dim3(256), 0, stream, ra);
-        });
-        auto commit = [&] {
-            if (!to_ring)
-                hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt,
-                                   dkeep, NKV, HD, n_slots, WIDE_COLS);
-        };
-        if (last && n_out == 0) { commit(); break; }
-        if (last && last_only) {
-            // only the output columns go on: the rest of the last layer and the head run as a batch of n_out decode
-            // columns over the ring, which now holds every key they see
-            commit();
-            std::vector<sp_token> ot(n_out);
-            for (int i = 0; i < n_out; ++i) ot[i] = toks[out_cols[i]];
-            AttnPlan ap = plan_attention(n_out, ot.data(), false);
-            upload(n_out, ot.data(), ap);
-            const int m1 = n_out > 1 ? (n_out + 15) / 16 : 0;
-            hipLaunchKernelGGL(wide::k_gather_rows, dim3(n_out), dim3(256), 0, stream, wd.x, dout, H, x);
-            hipLaunchKernelGGL(wide::k_gather_rows, dim3(n_out), dim3(256), 0, stream, wd.q, dout, NH * HD, q);
-            launch_attention(l, n_out, ap, m1, stream);
-            if (!ap.dec_direct)
-                hipLaunchKernelGGL(k_attn_combine, dim3(NH, n_out), dim3(HD), 0, stream, attn_part, dcolnc, NH, HD, ap.nchunk,
-                                   attn, NH * HD, m1);
-            pend = launch_gemv(ly.o, EPI_RESID, attn, NH * HD, n_out, x, nullptr, H, nullptr, stream, gpart, gpart_stride,
-                               PRO_NONE, nullptr, 0, 0, m1);
-            f16 *xlo = n_out == 1 ? xn_lo : nullptr, *alo = n_out == 1 ? act_lo : nullptr;
-            launch_rmsnorm(n_out, x, H, gpart, pend, gpart_stride, ly.post_norm, d.rms_eps, xn, xlo, stream, m1);
-            launch_gemv(ly.gate_up, EPI_SILU, xn, H, n_out, nullptr, act, I, nullptr, stream, nullptr, 0, PRO_NONE, nullptr, 0, 0,
-                        m1, m1, xlo, alo);
-            pend = launch_gemv(ly.down, EPI_RESID, act, I, n_out, x, nullptr, H, nullptr, stream, gpart, gpart_stride, PRO_NONE,
-                               nullptr, n_out == 1 ? 8 : 0, n_out == 1 ? 8 : 0, m1, 0, alo);
-            head_rows(n_out, x, pend, logits_dev, argmax);
-            HIPCHK(hipGetLastError());
-            return;
-        }
-        wide::AttnWideArgs aa{wd.q, kc[l], vc[l], wd.kn, wd.vn, dt, druns, ditems, NH, NKV, n_slots, WIDE_COLS, mtp, scale, wd.attn};
-        const dim3 agrid((unsigned)items.size(), NKV);
-        if (HD == 64) launch_attn_wide<64>(G, agrid, stream, aa);
-        else launch_attn_wide<128>(G, agrid, stream, aa);
-        commit();
-        pend = launch_gemm_wide(ly.o, EPI_RESID, wd.attn, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
-        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
-        launch_gemm_wide(ly.gate_up, EPI_SILU, wd.xn, nullptr, n, mtp, nullptr, wd.act, I, nullptr, nullptr, 0, stream);
-        pend = launch_gemm_wide(ly.down, EPI_RESID, wd.act, nullptr, n, mtp, wd.x, nullptr, H, nullptr, wd.part, ps, stream);
-    }
-    if (n_out > 0) {
-        // every column's final residual is needed: the pending slices go in with the norm (whose output is used when
-        // all columns have logits)
-        launch_norm_wide(n, wd.x, H, wd.part, pend, ps, final_norm, d.rms_eps, wd.xn, nullptr, stream, mtp);
-        bool all = n_out == n && logits_dev && !argmax;
-        for (int i = 0; i < n_out; ++i) all = all && out_cols[i] == i;
-        if (all) {
-            launch_gemm_wide(d.tied_head ? embed : head, EPI_STORE, wd.xn, nullptr, n, mtp, logits_dev, nullptr, d.vocab, nullptr,
-                             nullptr, 0, stream);
-        } else {
-            const int step = std::min(maxT, 64);
-            for (int i = 0; i < n_out; i += step) {
-                const int c = std::min(step, n_out - i);
-                hipLaunchKernelGGL(wide::k_gather_rows, dim3(c), dim3(256), 0, stream, wd.x, dout + i, H, x);
-                head_rows(c, x, 0, logits_dev ? logits_dev + (size_t)i * d.vocab : nullptr, argmax);
+        const WideOrder oq = wide_order(ly.qkv, GEMV_MAX_MT, true), oo = wide_order(ly.o, GEMV_MAX_MT, true, o_slices(64, ly.o.fmt)),
+                        og = wide_order(ly.gate_up, GEMV_MAX_MT, false), od = wide_order(ly.down, GEMV_MAX_MT, true);
+        launch_norm_wide(n, x, H, wd.part, pend, (size_t)n * H, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
+        launch_gemm_wide(ly.qkv, oq, EPI_STORE, wd.xn, wd.xn_lo, n, mtp, wd.qkv, nullptr, Nqkv, ly.qkv_b, nullptr, 0, stream);
+        const wide::RopeWideArgs ra{RopeArgs{wd.qkv, Nqkv, NH, NKV, HD, wd.rtab, dt, wd.q, kc[l], vc[l], n_slots, nullptr, 0,
+                                             ly.qkv_b}, wd.kn, wd.vn, WIDE_COLS, to_ring ? 1 : 0};
+        hipLaunchKernelGGL(wide::k_rope_wide, dim3(n), dim3(256), 0, stream, ra);
+        if (!last || n_out > 0) {
+            size_t oi = 0;                             // outs are in column order
+            for (const Launch &w : launches) {
+                if (last) {                            // of the last layer, only the chunks that hold an output column
+                    while (oi < outs.size() && outs[oi].col < w.col0) ++oi;
+                    if (oi == outs.size() || outs[oi].col >= w.col0 + w.cols) continue;
+                }
+                AttnMqArgs am{wd.q, kc[l], vc[l], dt, dgr + w.g0, NH, NKV, HD, n_slots, w.nchunk, scale, w.part, w.splits, wd.kn,
+                              wd.vn, WIDE_COLS, w.col0};
+                const dim3 grid(w.nchunk, NKV, w.groups * w.splits);
+                if (HD == 64) launch_attn_mq_ch<64, ATT_CH, true>(G, grid, stream, am);
+                else launch_attn_mq_ch<128, ATT_CH, true>(G, grid, stream, am);
+                hipLaunchKernelGGL(k_attn_combine, dim3(NH, w.cols), dim3(HD), 0, stream, w.part, dnc, NH, HD, w.nchunk, wd.attn,
+                                   NH * HD, mtp, w.col0);
             }
         }
+        if (!to_ring)
+            hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt, dkeep, NKV, HD,
+                               n_slots, WIDE_COLS);
+        if (last) {
+            if (n_out == 0) break;
+            // only the output columns go on, as compact rows (in the buffers of qkv and q, which are free)
+            nc = n_out; mtc = (nc + 15) / 16;
+            x = wd.qkv;
+            at = (f16 *)wd.q;
+            hipLaunchKernelGGL(wide::k_gather_cols, dim3(nc), dim3(256), 0, stream, wd.x, wd.attn, dout, H, NH * HD, mtp, x, at, mtc);
+        }
+        pend = launch_gemm_wide(ly.o, oo, EPI_RESID, at, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part, wd.part_bytes / 4, stream);
+        launch_norm_wide(nc, x, H, wd.part, pend, (size_t)nc * H, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtc);
+        launch_gemm_wide(ly.gate_up, og, EPI_SILU, wd.xn, nullptr, nc, mtc, nullptr, wd.act, I, nullptr, nullptr, 0, stream);
+        pend = launch_gemm_wide(ly.down, od, EPI_RESID, wd.act, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part, wd.part_bytes / 4, stream);
+    }
+    // ---- head: runs of outputs with neighbouring places whose chunks have as many column tiles (the head's order
+    // depends on them)
+    const DevMat &hm = d.tied_head ? embed : head;
+    for (int j0 = 0; j0 < n_out;) {
+        int j1 = j0 + 1;
+        while (j1 < n_out && outs[j1].i == outs[j1 - 1].i + 1 && mt_of[outs[j1].col] == mt_of[outs[j0].col] && (logits_dev || j1 - j0 < maxT)) ++j1;
+        const int c = j1 - j0, m1 = (c + 15) / 16;
+        float *rows = logits_dev ? logits_dev + (size_t)outs[j0].i * d.vocab : logits;
+        launch_norm_wide(c, x + (size_t)j0 * H, H, wd.part + (size_t)j0 * H, pend, (size_t)nc * H, final_norm, d.rms_eps, wd.xn,
+                         nullptr, stream, m1);
+        launch_gemm_wide(hm, wide_order(hm, mt_of[outs[j0].col], false), EPI_STORE, wd.xn, nullptr, c, m1, rows, nullptr, d.vocab, nullptr,
+                         nullptr, 0, stream);
+        if (argmax) launch_ids(rows, c, outs[j0].i);
+        j0 = j1;
     }
     HIPCHK(hipGetLastError());
 }
@@ -1329,7 +1362,7 @@ bool sp_engine::run_d1(const sp_token &t, int flags) {
     if (!launch_d1(t, flags)) return false;
     const DevMat &hm = d.tied_head ? embed : head;
     launch_gemv(hm, EPI_STORE, xn, d.hidden, 1, logits, nullptr, d.vocab, nullptr, stream);
-    if (flags & SP_F_ARGMAX) launch_ids(1);
+    if (flags & SP_F_ARGMAX) launch_ids(logits, 1, 0);
     HIPCHK(hipGetLastError());
     return true;
 }
@@ -1342,6 +1375,98 @@ void sp_engine::check_d1_error() {
 }
 
 // ============================================================================================== C ABI
+// The launches of one checked call over n <= max_tokens columns: the persistent step for one plain decode column where the
+// shape and the pool allow it, else the kernel chain.  Logits are left in the engine's rows, ids in am_out and the pinned
+// copy.
+void sp_engine::forward_columns(int n, const sp_token *toks, int flags) {
+    const bool devcols = flags & SP_F_DEVCOLS;
+    const bool use_graph = flags & SP_F_GRAPH;
+    const int sflags = flags & (SP_F_LOGITS | SP_F_ARGMAX | SP_F_UNFUSED | SP_F_FEED);
+    // one plain decode column: the persistent step, where the shape and the pool allow it
+    const sp_token &t0 = toks[0];
+    if (n == 1 && (flags & SP_F_LOGITS) && !(flags & (SP_F_UNFUSED | SP_F_CHAIN | SP_F_DEVCOLS)) && t0.tree_count == 0 &&
+        t0.ctx_hi >= t0.ctx_lo && t0.slot == t0.ctx_hi % n_slots && prepare_d1() && run_d1(t0, sflags)) {
+        last_path = 1;
+        last_dispatches = (sflags & SP_F_ARGMAX) ? 3 : 2;
+        return;
+    }
+    last_path = 0;
+    const AttnPlan ap = plan_attention(n, toks, use_graph);
+    upload(n, toks, ap);
+    if (devcols) {
+        hipLaunchKernelGGL(k_patch_columns, dim3((n + 63) / 64), dim3(64), 0, stream, dtoks, n, dev_tokens,
+                           dev_masks, d.vocab);
+        HIPCHK(hipGetLastError());
+    }
+    if (use_graph) {
+        // The step's three parts (the embedding and layer 0, layers 1-4, the rest) are recorded as graphs once per
+        // (columns, flags, attention plan); their kernel nodes are the reported dispatch count.  The first part
+        // always runs as plain launches (the GPU starts after the first of them, not after a graph launch's
+        // set-up).  The others run as plain launches too when the host runs ahead of the GPU -- a fed greedy loop,
+        // or several columns, whose kernels each take longer than their launch -- because a replayed graph costs
+        // the GPU more per kernel than in-order launches (A/B of whole steps: fed bs1 0.974 -> 0.968 ms/token, tree
+        // pass 1.499 -> 1.490 ms, 16-request 0.5B burst 18.0k -> 18.2k tok/s, bs16 1.442 -> 1.430 ms); a single
+        // column whose caller waits for every token replays them (plain launches there leave the GPU waiting for
+        // the host: 0.995 -> 1.02-1.05 ms per token).
+        const bool plain = (sflags & SP_F_FEED) || n > 1;
+        const int L = d.n_layers;
+        const int cuts[4] = {0, std::min(1, L), std::min(5, L), L};
+        const int plan_code = ap.mq ? (ap.mq_ch == 128 ? 1 << 20 : 0) + ap.ngroups * 1024 + ap.splits
+                                    : (ap.dec ? (ap.dec_direct ? -3 : -2) - 8 * ap.dec_kpb : (ap.rope_fused ? -4 : -1));
+        int total = 0;
+        for (int part = 0; part < 3; ++part) {
+            if (cuts[part] >= cuts[part + 1]) continue;      // empty (short models); the head ran in its part
+            auto key = std::make_tuple(n, sflags | (part << 8), plan_code);
+            const bool replay = part > 0 && !plain;
+            if (!graph_kernels.count(key) || (replay && !graphs.count(key))) {
+                // record on the private stream (the caller's may be the null stream, which cannot capture)
+                hipGraph_t g;
+                hipStream_t run_stream = stream;
+                stream = capture_stream;
+                HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+                try {
+                    step(n, sflags, ap, cuts[part], cuts[part + 1]);
+                } catch (...) {
+                    hipGraph_t dummy;
+                    (void)hipStreamEndCapture(stream, &dummy);
+                    stream = run_stream;
+                    throw;
+                }
+                hipError_t ce = hipStreamEndCapture(stream, &g);
+                stream = run_stream;
+                HIPCHK(ce);
+                size_t nn = 0;
+                HIPCHK(hipGraphGetNodes(g, nullptr, &nn));
+                std::vector<hipGraphNode_t> nodes(nn);
+                if (nn) HIPCHK(hipGraphGetNodes(g, nodes.data(), &nn));
+                int kernels = 0;
+                for (auto nd : nodes) {
+                    hipGraphNodeType ty;
+                    HIPCHK(hipGraphNodeGetType(nd, &ty));
+                    kernels += ty == hipGraphNodeTypeKernel;
+                }
+                if (replay) {               // instantiated only for the parts that are replayed
+                    hipGraphExec_t ge;
+                    hipError_t ie = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+                    (void)hipGraphDestroy(g);
+                    HIPCHK(ie);
+                    graphs[key] = ge;
+                } else {
+                    (void)hipGraphDestroy(g);
+                }
+                graph_kernels[key] = kernels;
+            }
+            if (replay) HIPCHK(hipGraphLaunch(graphs[key], stream));
+            else step(n, sflags, ap, cuts[part], cuts[part + 1]);
+            total += graph_kernels[key];
+        }
+        last_dispatches = total;
+    } else {
+        step(n, sflags, ap, 0, d.n_layers);
+        last_dispatches = -1;
+    }
+}
+
 namespace {
 int fail_engine(sp_engine *e, const Fail &f) {
     if (e) e->err = f.msg;
@@ -1609,104 +1734,13 @@ int sp_engine_forward(sp_engine *e, int32_t n, const sp_token *toks, int32_t fla
                 "SP_F_FEED needs a previous SP_F_ARGMAX call over at least as many columns");
         e->check_columns(n, toks, feed || devcols);
         e->check_d1_error();
-        const bool use_graph = flags & SP_F_GRAPH;
-        const int sflags = flags & (SP_F_LOGITS | SP_F_ARGMAX | SP_F_UNFUSED | SP_F_FEED);
-        // one plain decode column: the persistent step, where the shape and the pool allow it
-        const sp_token &t0 = toks[0];
-        if (n == 1 && (flags & SP_F_LOGITS) && !(flags & (SP_F_UNFUSED | SP_F_CHAIN | SP_F_DEVCOLS)) && t0.tree_count == 0 &&
-            t0.ctx_hi >= t0.ctx_lo && t0.slot == t0.ctx_hi % e->n_slots && e->prepare_d1() && e->run_d1(t0, sflags)) {
-            e->last_path = 1;
-            e->last_dispatches = (sflags & SP_F_ARGMAX) ? 3 : 2;
-            if (sflags & SP_F_ARGMAX) e->argmax_cols = 1;
-            if (logits_dev)
-                HIPCHK(hipMemcpyAsync(logits_dev, e->logits, (size_t)d.vocab * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
-            if (argmax_host) {
-                HIPCHK(hipStreamSynchronize(e->stream));
-                e->check_d1_error();
-                std::memcpy(argmax_host, e->h_ids, sizeof(int32_t));
-            }
-            return;
-        }
-        e->last_path = 0;
-        const sp_engine::AttnPlan ap = e->plan_attention(n, toks, use_graph);
-        e->upload(n, toks, ap);
-        if (devcols) {
-            hipLaunchKernelGGL(k_patch_columns, dim3((n + 63) / 64), dim3(64), 0, e->stream, e->dtoks, n, e->dev_tokens,
-                               e->dev_masks, d.vocab);
-            HIPCHK(hipGetLastError());
-        }
-        if (use_graph) {
-            // The step's three parts (the embedding and layer 0, layers 1-4, the rest) are recorded as graphs once per
-            // (columns, flags, attention plan); their kernel nodes are the reported dispatch count.  The first part
-            // always runs as plain launches (the GPU starts after the first of them, not after a graph launch's
-            // set-up).  The others run as plain launches too when the host runs ahead of the GPU -- a fed greedy loop,
-            // or several columns, whose kernels each take longer than their launch -- because a replayed graph costs
-            // the GPU more per kernel than in-order launches (A/B of whole steps: fed bs1 0.974 -> 0.968 ms/token, tree
-            // pass 1.499 -> 1.490 ms, 16-request 0.5B burst 18.0k -> 18.2k tok/s, bs16 1.442 -> 1.430 ms); a single
-            // column whose caller waits for every token replays them (plain launches there leave the GPU waiting for
-            // the host: 0.995 -> 1.02-1.05 ms per token).
-            const bool plain = (sflags & SP_F_FEED) || n > 1;
-            const int L = d.n_layers;
-            const int cuts[4] = {0, std::min(1, L), std::min(5, L), L};
-            const int plan_code = ap.mq ? (ap.mq_ch == 128 ? 1 << 20 : 0) + ap.ngroups * 1024 + ap.splits
-                                        : (ap.dec ? (ap.dec_direct ? -3 : -2) - 8 * ap.dec_kpb : (ap.rope_fused ? -4 : -1));
-            int total = 0;
-            for (int part = 0; part < 3; ++part) {
-                if (cuts[part] >= cuts[part + 1]) continue;      // empty (short models); the head ran in its part
-                auto key = std::make_tuple(n, sflags | (part << 8), plan_code);
-                const bool replay = part > 0 && !plain;
-                if (!e->graph_kernels.count(key) || (replay && !e->graphs.count(key))) {
-                    // record on the private stream (the caller's may be the null stream, which cannot capture)
-                    hipGraph_t g;
-                    hipStream_t run_stream = e->stream;
-                    e->stream = e->capture_stream;
-                    HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-                    try {
-                        e->step(n, sflags, ap, cuts[part], cuts[part + 1]);
-                    } catch (...) {
-                        hipGraph_t dummy;
-                        (void)hipStreamEndCapture(e->stream, &dummy);
-                        e->stream = run_stream;
-                        throw;
-                    }
-                    hipError_t ce = hipStreamEndCapture(e->stream, &g);
-                    e->stream = run_stream;
-                    HIPCHK(ce);
-                    size_t nn = 0;
-                    HIPCHK(hipGraphGetNodes(g, nullptr, &nn));
-                    std::vector<hipGraphNode_t> nodes(nn);
-                    if (nn) HIPCHK(hipGraphGetNodes(g, nodes.data(), &nn));
-                    int kernels = 0;
-                    for (auto nd : nodes) {
-                        hipGraphNodeType ty;
-                        HIPCHK(hipGraphNodeGetType(nd, &ty));
-                        kernels += ty == hipGraphNodeTypeKernel;
-                    }
-                    if (replay) {               // instantiated only for the parts that are replayed
-                        hipGraphExec_t ge;
-                        hipError_t ie = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-                        (void)hipGraphDestroy(g);
-                        HIPCHK(ie);
-                        e->graphs[key] = ge;
-                    } else {
-                        (void)hipGraphDestroy(g);
-                    }
-                    e->graph_kernels[key] = kernels;
-                }
-                if (replay) HIPCHK(hipGraphLaunch(e->graphs[key], e->stream));
-                else e->step(n, sflags, ap, cuts[part], cuts[part + 1]);
-                total += e->graph_kernels[key];
-            }
-            e->last_dispatches = total;
-        } else {
-            e->step(n, sflags, ap, 0, d.n_layers);
-            e->last_dispatches = -1;
-        }
-        if (sflags & SP_F_ARGMAX) e->argmax_cols = n;
+        e->forward_columns(n, toks, flags);
+        if (flags & SP_F_ARGMAX) e->argmax_cols = n;
         if (logits_dev && (flags & SP_F_LOGITS))
             HIPCHK(hipMemcpyAsync(logits_dev, e->logits, (size_t)n * d.vocab * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
         if (argmax_host) {
             HIPCHK(hipStreamSynchronize(e->stream));
+            if (e->last_path == 1) e->check_d1_error();
             std::memcpy(argmax_host, e->h_ids, n * sizeof(int32_t));
         }
     });
@@ -1743,13 +1777,67 @@ int sp_engine_prefill(sp_engine *e, int32_t n, const sp_token *toks, int32_t n_o
         }
         for (int i = 0; i < n_out; ++i) require(out_cols[i] >= 0 && out_cols[i] < n, SP_EINVAL, "output column out of range");
         e->check_d1_error();
-        e->alloc_wide();
-        e->prefill_pass(n, toks, n_out, out_cols, logits_dev, argmax_host != nullptr);
-        e->last_path = 0;
-        e->last_dispatches = -1;
-        if (argmax_host) {
+        // Chunks of max_tokens columns, as a caller of sp_engine_forward would cut them.  Neighbouring chunks that a wide
+        // pass can take go through it together; the others run one by one.
+        std::vector<sp_engine::Out> outs;
+        for (int i = 0; i < n_out; ++i) outs.push_back({i, out_cols[i]});
+        std::stable_sort(outs.begin(), outs.end(), [](const auto &a, const auto &b) { return a.col < b.col; });
+        const bool argmax = argmax_host != nullptr;
+        auto outs_of = [&](int c0, int c1) {           // the outputs of columns [c0, c1), columns counted from c0
+            std::vector<sp_engine::Out> v;
+            for (const auto &o : outs)
+                if (o.col >= c0 && o.col < c1) v.push_back({o.i, o.col - c0});
+            return v;
+        };
+        // the first column past c0 (at most c1) whose K/V would take a slot that a column from c0 on still sees: a step may
+        // not hold both (in a wide pass the ring is written after the attention)
+        auto fits_ring = [&](int c0, int c1) {
+            for (int c = c0, r = c0; c < c1; ++c) {
+                if (toks[c].seq != toks[r].seq) r = c;
+                if (toks[c].ctx_hi - toks[r].ctx_lo + 1 > e->n_slots) return c;
+            }
+            return c1;
+        };
+        const int T = e->maxT;
+        for (int c0 = 0; c0 < n;) {
+            std::vector<sp_engine::AttnPlan> plans;
+            int c1 = c0;
+            bool tight = false;
+            while (c1 < n) {
+                const int c = std::min(n, c1 / T * T + T) - c1;
+                const bool over = fits_ring(c1, c1 + c) < c1 + c;
+                sp_engine::AttnPlan ap = e->plan_attention(c, toks + c1, false, over);
+                if (!over && !e->wide_chunk(c, ap)) break;
+                tight = tight || over;
+                plans.push_back(std::move(ap));
+                c1 += c;
+            }
+            if ((plans.size() > 1 || tight) && e->alloc_wide()) {
+                e->prefill_pass(c1 - c0, toks + c0, plans, outs_of(c0, c1), logits_dev, argmax);
+                e->last_path = 0;
+                e->last_dispatches = -1;
+            } else {
+                c1 = fits_ring(c0, std::min(n, c0 / T * T + T));
+                const std::vector<sp_engine::Out> v = outs_of(c0, c1);
+                e->forward_columns(c1 - c0, toks + c0, v.empty() ? 0 : SP_F_LOGITS);
+                for (size_t j0 = 0; j0 < v.size();) {  // runs of neighbouring columns with neighbouring places
+                    size_t j1 = j0 + 1;
+                    while (j1 < v.size() && v[j1].col == v[j1 - 1].col + 1 && v[j1].i == v[j1 - 1].i + 1) ++j1;
+                    const float *rows = e->logits + (size_t)v[j0].col * d.vocab;
+                    if (logits_dev)
+                        HIPCHK(hipMemcpyAsync(logits_dev + (size_t)v[j0].i * d.vocab, rows, (j1 - j0) * d.vocab * sizeof(float),
+                                              hipMemcpyDeviceToDevice, e->stream));
+                    if (argmax) e->launch_ids(rows, (int)(j1 - j0), v[j0].i);
+                    j0 = j1;
+                }
+                HIPCHK(hipGetLastError());
+            }
+            c0 = c1;
+        }
+        if (argmax) {
             e->argmax_cols = n_out;
             HIPCHK(hipStreamSynchronize(e->stream));
+            e->check_d1_error();
             std::memcpy(argmax_host, e->h_ids, n_out * sizeof(int32_t));
         }
     });

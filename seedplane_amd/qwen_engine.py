@@ -29,7 +29,7 @@ from . import _lib
 from . import native_bundle
 
 GROUP = 32
-WIDE_COLS = 2048          # most columns of one wide prefill pass (sp_engine_prefill)
+WIDE_COLS = 2048          # most columns of one sp_engine_prefill call
 
 
 class _KVLayers:
@@ -427,9 +427,14 @@ class Qwen2Engine:
             a['ctx_lo'] = np.maximum(0, p - cache.window + 1)
         return a
 
+    @property
+    def _pass_cols(self):
+        """Columns of one prefill call: whole chunks of max_tokens, so that calls cut a prompt where chunks end."""
+        return WIDE_COLS // self.max_tokens * self.max_tokens
+
     def _wide(self, cols, out, logits_out=None, want_ids=False):
-        """One wide pass (sp_engine_prefill) over a TOKEN_DTYPE array of at most WIDE_COLS columns; logits (and greedy
-        ids) of the columns `out`."""
+        """One prefill call (sp_engine_prefill) over a TOKEN_DTYPE array of at most _pass_cols columns; logits (and
+        greedy ids) of the columns `out`.  The same bits as calls of run() over max_tokens columns each."""
         out = np.ascontiguousarray(out, dtype=np.int32)
         ids = np.zeros(len(out), dtype=np.int32) if want_ids else None
         dst = ctypes.c_void_p(logits_out.data_ptr()) if logits_out is not None else None
@@ -466,8 +471,9 @@ class Qwen2Engine:
         T = self.max_tokens
         if qlen > T:
             cols = self._prompt_columns(ids, cache, start, positions)
-            for c0 in range(0, qlen, WIDE_COLS):
-                part = cols[c0:c0 + WIDE_COLS]
+            step = self._pass_cols
+            for c0 in range(0, qlen, step):
+                part = cols[c0:c0 + step]
                 if all_logits:
                     self._wide(part, np.arange(len(part)), logits_out=logits[c0:c0 + len(part)])
                 elif c0 + len(part) == qlen:
@@ -676,8 +682,9 @@ class Qwen2Engine:
         out = None
         if len(ids) > T:
             cols = self._prompt_columns(ids, cache, start)
-            for c0 in range(0, len(ids), WIDE_COLS):
-                part = cols[c0:c0 + WIDE_COLS]
+            step = self._pass_cols
+            for c0 in range(0, len(ids), step):
+                part = cols[c0:c0 + step]
                 if c0 + len(part) == len(ids):
                     out = int(self._wide(part, [len(part) - 1], want_ids=True)[0])
                 else:
@@ -718,8 +725,8 @@ class Qwen2Engine:
         return nxt
 
     def _prefill_wide(self, prompts, caches, nxt):
-        """prefill() of distinct sequences in wide passes: each takes up to WIDE_COLS columns, a prompt cut where a pass
-        is full, and ends at most max_tokens prompts (the greedy ids of one call)."""
+        """prefill() of distinct sequences, the prompts' columns back to back, in calls of up to _pass_cols columns that
+        end with a chunk of max_tokens columns and end at most max_tokens prompts (the greedy ids of one call)."""
         lens = np.array([len(p) for p in prompts])
         first = np.cumsum(lens) - lens                       # each prompt's first column
         total = int(lens.sum())
@@ -732,25 +739,20 @@ class Qwen2Engine:
         if any(c.window is not None for c in caches):
             w = np.array([1 << 40 if c.window is None else c.window for c in caches])
             cols['ctx_lo'] = np.maximum(0, pos + 1 - np.repeat(w, lens))
-        c0, ends = 0, []                                     # first column of the pass, prompts that end in it
-
-        def flush(c1):
-            nonlocal c0, ends
-            ids = self._wide(cols[c0:c1], [first[s] + lens[s] - 1 - c0 for s in ends], want_ids=bool(ends))
-            for s, tid in zip(ends, ids if ends else []):
+        done = [s for s in range(len(prompts)) if lens[s]]   # prompts and the columns they end at, in column order
+        last = [int(first[s] + lens[s]) - 1 for s in done]
+        T, c0, e0 = self.max_tokens, 0, 0
+        while c0 < total:
+            c1 = min(total, c0 + self._pass_cols)
+            if e0 + T < len(last) and last[e0 + T] < c1:
+                c1 = c0 + (last[e0 + T] - c0) // T * T       # the chunk before the one that would end one too many
+            e1 = e0
+            while e1 < len(last) and last[e1] < c1:
+                e1 += 1
+            ids = self._wide(cols[c0:c1], [c - c0 for c in last[e0:e1]], want_ids=e1 > e0)
+            for s, tid in zip(done[e0:e1], ids if e1 > e0 else []):
                 nxt[s] = int(tid)
-            c0, ends = c1, []
-
-        for s in range(len(prompts)):
-            end = int(first[s] + lens[s])
-            while end - c0 > WIDE_COLS:
-                flush(c0 + WIDE_COLS)
-            if lens[s]:
-                ends.append(s)
-            if len(ends) == self.max_tokens:
-                flush(end)
-        if c0 < total:
-            flush(total)
+            c0, e0 = c1, e1
 
     @torch.inference_mode()
     def generate_batch(self, prompts, max_new_tokens=32, eos_token_id=None, window=None, graph=True):
