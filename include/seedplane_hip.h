@@ -306,8 +306,9 @@ int sp_op_sample(const float *logits_dev, int32_t vocab, int32_t ld, const int32
  * keeps z >= the k-th largest z (ties kept); top_p < 1 keeps the prefix of the z-descending order (ties by index)
  * whose exclusive cumulative mass is <= top_p of the kept mass; out_dev[s] = the inverse-CDF draw over what is kept
  * with uniform u_dev[s] (masses are 64-bit fixed point, exp(z - z_max) * 2^40, so every sum is exact).  Each draw
- * runs over many blocks (a short launch per radix level) with a histogram scratch the library keeps per device: calls
- * on one device must not overlap.  All pointers are device memory.  Errors: NULL pointers, bad sizes,
+ * runs over many blocks (3 to 6 launches) with a histogram scratch the library keeps per device: calls from several
+ * threads or on several streams of a device run one after the other (each waits, on the GPU, for the one before).  A call
+ * recorded by a stream capture is not ordered: its replays must not overlap other calls.  All pointers are device memory.  Errors: NULL pointers, bad sizes,
  * temperature <= 0, top_p <= 0. */
 int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, const int32_t *row_dev,
                           const double *u_dev, int32_t n, double temperature, int32_t top_k, double top_p,
@@ -316,7 +317,8 @@ int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, co
 /* sp_op_sample_filtered for callers whose uniforms are in host memory and who want the ids there (the same reference
  * interface and draws): u_host [n], out_host [n], and the row indices either on the device (row_dev) or in host memory
  * (row_host; exactly one of the two).  The kernels read the uniforms from and write the ids to pinned memory the
- * library keeps per device, so no copy runs on the stream; the call returns when the stream has finished. */
+ * library keeps per device, so no copy runs on the stream; the call returns when the stream has finished (SP_ESTATE on a
+ * stream that is being captured).  Calls from several threads take turns. */
 int sp_op_sample_filtered_host(const float *logits_dev, int32_t vocab, int32_t ld, const int32_t *row_dev,
                                const int32_t *row_host, const double *u_host, int32_t n, double temperature,
                                int32_t top_k, double top_p, int32_t *out_host, void *hip_stream);

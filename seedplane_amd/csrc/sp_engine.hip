@@ -12,6 +12,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <set>
 #include <mutex>
 #include <tuple>
@@ -2255,11 +2256,28 @@ int sp_op_gemv(const sp_weight *w, const void *x_dev, int32_t m_cols, float *y_d
 namespace lib_scratch {
 struct Smp { float *pmax; double *csum; };
 struct FmHost { double u[FM_ROWS]; int32_t row[FM_ROWS], id[FM_ROWS]; };       // pinned
-struct Fm { FmState *st; FmPair *list; FmHost *host; };
+// Filtered sampling: one call at a time uses a device's set (mu; the host entry holds it until its stream has finished, the
+// device entry leaves an event that the next call's stream waits for).  dirty: a call's launches did not all go through, so
+// the state is cleared before the next.
+struct Fm {
+    std::mutex mu;
+    FmState *st = nullptr;
+    FmPair *list = nullptr;
+    FmHost *host = nullptr;
+    hipEvent_t done = nullptr;
+    bool pending = false, dirty = false;
+    void release() {
+        dev_free(st);
+        dev_free(list);
+        if (host) (void)hipHostFree(host);
+        if (done) (void)hipEventDestroy(done);
+        st = nullptr; list = nullptr; host = nullptr; done = nullptr;
+    }
+};
 struct Acc { unsigned long long *xbuf; unsigned *err; int32_t *host; };
 struct Stage { unsigned char *buf = nullptr; size_t cap = 0; hipEvent_t done = nullptr; bool used = false; };
 std::map<int, Smp> smp;
-std::map<int, Fm> fm;
+std::map<int, std::shared_ptr<Fm>> fm;
 std::map<int, Acc> acc;
 std::map<int, Stage> stage;
 std::mutex smp_mu, fm_mu, acc_mu, stage_mu;
@@ -2304,28 +2322,48 @@ int sp_op_sample(const float *logits_dev, int32_t vocab, int32_t ld, const int32
 
 }  // extern "C"
 
-// Histograms, lists and per-row state for FM_ROWS draws and the pinned block, one set per device (calls on one device
-// must not overlap); zeroed once, each call's last kernel clears what the call used.
-static lib_scratch::Fm filtered_scratch() {
+// Histograms, lists and per-row state for FM_ROWS draws and the pinned block of the current device.
+static std::shared_ptr<lib_scratch::Fm> filtered_scratch() {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(lib_scratch::fm_mu);
     auto it = lib_scratch::fm.find(dev);
     if (it == lib_scratch::fm.end()) {
-        lib_scratch::Fm f{dev_alloc<FmState>(FM_ROWS), nullptr, nullptr};
+        auto f = std::make_shared<lib_scratch::Fm>();
         try {
-            f.list = dev_alloc<FmPair>((size_t)3 * FM_ROWS * FM_CAP);
-            HIPCHK(hipHostMalloc((void **)&f.host, sizeof(lib_scratch::FmHost), hipHostMallocDefault));
-            HIPCHK(hipMemset(f.st, 0, FM_ROWS * sizeof(FmState)));
+            f->st = dev_alloc<FmState>(FM_ROWS);
+            f->list = dev_alloc<FmPair>((size_t)3 * FM_ROWS * FM_CAP);
+            HIPCHK(hipHostMalloc((void **)&f->host, sizeof(lib_scratch::FmHost), hipHostMallocDefault));
+            HIPCHK(hipEventCreateWithFlags(&f->done, hipEventDisableTiming));
+            HIPCHK(hipMemset(f->st, 0, FM_ROWS * sizeof(FmState)));
         } catch (...) {
-            dev_free(f.st);
-            dev_free(f.list);
-            if (f.host) (void)hipHostFree(f.host);
+            f->release();
             throw;
         }
         it = lib_scratch::fm.emplace(dev, f).first;
     }
     return it->second;
+}
+static bool is_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(st, &cs));
+    return cs != hipStreamCaptureStatusNone;
+}
+// Before a call's first launch on st (mu is held): the scratch is clean and no earlier call still uses it.
+static void filtered_begin(lib_scratch::Fm &f, hipStream_t st) {
+    if (f.dirty) {
+        HIPCHK(hipDeviceSynchronize());
+        HIPCHK(hipMemset(f.st, 0, FM_ROWS * sizeof(FmState)));
+        f.dirty = f.pending = false;
+    }
+    if (f.pending) {
+        const hipError_t q = hipEventQuery(f.done);
+        if (q == hipErrorNotReady) (void)hipGetLastError();
+        else HIPCHK(q);
+        if (q == hipErrorNotReady) HIPCHK(hipStreamWaitEvent(st, f.done, 0));
+        else f.pending = false;
+    }
+    f.dirty = true;         // until the call's launches have all gone through
 }
 
 // The launches of at most FM_ROWS draws.
@@ -2333,24 +2371,24 @@ static void filtered_launch(const lib_scratch::Fm &sc, const float *logits, int 
                             const double *u, int n, double temperature, int top_k, double top_p, int32_t *out,
                             hipStream_t st) {
     const int k = top_k > 0 && top_k < vocab ? top_k : 0;
-    const FmArgs a{logits, vocab, ld, rows, u, (float)temperature, k, top_p, out, sc.st, sc.list, 0};
+    const FmArgs a{logits, vocab, ld, rows, u, (float)temperature, k, top_p, out, sc.st, sc.list};
     const dim3 grid((vocab + FM_SPAN - 1) / FM_SPAN, n), block(FS_THREADS);
-    hipLaunchKernelGGL(k_fm_top, grid, block, 0, st, a);
+    auto run = [&](auto kernel, dim3 g) {
+        hipLaunchKernelGGL(kernel, g, block, 0, st, a);
+        HIPCHK(hipGetLastError());
+    };
+    run(k_fm_top, grid);
     if (k && k <= FM_SMALL_K) {
-        hipLaunchKernelGGL(k_fm_gather<0>, grid, block, 0, st, a);
-        hipLaunchKernelGGL(k_fm_finish<true>, dim3(n), block, 0, st, a);
+        run(k_fm_gather<0>, grid);
+        run(k_fm_finish<true>, dim3(n));
     } else {
-        if (k) {
-            hipLaunchKernelGGL(k_fm_gather<1>, grid, block, 0, st, a);
-            hipLaunchKernelGGL(k_fm_mass<true>, grid, block, 0, st, a);
-        } else {
-            hipLaunchKernelGGL(k_fm_mass<false>, grid, block, 0, st, a);
-        }
-        if (top_p < 1.0) hipLaunchKernelGGL(k_fm_gather<2>, grid, block, 0, st, a);
-        hipLaunchKernelGGL(k_fm_gather<3>, grid, block, 0, st, a);
-        hipLaunchKernelGGL(k_fm_finish<false>, dim3(n), block, 0, st, a);
+        if (k) run(k_fm_gather<1>, grid);
+        if (k) run(k_fm_mass<true>, grid);
+        else run(k_fm_mass<false>, grid);
+        if (top_p < 1.0) run(k_fm_gather<2>, grid);
+        run(k_fm_gather<3>, grid);
+        run(k_fm_finish<false>, dim3(n));
     }
-    HIPCHK(hipGetLastError());
 }
 static void filtered_check(int32_t vocab, int32_t ld, int32_t n, double temperature, double top_p) {
     require(vocab >= 1 && ld >= vocab && n >= 1 && n <= 65535, SP_EINVAL, "bad sizes");
@@ -2366,10 +2404,20 @@ int sp_op_sample_filtered(const float *logits_dev, int32_t vocab, int32_t ld, co
     return guarded(nullptr, [&] {
         require(logits_dev && row_dev && u_dev && out_dev, SP_EINVAL, "NULL pointer");
         filtered_check(vocab, ld, n, temperature, top_p);
-        const lib_scratch::Fm sc = filtered_scratch();
+        const std::shared_ptr<lib_scratch::Fm> sc = filtered_scratch();
+        std::lock_guard<std::mutex> lock(sc->mu);
+        const hipStream_t st = (hipStream_t)stream;
+        const bool capturing = is_capturing(st);       // recorded launches run later: the caller orders the replays
+        require(!capturing || !sc->dirty, SP_ESTATE, "the sampling scratch needs a call outside a capture first");
+        if (!capturing) filtered_begin(*sc, st);
         for (int r0 = 0; r0 < n; r0 += FM_ROWS)
-            filtered_launch(sc, logits_dev, vocab, ld, row_dev + r0, u_dev + r0, std::min(FM_ROWS, n - r0), temperature, top_k,
-                            top_p, out_dev + r0, (hipStream_t)stream);
+            filtered_launch(*sc, logits_dev, vocab, ld, row_dev + r0, u_dev + r0, std::min(FM_ROWS, n - r0), temperature, top_k,
+                            top_p, out_dev + r0, st);
+        if (!capturing) {
+            HIPCHK(hipEventRecord(sc->done, st));
+            sc->pending = true;
+            sc->dirty = false;
+        }
     });
 }
 
@@ -2380,16 +2428,21 @@ int sp_op_sample_filtered_host(const float *logits_dev, int32_t vocab, int32_t l
         require(logits_dev && u_host && out_host && (row_dev != nullptr) != (row_host != nullptr), SP_EINVAL,
                 "NULL pointer, or not exactly one of row_dev and row_host");
         filtered_check(vocab, ld, n, temperature, top_p);
-        const lib_scratch::Fm sc = filtered_scratch();
+        const std::shared_ptr<lib_scratch::Fm> sc = filtered_scratch();
+        std::lock_guard<std::mutex> lock(sc->mu);
+        const hipStream_t st = (hipStream_t)stream;
+        require(!is_capturing(st), SP_ESTATE, "the call waits for its stream, which is being captured");
+        filtered_begin(*sc, st);
+        lib_scratch::FmHost &h = *sc->host;
         for (int r0 = 0; r0 < n; r0 += FM_ROWS) {
             const int nr = std::min(FM_ROWS, n - r0);
-            std::memcpy(sc.host->u, u_host + r0, nr * sizeof(double));
-            if (row_host) std::memcpy(sc.host->row, row_host + r0, nr * sizeof(int32_t));
-            filtered_launch(sc, logits_dev, vocab, ld, row_host ? sc.host->row : row_dev + r0, sc.host->u, nr, temperature, top_k,
-                            top_p, sc.host->id, (hipStream_t)stream);
-            HIPCHK(hipStreamSynchronize((hipStream_t)stream));
-            std::memcpy(out_host + r0, sc.host->id, nr * sizeof(int32_t));
+            std::memcpy(h.u, u_host + r0, nr * sizeof(double));
+            if (row_host) std::memcpy(h.row, row_host + r0, nr * sizeof(int32_t));
+            filtered_launch(*sc, logits_dev, vocab, ld, row_host ? h.row : row_dev + r0, h.u, nr, temperature, top_k, top_p, h.id, st);
+            HIPCHK(hipStreamSynchronize(st));
+            std::memcpy(out_host + r0, h.id, nr * sizeof(int32_t));
         }
+        sc->pending = sc->dirty = false;
     });
 }
 
@@ -2581,7 +2634,11 @@ int sp_library_release(void) {
                 HIPCHK(hipDeviceSynchronize());
             }
             for (auto &kv : lib_scratch::smp) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.pmax); dev_free(kv.second.csum); }
-            for (auto &kv : lib_scratch::fm) { HIPCHK(hipSetDevice(kv.first)); dev_free(kv.second.st); dev_free(kv.second.list); if (kv.second.host) HIPCHK(hipHostFree(kv.second.host)); }
+            for (auto &kv : lib_scratch::fm) {
+                std::lock_guard<std::mutex> f(kv.second->mu);
+                HIPCHK(hipSetDevice(kv.first));
+                kv.second->release();
+            }
             for (auto &kv : lib_scratch::acc) {
                 HIPCHK(hipSetDevice(kv.first));
                 dev_free(kv.second.xbuf);

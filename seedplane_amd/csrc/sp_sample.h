@@ -134,8 +134,7 @@ __global__ void __launch_bounds__(SMS_T) k_smp_draw(const float *logits, int V, 
             for (int i = wlo + t; i < whi; i += SMS_T) w[i - wlo] = smp_weight(l, i, m, invT);
             __syncthreads();
             if (t == 0 && pick < 0) {
-                // in index order, 16 weights read ahead at a time (entries past the window read a zero pad and are
-                // not visited)
+                // in index order, 16 weights read ahead at a time (what lies past the window is read, never used)
                 for (int i0 = wlo; i0 < whi && pick < 0; i0 += 16) {
                     double c[16];
 #pragma unroll
@@ -751,7 +750,8 @@ constexpr int FM_CAP = 8192;                       // entries a list holds
 // octave of z each) hold a few thousand entries at most for ordinary logits
 constexpr int FM_SMALL_K = 1024;
 struct FmPair { uint32_t key; int idx; };
-// Per-row scratch.  kmax, n and the histograms are zero between calls: the finishing kernel clears what the call used.
+// Per-row scratch.  kmax, n and the histograms are zero between calls: the finishing kernel clears what the call used, and
+// the host clears everything after a call whose launches did not all go through.
 struct FmState {
     unsigned long long mass[FM_B0];
     unsigned int cnt[FM_B0];
@@ -759,8 +759,7 @@ struct FmState {
     unsigned int n[3];                             // entries of lists 0 (top-k), 1 (top-p), 2 (draw)
     unsigned int kbin, krem, kmin;                 // top-k: boundary bin, tokens to take from it; smallest kept key
     unsigned int tbin, dbin;                       // bins of the top-p cut and of the draw
-    unsigned long long tabove, dabove, tp, tgt;    // mass before those bins, and the targets
-    int topp;                                      // 1: the top-p cut applies (tp < kept mass)
+    unsigned long long tabove, dabove, tgt;        // mass before those bins, and the draw's target
 };
 struct FmArgs {
     const float *logits;
@@ -773,7 +772,6 @@ struct FmArgs {
     int *out;
     FmState *st;                                   // [FM_ROWS]
     FmPair *list;                                  // [3][FM_ROWS][FM_CAP]
-    int row0;                                      // draws row0 .. row0 + gridDim.y - 1 (blockIdx.y = draw - row0)
 };
 
 struct FmScan {                                    // LDS of the block-wide choices
@@ -952,7 +950,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_top(FmArgs a) {
     __shared__ unsigned int red[FS_THREADS / 64];
     __shared__ unsigned int h[FM_B0];
     const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    const float *row = a.logits + (size_t)a.rows[r] * a.ld;
     float lv[FM_U];
 #pragma unroll
     for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
@@ -995,7 +993,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_mass(FmArgs a) {
     __shared__ FmScan sc;
     const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
     FmState &S = a.st[r];
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    const float *row = a.logits + (size_t)a.rows[r] * a.ld;
     float lv[FM_U];
 #pragma unroll
     for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
@@ -1027,7 +1025,7 @@ __device__ __forceinline__ bool fm_cut(const FmArgs &a, unsigned long long F, un
     return a.top_p < 1.0 && tp < F;
 }
 __device__ __forceinline__ unsigned long long fm_target(const FmArgs &a, int r, unsigned long long K) {
-    unsigned long long t = (unsigned long long)(a.u[a.row0 + r] * (double)K);
+    unsigned long long t = (unsigned long long)(a.u[r] * (double)K);
     return t >= K ? K - 1 : t;
 }
 // The kept mass after the cut: the tokens before the cut's key and those of the key up to the cut.
@@ -1049,7 +1047,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_gather(FmArgs a) {
     const int r = blockIdx.y, i0 = blockIdx.x * FM_SPAN;
     FmState &S = a.st[r];
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    const float *row = a.logits + (size_t)a.rows[r] * a.ld;
     float lv[FM_U];
 #pragma unroll
     for (int u = 0; u < FM_U; ++u) lv[u] = row[min(i0 + u * FS_THREADS + (int)threadIdx.x, a.V - 1)];
@@ -1064,7 +1062,6 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_gather(FmArgs a) {
         unsigned long long tp;
         const bool cut = fm_cut(a, F, tp);
         if constexpr (MODE == 2) {
-            if (lead) { S.topp = cut; S.tp = tp; }
             if (!cut) return;
             bin = fm_choose<FM_B0>(S.mass, 0ull, tp, above, sc);
             if (lead) { S.tbin = bin; S.tabove = above; }
@@ -1226,14 +1223,14 @@ __global__ void __launch_bounds__(FS_THREADS) k_fm_finish(FmArgs a) {
     __shared__ FmScan sc;
     const int r = blockIdx.x;
     FmState &S = a.st[r];
-    const float *row = a.logits + (size_t)a.rows[a.row0 + r] * a.ld;
+    const float *row = a.logits + (size_t)a.rows[r] * a.ld;
     const float zmax = fs_unkey(S.kmax);
     const FmSource src = fm_source(a, r, SMALL ? 0 : 2, row, lds);
     int tok;
     if (SMALL && src.listed && src.n >= 1 && src.n <= FS_THREADS) tok = fm_small_list(a, r, src, zmax, h, sc);
     else tok = fm_descents<SMALL>(a, r, src, row, zmax, m0, h, sc);
     if (threadIdx.x == 0) {
-        a.out[a.row0 + r] = tok;
+        a.out[r] = tok;
         S.kmax = 0u;
         S.n[0] = S.n[1] = S.n[2] = 0u;
     }
