@@ -92,10 +92,10 @@ def _ptr(a):
 def _id_array(ids):
     """Token ids (or positions) of any shape and integer-like type as a flat int64 array (reference:
     torch.as_tensor(ids, dtype=torch.long).flatten(), qwen_engine.py:107)."""
-    if isinstance(ids, list):
-        a = np.array(ids)                      # a list of plain integers, without a tensor in between
+    if isinstance(ids, list) and set(map(type, ids)) == {int}:
+        a = np.array(ids)                      # without a tensor in between
         if a.dtype == np.int64:
-            return a.reshape(-1)
+            return a
     return torch.as_tensor(ids, dtype=torch.long).flatten().cpu().numpy()
 
 
