@@ -26,6 +26,7 @@
 #include "sp_decode1.h"
 #include "sp_gemv.h"
 #include "sp_gemv1.h"
+#include "sp_order.h"
 #include "sp_pack.h"
 #include "sp_sample.h"
 #include "sp_wide.h"
@@ -1368,10 +1369,10 @@ bool sp_engine::run_d1(const sp_token &t, int flags) {
     return true;
 }
 
-// After a synchronisation: a persistent step whose block gave up (a hand-off that never arrived) is reported once.
+// A persistent step whose block gave up (a hand-off that never arrived) is reported once.  Looked at when a call begins,
+// without a wait, and after a synchronisation.
 void sp_engine::check_d1_error() {
-    if (!h_d1err || *(volatile unsigned *)h_d1err == 0) return;
-    *(volatile unsigned *)h_d1err = 0;
+    if (!sp::take_error(h_d1err, [&] { HIPCHK(hipStreamSynchronize(stream)); })) return;
     throw Fail{SP_EHIP, "persistent decode step: a block hand-off timed out (the step's results are invalid)"};
 }
 
