@@ -672,6 +672,8 @@ struct sp_engine {
     d1::LayerPtr *d1_layers = nullptr;
     d1::Static *d1_static = nullptr;
     unsigned d1_seq = 0;
+    bool d1_joined = false;      // the engine's stream is known to the order of the persistent launches
+    void leave_stream();
     bool prepare_d1();
     bool launch_d1(const sp_token &t, int flags);     // the persistent kernel alone
     bool run_d1(const sp_token &t, int flags);        // + the error word copy, the head GEMV and the argmax
@@ -1311,20 +1313,34 @@ bool sp_engine::prepare_d1() {
     return true;
 }
 
-// The stream of the last persistent launch on each device.  Two such kernels must not run at once (each needs every CU
-// for one of its blocks): a launch on another stream first waits for that one.  The entry is dropped, after a
-// synchronisation, when an engine leaves a stream, so the stream named here belongs to a live engine.
 namespace {
-struct D1Last { hipStream_t stream = nullptr; hipEvent_t ev = nullptr; bool any = false; };
+struct HipOrder {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    bool capturing(hipStream_t s) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(s, &cs));
+        return cs != hipStreamCaptureStatusNone;
+    }
+    void sync(hipStream_t s) { HIPCHK(hipStreamSynchronize(s)); }
+    void record(hipEvent_t &ev, hipStream_t s) {
+        if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        HIPCHK(hipEventRecord(ev, s));
+    }
+    void wait(hipStream_t s, hipEvent_t ev) { HIPCHK(hipStreamWaitEvent(s, ev, 0)); }
+};
 std::mutex d1_mu;
-std::map<int, D1Last> d1_last;
-void d1_leave_stream(int device, hipStream_t stream) {
-    std::lock_guard<std::mutex> lock(d1_mu);
-    (void)hipStreamSynchronize(stream);
-    auto it = d1_last.find(device);
-    if (it != d1_last.end() && it->second.stream == stream) it->second.any = false;
-}
+std::map<int, sp::PersistentOrder<HipOrder>> d1_order;       // by device
 }  // namespace
+
+// The engine is about to leave its stream: what it queued there is waited for.
+void sp_engine::leave_stream() {
+    (void)hipStreamSynchronize(stream);
+    if (!d1_joined) return;
+    std::lock_guard<std::mutex> lock(d1_mu);
+    d1_order[device].leave(stream);
+    d1_joined = false;
+}
 
 // One column through the persistent kernel, then the LM head GEMV and the argmax as in the chain.
 // The kernel needs its blocks co-resident (one per CU; the LDS size allows no second one, checked in prepare_d1) but
@@ -1343,12 +1359,10 @@ bool sp_engine::launch_d1(const sp_token &t, int flags) {
     const d1::Static *sp = d1_static;
     void *args[] = {(void *)&sp, &a};
     std::lock_guard<std::mutex> lock(d1_mu);
-    D1Last &last = d1_last[device];
-    if (last.any && last.stream != stream) {
-        if (!last.ev) HIPCHK(hipEventCreateWithFlags(&last.ev, hipEventDisableTiming));
-        HIPCHK(hipEventRecord(last.ev, last.stream));
-        HIPCHK(hipStreamWaitEvent(stream, last.ev, 0));
-    }
+    sp::PersistentOrder<HipOrder> &order = d1_order[device];
+    HipOrder rt;
+    if (!d1_joined) { order.join(stream); d1_joined = true; }
+    order.before(rt, stream);
     const hipError_t le = hipLaunchKernel(d1k->fn, dim3(d1g.nb), dim3(d1::NT), args, d1::SMEM_BYTES, stream);
     if (le != hipSuccess) {
         (void)hipGetLastError();
@@ -1356,8 +1370,7 @@ bool sp_engine::launch_d1(const sp_token &t, int flags) {
         d1_why = std::string("launch refused: ") + hipGetErrorString(le);
         return false;
     }
-    last.any = true;
-    last.stream = stream;
+    order.after(rt, stream);
     return true;
 }
 bool sp_engine::run_d1(const sp_token &t, int flags) {
@@ -1530,7 +1543,7 @@ int sp_engine_create(const sp_model_desc *desc, sp_engine **out) {
 
 void sp_engine_destroy(sp_engine *e) {
     if (!e) return;
-    d1_leave_stream(e->device, e->stream);
+    e->leave_stream();
     e->free_all();
     delete e;
 }
@@ -1539,7 +1552,7 @@ int sp_engine_set_stream(sp_engine *e, void *s) {
     if (!e) { g_err = "engine is NULL"; return SP_EINVAL; }
     return guarded(e, [&] {
         HIPCHK(hipStreamSynchronize(e->stream));
-        d1_leave_stream(e->device, e->stream);
+        e->leave_stream();
         if (e->own_stream) HIPCHK(hipStreamDestroy(e->stream));
         e->drop_graphs();
         e->stream = (hipStream_t)s;
