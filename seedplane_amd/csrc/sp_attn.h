@@ -678,13 +678,19 @@ __device__ __forceinline__ void argmax_range(const float *x, int lo, int hi, flo
 // 64-bit atomic maximum, the larger value first and the smaller index on equal values (-0 counts as +0); the block that
 // completes the row's count writes the id, also to pinned host memory (host, so that a caller's read-back is no copy of
 // its own), and clears both words for the next call.  Relaxed agent-scope atomics only: the count is raised after the
-// maximum has returned.  gridDim.x: argmax_blocks(cols), one load batch per thread for short rows (their blocks would
-// do little but queue on the row's words).  One 151936-entry row: 10.8 us as two launches and serial loads, then a 4 us copy of the id.
-__host__ __device__ constexpr int argmax_blocks(int cols) {
-    return cols <= 2048 ? 1 : cols >= 2048 * ARGMAX_BLOCKS ? ARGMAX_BLOCKS : (cols + 2047) / 2048;
+// maximum has returned.  Each row's words have a 256-byte line of their own: packed words of 16 rows queued on one line
+// (151936 entries: 1, 16, 32, 64 rows 5.1, 16.7, 25.6, 43.8 us; the two passes 5.7, 6.7, 8.4, 13.0; padded, with
+// argmax_blocks, 5.1, 5.6, 6.7, 9.2).
+struct __align__(256) ArgmaxRow { unsigned long long best; unsigned count; };
+// Blocks per row: one load batch per thread for short rows (their blocks would do little but queue on the row's words), and
+// about 512 in all for many long ones (64 rows of 151936: 64 blocks each 12.5 us, 16 blocks 9.2; 1 row: 64 blocks 5.1, 16
+// blocks 6.2).
+__host__ __device__ constexpr int argmax_blocks(int cols, int rows) {
+    const int most = rows <= 8 ? ARGMAX_BLOCKS : rows >= 32 ? 16 : 512 / rows;
+    return cols <= 2048 ? 1 : (cols + 2047) / 2048 < most ? (cols + 2047) / 2048 : most;
 }
-__global__ void __launch_bounds__(256) k_argmax_row(const float *x, int cols, int ld, unsigned long long *best,
-                                                    unsigned *count, int *out, int *host) {
+__global__ void __launch_bounds__(256) k_argmax_row(const float *x, int cols, int ld, ArgmaxRow *words, int *out,
+                                                    int *host) {
     __shared__ float sv[4];
     __shared__ int si[4];
     const int row = blockIdx.y, per = (cols + gridDim.x - 1) / gridDim.x;
@@ -699,11 +705,11 @@ __global__ void __launch_bounds__(256) k_argmax_row(const float *x, int cols, in
     const uint32_t b = __float_as_uint(bv == 0.f ? 0.f : bv);
     const uint32_t key = (b & 0x80000000u) ? ~b : (b | 0x80000000u);       // larger value, larger key
     const unsigned long long mine = ((unsigned long long)key << 32) | (uint32_t)~bi;
-    unsigned long long prev = __hip_atomic_fetch_max(best + row, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long prev = __hip_atomic_fetch_max(&words[row].best, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("" : "+v"(prev)::"memory");
-    if (__hip_atomic_fetch_add(count + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
-    const unsigned long long all = __hip_atomic_exchange(best + row, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(count + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(&words[row].count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
+    const unsigned long long all = __hip_atomic_exchange(&words[row].best, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&words[row].count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int id = (int)~(uint32_t)all;
     out[row] = host[row] = id == 0x7fffffff ? 0 : id;
 }

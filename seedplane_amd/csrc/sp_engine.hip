@@ -628,8 +628,7 @@ struct sp_engine {
     // the fp16 remainders (split_f16) of the normalised GEMV inputs (qkv always; gate_up in one-column steps) and of
     // the SwiGLU activation of one-column steps
     f16 *xn_lo = nullptr, *act_lo = nullptr;
-    unsigned long long *am_best = nullptr;      // the argmax's row words and counts (zero between calls)
-    unsigned *am_count = nullptr;
+    ArgmaxRow *am_words = nullptr;              // the argmax's words per row (zero between calls)
     int *am_out = nullptr;
     int argmax_cols = 0;         // columns whose argmax ids am_out holds (the last SP_F_ARGMAX call)
     // column descriptors of a call: tokens, attention groups, chunk counts, uploaded together from a pinned staging
@@ -736,7 +735,7 @@ void sp_engine::free_all() {
     dev_free(final_norm); dev_free(inv_freq);
     for (void *p : {(void *)x, (void *)x2, (void *)qkv, (void *)q, (void *)rtab, (void *)logits, (void *)attn_part, (void *)gpart,
                     (void *)gpart2, (void *)xn, (void *)attn, (void *)xn_lo, (void *)act_lo,
-                    (void *)act, (void *)am_best, (void *)am_count, (void *)am_out,
+                    (void *)act, (void *)am_words, (void *)am_out,
                     (void *)d_upload, (void *)d_kl, (void *)d_vl, (void *)d_move})
         dev_free(p);
     for (auto p : kc) dev_free(p);
@@ -774,10 +773,8 @@ void sp_engine::alloc_activations() {
     attn = dev_alloc<f16>(tpad * d.n_heads * d.head_dim);
     act = dev_alloc<f16>(tpad * I);
     logits = dev_alloc<float>((size_t)maxT * V);
-    am_best = dev_alloc<unsigned long long>(maxT);
-    am_count = dev_alloc<unsigned>(maxT);
-    HIPCHK(hipMemset(am_best, 0, maxT * sizeof(unsigned long long)));
-    HIPCHK(hipMemset(am_count, 0, maxT * sizeof(unsigned)));
+    am_words = dev_alloc<ArgmaxRow>(maxT);
+    HIPCHK(hipMemset(am_words, 0, maxT * sizeof(ArgmaxRow)));
     am_out = dev_alloc<int>(maxT);
     HIPCHK(hipMemset(am_out, 0, maxT * sizeof(int)));
     argmax_cols = 0;
@@ -1106,8 +1103,8 @@ bool sp_engine::alloc_wide() {
 
 // Greedy ids of n rows of logits (vocab apart) into am_out[first ..) and the pinned copy.
 void sp_engine::launch_ids(const float *rows, int n, int first) {
-    hipLaunchKernelGGL(k_argmax_row, dim3(argmax_blocks(d.vocab), n), dim3(256), 0, stream, rows, d.vocab, d.vocab, am_best,
-                       am_count, am_out + first, h_ids + first);
+    hipLaunchKernelGGL(k_argmax_row, dim3(argmax_blocks(d.vocab, n), n), dim3(256), 0, stream, rows, d.vocab, d.vocab, am_words,
+                       am_out + first, h_ids + first);
 }
 
 // Whether a chunk of n columns can be part of a wide pass: its step sums every product in the order of several column tiles

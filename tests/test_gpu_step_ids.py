@@ -64,3 +64,20 @@ def test_two_engines_on_two_streams(gpu_device):
     for k, (e, _) in enumerate(pairs):
         _lib.check(e.lib.sp_engine_sync(e.h), e.h)
         assert [int(t) for t in got[k]] == want
+
+
+@pytest.mark.parametrize('n', [9, 31, 64])
+def test_ids_of_many_long_rows(gpu_device, n):
+    """Batches whose rows share the launch's blocks (fewer per row than for one row), step after step."""
+    print(f'ids of {n} rows', flush=True)
+    vocab = 140000
+    cfg, w = make_weights(preset('tiny', vocab_size=vocab), 'q8', seed=n)
+    eng = Qwen2Engine(config=cfg, tensors=w, max_tokens=64)
+    eng.reserve(n, 32)
+    caches = [eng.new_cache(32) for _ in range(n)]
+    rows = torch.empty((n, vocab), device=eng.device)
+    toks = random_prompt(n, vocab, seed=n)
+    for step in range(3):
+        ids = eng.decode(toks, caches, logits_out=rows)
+        assert [int(i) for i in ids] == rows.cpu().argmax(dim=1).tolist(), step
+        toks = [(t * 5 + 1) % vocab for t in toks]
