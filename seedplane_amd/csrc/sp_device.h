@@ -69,8 +69,16 @@ __device__ __forceinline__ uint32_t q4_nibbles(uint32_t v) {
     asm("" : "+v"(exponent));
     return (v & mask) | exponent;
 }
-// 8 uint4 codes of one dword -> 8 fp16 1024 + c (exact; see q4_unpack8 for the nibble order).
+// 8 uint4 codes of one dword -> 8 fp16 1024 + c (exact; see q4_unpack8 for the nibble order).  PIN: the constants in
+// registers (q4_nibbles).  The one-column GEMV leaves them literals: its waves hold all their tiles in 128 registers, and
+// the pinned constants spilled more of them (Qwen2-7B gate_up 58.5 -> 61.0 us, 8192 rows of the head 14.8 -> 20.8).
+template <bool PIN = true>
 __device__ __forceinline__ f16x8 q4_biased8(uint32_t v) {
+    if constexpr (!PIN) {
+        const uint32_t a = (v & 0x000F000Fu) | 0x64006400u, b = ((v >> 4) & 0x000F000Fu) | 0x64006400u;
+        const uint32_t c = ((v >> 8) & 0x000F000Fu) | 0x64006400u, d = ((v >> 12) & 0x000F000Fu) | 0x64006400u;
+        return __builtin_bit_cast(f16x8, (u32x4){a, b, c, d});
+    }
     return __builtin_bit_cast(f16x8, (u32x4){q4_nibbles(v), q4_nibbles(v >> 4), q4_nibbles(v >> 8), q4_nibbles(v >> 12)});
 }
 // 8 uint4 codes of one dword -> 8 fp16 in k order.  The packer stores k-order codes c0..c7 at nibble positions

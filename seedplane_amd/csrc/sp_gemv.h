@@ -62,10 +62,10 @@ __device__ __forceinline__ f16x8 unpack_step(const u32x4 &t, int s) {
 }
 // The codes of step s offset by QBIAS<FMT> (exact fp16; Q8 and Q4 only).
 template <int FMT> struct QBias { static constexpr float V = FMT == 2 ? 1152.f : 1024.f; };
-template <int FMT>
+template <int FMT, bool PIN = true>
 __device__ __forceinline__ f16x8 biased_step(const u32x4 &t, int s) {
     if constexpr (FMT == 2) return s == 0 ? q8_biased8(t[0], t[1]) : q8_biased8(t[2], t[3]);
-    else return q4_biased8(t[s]);
+    else return q4_biased8<PIN>(t[s]);
 }
 
 // Threads per block: single-column-tile variants with one unit per block use up to 16 waves (128 VGPRs each), those

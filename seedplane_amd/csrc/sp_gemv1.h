@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(1024) k_gemv1(GemvArgs a, ProArgs p) {
                 const f32x4 sx = mfma16(xa, ones8, (f32x4){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                 for (int i = 0; i < RG; ++i) {
-                    const f32x4 dd = mfma16(xa, biased_step<FMT>(wt[t][i], s), (f32x4){0.f, 0.f, 0.f, 0.f});
+                    const f32x4 dd = mfma16(xa, biased_step<FMT, false>(wt[t][i], s), (f32x4){0.f, 0.f, 0.f, 0.f});
                     float scale, offs;
                     if constexpr (FMT == 2) {
                         const uint32_t d = sq8[t][i];
