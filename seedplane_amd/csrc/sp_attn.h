@@ -1,6 +1,8 @@
 // Decode-side kernels around the GEMVs: embedding gather, RMSNorm, RoPE + KV-cache write, split-K GQA attention
 // (windowed ring slots + tree ancestor mask), split-K combine, two-pass argmax, KV slot moves.
 #pragma once
+#include <type_traits>
+
 #include "sp_device.h"
 #include "../../include/seedplane_hip.h"
 
@@ -612,16 +614,16 @@ __global__ void __launch_bounds__(64 * NWV) k_attn_dec(AttnArgs a, f16 *out, int
 // The chunk outputs are read in batches of CMB_BATCH with every load of a batch in flight together (the first batch
 // before the weights are known); the accumulation runs over the chunks in ascending order.
 constexpr int CMB_BATCH = 16;
-// (col0: the launch's first column, whose records stand first in part.)
+// (col0: the launch's first column, whose record comes first in part and whose count comes first in col_nchunk.)
 __global__ void __launch_bounds__(128) k_attn_combine(const float *part, const int *col_nchunk, int NH, int HD,
                                                       int nchunk, f16 *out, int ldo, int mtp, int col0) {
     __shared__ float w_s[ATT_MAX_CHUNKS];
     __shared__ float l_s[ATT_MAX_CHUNKS];
     __shared__ float red[16];
-    const int h = blockIdx.x, b = col0 + blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
+    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
     const int nc = col_nchunk[b];
     const int rec = part_floats(HD);
-    const float *p = part + ((size_t)blockIdx.y * NH + h) * nchunk * rec;
+    const float *p = part + ((size_t)b * NH + h) * nchunk * rec;
     const int d = min(tid, HD - 1), last = max(nc - 1, 0);     // clamped: every load is in bounds
     float v[CMB_BATCH];
 #pragma unroll
@@ -657,7 +659,7 @@ __global__ void __launch_bounds__(128) k_attn_combine(const float *part, const i
         for (int i = 0; i < CMB_BATCH; ++i)
             if (c0 + i < nc) acc += w_s[c0 + i] * v[i];
     }
-    if (tid < HD) out[act_off(b, h * HD + tid, ldo, mtp)] = (f16)(acc / L);
+    if (tid < HD) out[act_off(col0 + b, h * HD + tid, ldo, mtp)] = (f16)(acc / L);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -802,7 +804,8 @@ __global__ void __launch_bounds__(256) k_kv_fill(f16 *const *kl, f16 *const *vl,
 // k_attn_part, so k_attn_combine merges them (with the group's chunk count per column).
 struct AttnGroup {
     int first_col, ncols, seq, lo, nlin, tree_base, tree_count;
-    int run_col, run_pos;  // STAGED: the first column of the sequence's run in the call, and its position
+    int run_col;           // STAGED: the first column of the sequence's run in the call, whose position stands in tree_base
+                           // (there are no tree blocks)
 };
 
 struct AttnMqArgs {
@@ -814,7 +817,8 @@ struct AttnMqArgs {
     float scale;
     float *part;
     int splits;            // blocks per (chunk, kv head, group); block s takes row tiles 4s .. 4s+3
-    // STAGED only
+};
+struct AttnMqStaged : AttnMqArgs {
     const f16 *kn, *vn;    // K and V of the call's columns [kv_head][cap][HD], beside the ring
     int cap, col0;         // columns the staging area holds; the launch's first column (its records stand first in part)
 };
@@ -825,7 +829,7 @@ struct AttnMqArgs {
 // Qwen2-1.5B, window 1024: 70 us and 31 for the combine (two chunks per block, one after the other on the same queries: 84;
 // one pass with an online softmax, whose bits differ from a step's: 55).
 template <int HD, int G, int CH, bool STAGED = false>
-__global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
+__global__ void __launch_bounds__(256) k_attn_mq(std::conditional_t<STAGED, AttnMqStaged, AttnMqArgs> a) {
     constexpr int KP = HD + 8, VP = CH + 8;          // padded rows (halves), 16-byte aligned
     constexpr int NST = CH / 16, NS2 = CH / 32, NP2 = CH / 2;   // key tiles, P.V k-steps, key pairs
     constexpr int ST = HD / 32;                      // MFMA k-steps over head dim
@@ -872,13 +876,20 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
         kp = lin ? gr.lo + vis : ~tj;
         return wrap(lin ? lin_base + j : gr.tree_base + tj);
     };
-    const size_t stage_base = STAGED ? (size_t)kvh * a.cap + gr.run_col : 0;
-    // row (of HD values) of visible key j, in the ring or (staged) in the staging area
-    auto row_at = [&](int j, bool &staged) -> size_t {
+    // K and V row (HD values) of visible key j, in the ring or (staged) in the staging area
+    auto rows_at = [&](int j, const f16 *&k, const f16 *&v) {
         int kp;
-        const int slot = key_at(j, kp);
-        staged = STAGED && kp >= gr.run_pos;
-        return staged ? stage_base + (kp - gr.run_pos) : head_base + slot;
+        size_t row = head_base + key_at(j, kp);
+        k = a.kc;
+        v = a.vc;
+        if constexpr (STAGED) {
+            const bool staged = kp >= gr.tree_base;
+            row = staged ? (size_t)kvh * a.cap + gr.run_col + (kp - gr.tree_base) : row;
+            k = staged ? a.kn : k;
+            v = staged ? a.vn : v;
+        }
+        k += row * HD;
+        v += row * HD;
     };
 
     // ---- every global load before the first LDS store.  Keys past cnt load key 0 of the chunk (clamped address,
@@ -888,9 +899,9 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
 #pragma unroll
     for (int i = 0; i < KPER; ++i) {
         const int idx = tid + 256 * i, j = idx / CPR, ch = idx - j * CPR;
-        bool sg;
-        const size_t row = row_at(j < cnt ? j : 0, sg);
-        kf[i] = *(const f16x8 *)((sg ? a.kn : a.kc) + row * HD + ch * 8);
+        const f16 *k, *v;
+        rows_at(j < cnt ? j : 0, k, v);
+        kf[i] = *(const f16x8 *)(k + ch * 8);
     }
 #pragma unroll
     for (int i = 0; i < VPER; ++i) {
@@ -898,9 +909,9 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int j = 2 * kp2 + h;
-            bool sg;
-            const size_t row = row_at(j < cnt ? j : 0, sg);
-            vf[i][h] = *(const f16x8 *)((sg ? a.vn : a.vc) + row * HD + ch * 8);
+            const f16 *k, *v;
+            rows_at(j < cnt ? j : 0, k, v);
+            vf[i][h] = *(const f16x8 *)(v + ch * 8);
         }
     }
     // Q fragments (A operand) of row rt*16 + r16, dims 32s + 8*g4 .. +8, from a clamped row; rows past R are zero.
@@ -1056,7 +1067,8 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnMqArgs a) {
         const int row = rt * 16 + 4 * g4 + j;
         if (row < R) {
             const int col = row / G, h = row - col * G;
-            const size_t pcol = gr.first_col + col - (STAGED ? a.col0 : 0);
+            size_t pcol = gr.first_col + col;
+            if constexpr (STAGED) pcol -= a.col0;
             float *out = a.part + ((pcol * a.NH + kvh * G + h) * a.nchunk + c) * part_floats(HD);
             f16 *oh = (f16 *)(out + 2);
             const float il = lrow[j] > 0.f ? 1.f / lrow[j] : 0.f;

@@ -376,7 +376,7 @@ void launch_attn_rope_hd(int G, dim3 grid, hipStream_t st, const AttnArgs &a, co
 // query rows, fewer and larger blocks, half the records to merge; -1 % per pass), 64 otherwise (the plain batches
 // and prefill chunks got slower with 128: bs16 +16 %, prefill +3 %).
 template <int HD, int CH, bool STAGED>
-void launch_attn_mq_ch(int G, dim3 grid, hipStream_t st, const AttnMqArgs &a) {
+void launch_attn_mq_ch(int G, dim3 grid, hipStream_t st, const std::conditional_t<STAGED, AttnMqStaged, AttnMqArgs> &a) {
     switch (G) {
         case 1: hipLaunchKernelGGL((k_attn_mq<HD, 1, CH, STAGED>), grid, dim3(256), 0, st, a); break;
         case 2: hipLaunchKernelGGL((k_attn_mq<HD, 2, CH, STAGED>), grid, dim3(256), 0, st, a); break;
@@ -940,8 +940,7 @@ void sp_engine::launch_attention(int l, int n, const AttnPlan &ap, int mtp, hipS
     const int NH = d.n_heads, NKV = d.n_kv_heads, HD = d.head_dim, G = NH / NKV, nchunk = ap.nchunk;
     const float scale = 1.0f / std::sqrt((float)HD);
     if (ap.mq) {
-        AttnMqArgs am{q, kc[l], vc[l], dtoks, dgroups, NH, NKV, HD, n_slots, nchunk, scale, attn_part, ap.splits, nullptr,
-                      nullptr, 0, 0};
+        AttnMqArgs am{q, kc[l], vc[l], dtoks, dgroups, NH, NKV, HD, n_slots, nchunk, scale, attn_part, ap.splits};
         dim3 agrid(nchunk, NKV, ap.ngroups * ap.splits);
         if (HD == 64) launch_attn_mq_hd<64>(G, ap.mq_ch, agrid, st, am);
         else launch_attn_mq_hd<128>(G, ap.mq_ch, agrid, st, am);
@@ -1153,7 +1152,7 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<Attn
             for (AttnGroup g : ap.groups) {
                 g.first_col += col;
                 g.run_col = run_of[g.first_col];
-                g.run_pos = toks[g.run_col].ctx_hi;
+                g.tree_base = toks[g.run_col].ctx_hi;
                 groups.push_back(g);
             }
             colnc.insert(colnc.end(), ap.colnc.begin(), ap.colnc.end());
@@ -1214,12 +1213,12 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<Attn
                     while (oi < outs.size() && outs[oi].col < w.col0) ++oi;
                     if (oi == outs.size() || outs[oi].col >= w.col0 + w.cols) continue;
                 }
-                AttnMqArgs am{wd.q, kc[l], vc[l], dt, dgr + w.g0, NH, NKV, HD, n_slots, w.nchunk, scale, w.part, w.splits, wd.kn,
-                              wd.vn, WIDE_COLS, w.col0};
+                const AttnMqStaged am{{wd.q, kc[l], vc[l], dt, dgr + w.g0, NH, NKV, HD, n_slots, w.nchunk, scale, w.part, w.splits},
+                                      wd.kn, wd.vn, WIDE_COLS, w.col0};
                 const dim3 grid(w.nchunk, NKV, w.groups * w.splits);
                 if (HD == 64) launch_attn_mq_ch<64, ATT_CH, true>(G, grid, stream, am);
                 else launch_attn_mq_ch<128, ATT_CH, true>(G, grid, stream, am);
-                hipLaunchKernelGGL(k_attn_combine, dim3(NH, w.cols), dim3(HD), 0, stream, w.part, dnc, NH, HD, w.nchunk, wd.attn,
+                hipLaunchKernelGGL(k_attn_combine, dim3(NH, w.cols), dim3(HD), 0, stream, w.part, dnc + w.col0, NH, HD, w.nchunk, wd.attn,
                                    NH * HD, mtp, w.col0);
             }
         }

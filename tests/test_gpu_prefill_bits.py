@@ -55,7 +55,8 @@ SWEEP = [
     ('small', 'f16', [65, 81, 129, 640], None), ('small', 'q8', [80, 145, 700, 2049], 100), ('small', 'q4', [96, 130, 2112], 64),
     ('qwen2-0.5b', 'f16', [193, 576, 1152, 2048], None), ('qwen2-0.5b', 'q8', [130, 705, 1500], 256),
     ('qwen2-1.5b', 'q8', [257, 700, 1100, 2048], 1024), ('qwen2-1.5b', 'q4', [128, 513, 1300], None),
-    ('qwen2-7b', 'q4', [100, 500, 737, 777], None), ('qwen2-7b', 'q8', [500, 1400], None), ('qwen2-7b', 'f16', [497, 600], None)]
+    ('qwen2-7b', 'q4', [100, 360, 500, 737, 777, 1760], None), ('qwen2-7b', 'q8', [500, 1400, 1800], None),
+    ('qwen2-7b', 'f16', [497, 600, 1500], None)]
 
 
 @pytest.mark.parametrize('shape,fmt,counts,window', SWEEP)
