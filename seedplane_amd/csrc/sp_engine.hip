@@ -1159,7 +1159,8 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<Attn
             std::fill(mt_of.begin() + col, mt_of.begin() + col + cols, (cols + 15) / 16);
             const bool small = (size_t)cols * NH * ap.nchunk * rec <= room;
             Launch *w = launches.empty() ? nullptr : &launches.back();
-            if (w && small && w->part == wd.part && (size_t)(w->cols + cols) * NH * std::max(w->nchunk, ap.nchunk) * rec <= room) {
+            if (w && small && w->part == wd.part &&
+                (size_t)(w->cols + cols) * NH * std::max(w->nchunk, ap.nchunk) * rec <= room) {
                 w->cols += cols; w->groups += ap.ngroups;
                 w->nchunk = std::max(w->nchunk, ap.nchunk); w->splits = std::max(w->splits, ap.splits);
             } else {
@@ -1199,8 +1200,9 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<Attn
     for (int l = 0; l < d.n_layers; ++l) {
         Layer &ly = layers[l];
         const bool last = l + 1 == d.n_layers;
-        const WideOrder oq = wide_order(ly.qkv, GEMV_MAX_MT, true), oo = wide_order(ly.o, GEMV_MAX_MT, true, o_slices(64, ly.o.fmt)),
-                        og = wide_order(ly.gate_up, GEMV_MAX_MT, false), od = wide_order(ly.down, GEMV_MAX_MT, true);
+        const WideOrder oq = wide_order(ly.qkv, GEMV_MAX_MT, true), og = wide_order(ly.gate_up, GEMV_MAX_MT, false),
+                        oo = wide_order(ly.o, GEMV_MAX_MT, true, o_slices(64, ly.o.fmt)),
+                        od = wide_order(ly.down, GEMV_MAX_MT, true);
         launch_norm_wide(n, x, H, wd.part, pend, (size_t)n * H, ly.in_norm, d.rms_eps, wd.xn, wd.xn_lo, stream, mtp);
         launch_gemm_wide(ly.qkv, oq, EPI_STORE, wd.xn, wd.xn_lo, n, mtp, wd.qkv, nullptr, Nqkv, ly.qkv_b, nullptr, 0, stream);
         const wide::RopeWideArgs ra{RopeArgs{wd.qkv, Nqkv, NH, NKV, HD, wd.rtab, dt, wd.q, kc[l], vc[l], n_slots, nullptr, 0,
@@ -1213,42 +1215,46 @@ void sp_engine::prefill_pass(int n, const sp_token *toks, const std::vector<Attn
                     while (oi < outs.size() && outs[oi].col < w.col0) ++oi;
                     if (oi == outs.size() || outs[oi].col >= w.col0 + w.cols) continue;
                 }
-                const AttnMqStaged am{{wd.q, kc[l], vc[l], dt, dgr + w.g0, NH, NKV, HD, n_slots, w.nchunk, scale, w.part, w.splits},
-                                      wd.kn, wd.vn, WIDE_COLS, w.col0};
+                const AttnMqStaged am{{wd.q, kc[l], vc[l], dt, dgr + w.g0, NH, NKV, HD, n_slots, w.nchunk, scale, w.part,
+                                       w.splits}, wd.kn, wd.vn, WIDE_COLS, w.col0};
                 const dim3 grid(w.nchunk, NKV, w.groups * w.splits);
                 if (HD == 64) launch_attn_mq_ch<64, ATT_CH, true>(G, grid, stream, am);
                 else launch_attn_mq_ch<128, ATT_CH, true>(G, grid, stream, am);
-                hipLaunchKernelGGL(k_attn_combine, dim3(NH, w.cols), dim3(HD), 0, stream, w.part, dnc + w.col0, NH, HD, w.nchunk, wd.attn,
-                                   NH * HD, mtp, w.col0);
+                hipLaunchKernelGGL(k_attn_combine, dim3(NH, w.cols), dim3(HD), 0, stream, w.part, dnc + w.col0, NH, HD, w.nchunk,
+                                   wd.attn, NH * HD, mtp, w.col0);
             }
         }
         if (!to_ring)
-            hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt, dkeep, NKV, HD,
-                               n_slots, WIDE_COLS);
+            hipLaunchKernelGGL(wide::k_ring_commit, dim3(n), dim3(256), 0, stream, wd.kn, wd.vn, kc[l], vc[l], dt, dkeep, NKV,
+                               HD, n_slots, WIDE_COLS);
         if (last) {
             if (n_out == 0) break;
             // only the output columns go on, as compact rows (in the buffers of qkv and q, which are free)
             nc = n_out; mtc = (nc + 15) / 16;
             x = wd.qkv;
             at = (f16 *)wd.q;
-            hipLaunchKernelGGL(wide::k_gather_cols, dim3(nc), dim3(256), 0, stream, wd.x, wd.attn, dout, H, NH * HD, mtp, x, at, mtc);
+            hipLaunchKernelGGL(wide::k_gather_cols, dim3(nc), dim3(256), 0, stream, wd.x, wd.attn, dout, H, NH * HD, mtp, x, at,
+                               mtc);
         }
-        pend = launch_gemm_wide(ly.o, oo, EPI_RESID, at, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part, wd.part_bytes / 4, stream);
+        pend = launch_gemm_wide(ly.o, oo, EPI_RESID, at, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part, wd.part_bytes / 4,
+                                stream);
         launch_norm_wide(nc, x, H, wd.part, pend, (size_t)nc * H, ly.post_norm, d.rms_eps, wd.xn, nullptr, stream, mtc);
         launch_gemm_wide(ly.gate_up, og, EPI_SILU, wd.xn, nullptr, nc, mtc, nullptr, wd.act, I, nullptr, nullptr, 0, stream);
-        pend = launch_gemm_wide(ly.down, od, EPI_RESID, wd.act, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part, wd.part_bytes / 4, stream);
+        pend = launch_gemm_wide(ly.down, od, EPI_RESID, wd.act, nullptr, nc, mtc, x, nullptr, H, nullptr, wd.part,
+                                wd.part_bytes / 4, stream);
     }
     // ---- head: runs of outputs with neighbouring places whose chunks have as many column tiles (the head's order
     // depends on them)
     const DevMat &hm = d.tied_head ? embed : head;
     for (int j0 = 0; j0 < n_out;) {
         int j1 = j0 + 1;
-        while (j1 < n_out && outs[j1].i == outs[j1 - 1].i + 1 && mt_of[outs[j1].col] == mt_of[outs[j0].col] && (logits_dev || j1 - j0 < maxT)) ++j1;
+        const int mt = mt_of[outs[j0].col];
+        while (j1 < n_out && outs[j1].i == outs[j1 - 1].i + 1 && mt_of[outs[j1].col] == mt && (logits_dev || j1 - j0 < maxT)) ++j1;
         const int c = j1 - j0, m1 = (c + 15) / 16;
         float *rows = logits_dev ? logits_dev + (size_t)outs[j0].i * d.vocab : logits;
         launch_norm_wide(c, x + (size_t)j0 * H, H, wd.part + (size_t)j0 * H, pend, (size_t)nc * H, final_norm, d.rms_eps, wd.xn,
                          nullptr, stream, m1);
-        launch_gemm_wide(hm, wide_order(hm, mt_of[outs[j0].col], false), EPI_STORE, wd.xn, nullptr, c, m1, rows, nullptr, d.vocab, nullptr,
+        launch_gemm_wide(hm, wide_order(hm, mt, false), EPI_STORE, wd.xn, nullptr, c, m1, rows, nullptr, d.vocab, nullptr,
                          nullptr, 0, stream);
         if (argmax) launch_ids(rows, c, outs[j0].i);
         j0 = j1;
@@ -2448,7 +2454,8 @@ int sp_op_sample_filtered_host(const float *logits_dev, int32_t vocab, int32_t l
             const int nr = std::min(FM_ROWS, n - r0);
             std::memcpy(h.u, u_host + r0, nr * sizeof(double));
             if (row_host) std::memcpy(h.row, row_host + r0, nr * sizeof(int32_t));
-            filtered_launch(*sc, logits_dev, vocab, ld, row_host ? h.row : row_dev + r0, h.u, nr, temperature, top_k, top_p, h.id, st);
+            filtered_launch(*sc, logits_dev, vocab, ld, row_host ? h.row : row_dev + r0, h.u, nr, temperature, top_k, top_p,
+                            h.id, st);
             HIPCHK(hipStreamSynchronize(st));
             std::memcpy(out_host + r0, h.id, nr * sizeof(int32_t));
         }

@@ -67,7 +67,11 @@ struct Tile {
 // turn; of a wave the tiles w, w + nw, ... of the slice.  A walk visits the tiles of [first, last) in that order.
 struct Walk {
     int kt, w, lo, hi;     // the tile, its wave, its slice's tiles [lo, hi)
-    __device__ __forceinline__ void start(int first, int last, int per) { kt = lo = first; w = 0; hi = min(last, first + per); }
+    __device__ __forceinline__ void start(int first, int last, int per) {
+        kt = lo = first;
+        w = 0;
+        hi = min(last, first + per);
+    }
     __device__ __forceinline__ bool wave_ends(int nw) const { return kt + nw >= hi; }
     __device__ __forceinline__ bool slice_ends(int nw) const { return wave_ends(nw) && (w + 1 >= nw || lo + w + 1 >= hi); }
     __device__ __forceinline__ void next(int last, int per, int nw) {
@@ -414,7 +418,8 @@ __global__ void __launch_bounds__(256) k_ring_commit(const f16 *kn, const f16 *v
 // their 64 threads by wave_sum_dpp, and the 16 wave sums are added in order.  Lane L of a column here holds the elements
 // of threads 8 L .. 8 L + 7 (octets L, L + 128, ..), so eight lanes are one of those waves.
 constexpr int NORM_COLS = 4, NORM_LANES = 128, NORM_MAX_H = 8 * NORM_LANES * 4;
-static_assert(NORM_THREADS == 8 * NORM_LANES && NORM_PER_THREAD * NORM_THREADS == NORM_MAX_H, "k_rmsnorm's assignment of elements");
+static_assert(NORM_THREADS == 8 * NORM_LANES && NORM_PER_THREAD * NORM_THREADS == NORM_MAX_H,
+              "k_rmsnorm's assignment of elements");
 
 template <int NP, int NO>
 __device__ __forceinline__ void norm_wide_body(float *x, int n, const float *part, size_t pstride, const float *w, int H,
