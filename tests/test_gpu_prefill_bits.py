@@ -66,7 +66,7 @@ def test_prompt_gives_the_bits_of_its_steps(gpu_device, shape, fmt, counts, wind
     for n in counts:
         print(f'prefill bits {shape} {fmt} n={n} window={window}', flush=True)
         ids = random_prompt(n, cfg['vocab_size'], seed=n)
-        cap = max(counts) + 80
+        cap = max(counts) + 160
         ref = eng.new_cache(cap, window=window)
         want, greedy = _steps(eng, [(ref, t) for t in ids])
         cache = eng.new_cache(cap, window=window)
@@ -78,8 +78,8 @@ def test_prompt_gives_the_bits_of_its_steps(gpu_device, shape, fmt, counts, wind
         last, _ = eng.forward(ids, cache)
         assert torch.equal(last, want[-1:]), f'{n}: last logits'
         _same_kv(_kv(cache, L), kv, f'{n}: K/V, last logits only')
-        # a second prompt on top of the first, as one call and as steps
-        more = random_prompt(75, cfg['vocab_size'], seed=1)
+        # a second prompt on top of the first (keys from the ring and from the call), as one call and as steps
+        more = random_prompt(150, cfg['vocab_size'], seed=1)
         want2, g2 = _steps(eng, [(ref, t) for t in more])
         assert eng._prefill_greedy(more, cache) == g2[-1], f'{n}: second prompt'
         _same_kv(_kv(cache, L), _kv(ref, L), f'{n}: K/V of the second prompt')
